@@ -1,0 +1,304 @@
+// The matrix-core main loop shared by the prefill GEMMs: C = A W^T with FP32 (or BF16)
+// weights and FP32 results, on the BF16 matrix instructions.
+//
+// Every FP32 operand x is held as three BF16 numbers, x = hi + mid + lo, each the nearest BF16
+// to what the ones before it leave (8 + 8 + 8 significant bits: nothing is left over), and a
+// product is the sum of the six partial products whose size can reach an FP32 rounding:
+//   hi hi + (hi mid + mid hi) + (mid mid + hi lo + lo hi),
+// each exact in the matrix cores and added in FP32.  The three dropped products are below
+// 2^-25 of hi hi, less than the rounding of one FP32 addition.  A BF16 weight is its own hi:
+// three products.  The hi hi products have an accumulator of their own and the others, 2^-8
+// of it and less, a second one added at the end, so the running sum is rounded by one
+// instruction in six (all six into one accumulator: twice the error, and above the FP32
+// instruction's).  Against that instruction (v_mfma_f32_16x16x4f32: 2048 FLOP in 32 cycles) six
+// v_mfma_f32_16x16x32_bf16 (16384 FLOP in 16 cycles each) take 96 cycles where it takes 256.
+//
+// Non-finite inputs: an infinity (or a value past the largest BF16) turns into NaN products, so
+// a result that would have been infinite may come out NaN; NaN stays NaN.
+#pragma once
+#include "common.h"
+
+namespace itts {
+
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+// ------------------------------------------------------------------ split operands
+// Layout of a split [rows][K] operand in memory: tiles of 16 rows x 32 k, and per tile the hi,
+// mid and lo planes of 64 pieces of eight consecutive k, piece 16 (k / 8 % 4) + row % 16.  A
+// plane of a tile is what the 64 lanes of one matrix instruction hold (lane l: row l & 15,
+// k 8 (l >> 4) .. + 7), 1 KB in lane order, so a wave reads its operand with one 16-byte load
+// per lane and no LDS.  Rows are padded to a multiple of 16; the padding is never written
+// (a result row depends on its own operand row only).
+constexpr int kPlaneElems = 512;              // one plane of a tile
+constexpr int kTileElems = 3 * kPlaneElems;   // hi, mid, lo
+__host__ __device__ inline size_t split_elems(size_t rows, size_t k) { return (rows + 15) / 16 * 16 * k * 3; }
+__device__ __forceinline__ size_t split_off(int row, int col, int k) {
+    return (static_cast<size_t>(row >> 4) * (k >> 5) + (col >> 5)) * kTileElems + ((col >> 3) & 3) * 128 + (row & 15) * 8 + (col & 7);
+}
+
+// Two floats to BF16, nearest even, the first in the low half (v_cvt_pk_bf16_f32).
+__device__ __forceinline__ uint32_t bf16_pair(float a, float b) {
+    const bf16x2 v = {static_cast<__bf16>(a), static_cast<__bf16>(b)};
+    return __builtin_bit_cast(uint32_t, v);
+}
+__device__ __forceinline__ float bf16_lo(uint32_t v) { return __uint_as_float(v << 16); }
+__device__ __forceinline__ float bf16_hi(uint32_t v) { return __uint_as_float(v & 0xffff0000u); }
+
+// hi, mid and lo of a pair; x - hi and (x - hi) - mid are exact.
+__device__ __forceinline__ void split_pair(float a, float b, uint32_t& h, uint32_t& m, uint32_t& l) {
+    h = bf16_pair(a, b);
+    a -= bf16_lo(h);
+    b -= bf16_hi(h);
+    m = bf16_pair(a, b);
+    l = bf16_pair(a - bf16_lo(m), b - bf16_hi(m));
+}
+__device__ __forceinline__ void split_piece(const float (&x)[8], u32x4& h, u32x4& m, u32x4& l) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        uint32_t a, b, c;
+        split_pair(x[2 * i], x[2 * i + 1], a, b, c);
+        h[i] = a;
+        m[i] = b;
+        l[i] = c;
+    }
+}
+// Stores one element / four / one eight-element piece of a split operand.
+__device__ __forceinline__ void split_store(uint16_t* p, size_t off, float x) {
+    uint32_t h, m, l;
+    split_pair(x, 0.0f, h, m, l);
+    p[off] = static_cast<uint16_t>(h);
+    p[off + kPlaneElems] = static_cast<uint16_t>(m);
+    p[off + 2 * kPlaneElems] = static_cast<uint16_t>(l);
+}
+// Four consecutive elements, from a column that is a multiple of four.
+__device__ __forceinline__ void split_store4(uint16_t* p, size_t off, const float (&x)[4]) {
+    u32x2 h, m, l;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        uint32_t a, b, c;
+        split_pair(x[2 * i], x[2 * i + 1], a, b, c);
+        h[i] = a;
+        m[i] = b;
+        l[i] = c;
+    }
+    *reinterpret_cast<u32x2*>(p + off) = h;
+    *reinterpret_cast<u32x2*>(p + off + kPlaneElems) = m;
+    *reinterpret_cast<u32x2*>(p + off + 2 * kPlaneElems) = l;
+}
+__device__ __forceinline__ void split_store_piece(uint16_t* p, size_t off, const float (&x)[8]) {
+    u32x4 h, m, l;
+    split_piece(x, h, m, l);
+    *reinterpret_cast<u32x4*>(p + off) = h;
+    *reinterpret_cast<u32x4*>(p + off + kPlaneElems) = m;
+    *reinterpret_cast<u32x4*>(p + off + 2 * kPlaneElems) = l;
+}
+
+// ------------------------------------------------------------------ tile shapes
+// A workgroup of eight waves computes RT x 16 rows by BN columns: four waves load and split
+// weights, four multiply.  The multiplying waves stand WR x WC (WR WC = 4) over TR row tiles
+// and TC column strips of 16 each.  One loading and one multiplying wave share a SIMD, so the
+// splitting (vector ALU) runs beside the matrix instructions, and the weight loads have a
+// vmcnt of their own: the operand loads of a multiplying wave never wait behind HBM.
+constexpr int kGemmThreads = 512;
+constexpr int kGemmUnroll = 4;  // k steps per turn of the multiplying waves' loop
+constexpr int kGemmK = 32 * kGemmUnroll;  // K ranges are multiples of this
+constexpr int kGemmRing = 3;  // k steps of split weights in LDS: read, read ahead, being written
+template <typename WT, int WR_, int TR_, int TC_>
+struct GemmTile {
+    using W = WT;
+    static constexpr int WR = WR_, WC = 4 / WR_, TR = TR_, TC = TC_;
+    static constexpr int RT = WR * TR, BM = RT * 16, NS = WC * TC, BN = NS * 16;
+    static constexpr int PB = sizeof(WT) == 4 ? 3 : 1;       // planes of a weight
+    static constexpr int NP = BN / 64;                       // pieces of a k step per loading thread
+    static constexpr int PD = NP == 1 ? 2 * kGemmUnroll : kGemmUnroll;  // k steps of weights requested ahead
+    static constexpr int NLOW = TR == 1 ? 2 : 1;             // accumulators of the small products per tile
+    static constexpr int NA = TR <= 2 ? 4 : 3;         // operand register sets (NA - 1 k steps ahead)
+    static constexpr int kStepElems = NS * PB * kPlaneElems;
+    // the epilogues that write split rows pass each wave's 16 x 16 TC values through LDS
+    static constexpr int kEpiFloats = 16 * (16 * TC + 4);
+    static constexpr int kLdsBytes =
+        kGemmRing * kStepElems * 2 > 4 * kEpiFloats * 4 ? kGemmRing * kStepElems * 2 : 4 * kEpiFloats * 4;
+    static_assert(BN % 64 == 0, "loading threads cover 64 columns");
+};
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t gemm_rsrc(const void* p, uint32_t bytes) {
+    const uint64_t u = reinterpret_cast<uint64_t>(p);
+    const uint32_t lo = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(static_cast<uint32_t>(u))));
+    const uint32_t hi = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(static_cast<uint32_t>(u >> 32))));
+    // descriptor word 3: raw 32-bit buffer; reads past `bytes` return zero and touch no memory
+    return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>((static_cast<uint64_t>(hi) << 32) | lo), 0,
+                                             __builtin_amdgcn_readfirstlane(static_cast<int>(bytes)), 0x00020000);
+}
+__device__ __forceinline__ u32x4 gemm_load16(__amdgpu_buffer_rsrc_t rs, uint32_t voff, uint32_t soff) {
+    return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, static_cast<int>(voff), static_cast<int>(soff), 0));
+}
+
+// ------------------------------------------------------------------ loading waves
+// Thread t of 256 owns, of each 32-wide k step, the piece (column t / 4 (+ 64), eight k at
+// 8 (t % 4)): four threads read 128 consecutive bytes of a weight row.  In LDS a piece goes to
+// slot 16 g + (c ^ 2 g) of its strip (g = k / 8 % 4, c = column % 16): eight neighbouring
+// threads (two columns, four g) write, and eight neighbouring lanes (one g, eight c) read,
+// eight different 16-byte banks.  k step s + 2 is written while the multiplying waves use step
+// s, one barrier per step; PD steps are in flight from memory.  `w`: the tile's first
+// row, at its first k.
+template <class T>
+__device__ __forceinline__ void gemm_loader(uint16_t* ring, const typename T::W* w, int K, int nst, int t) {
+    using WT = typename T::W;
+    constexpr int NL = sizeof(WT) == 4 ? 2 : 1;  // 16-byte loads per piece
+    constexpr int PD = T::PD;
+    const __amdgpu_buffer_rsrc_t rs = gemm_rsrc(w, static_cast<uint32_t>((static_cast<size_t>(T::BN - 1) * K + nst * 32) * sizeof(WT)));
+    const int g = t & 3, c0 = t >> 2;
+    uint32_t voff[T::NP];
+    uint16_t* dst[T::NP];
+#pragma unroll
+    for (int p = 0; p < T::NP; ++p) {
+        const int c = c0 + 64 * p;
+        voff[p] = static_cast<uint32_t>((static_cast<size_t>(c) * K + 8 * g) * sizeof(WT));
+        dst[p] = ring + (c >> 4) * T::PB * kPlaneElems + (16 * g + ((c & 15) ^ (2 * g))) * 8;
+    }
+    u32x4 raw[PD][T::NP][NL];
+    auto load = [&](int slot, int s) {  // steps past the last: out of the buffer's range, no memory access
+#pragma unroll
+        for (int p = 0; p < T::NP; ++p) {
+            const uint32_t o = s < nst ? voff[p] + static_cast<uint32_t>(s) * 32 * sizeof(WT) : 0x40000000u;
+#pragma unroll
+            for (int q = 0; q < NL; ++q) raw[slot][p][q] = gemm_load16(rs, o + 16 * q, 0);
+        }
+    };
+    int buf = 0;
+    auto put = [&](int slot) {
+#pragma unroll
+        for (int p = 0; p < T::NP; ++p) {
+            uint16_t* d = dst[p] + buf * T::kStepElems;
+            if constexpr (T::PB == 3) {
+                float x[8];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) x[i] = __uint_as_float(raw[slot][p][i >> 2][i & 3]);
+                u32x4 h, m, l;
+                split_piece(x, h, m, l);
+                *reinterpret_cast<u32x4*>(d) = h;
+                *reinterpret_cast<u32x4*>(d + kPlaneElems) = m;
+                *reinterpret_cast<u32x4*>(d + 2 * kPlaneElems) = l;
+            } else {
+                *reinterpret_cast<u32x4*>(d) = raw[slot][p][0];
+            }
+        }
+        buf = buf + 1 == kGemmRing ? 0 : buf + 1;
+    };
+#pragma unroll
+    for (int s = 0; s < PD; ++s) load(s, s);
+    put(0);
+    load(0, PD);
+    put(1);
+    load(1, PD + 1);
+    __syncthreads();
+    // sched_barrier: each step's split stays behind the barrier ahead of it and its loads are
+    // issued at once; moved across, they made a step wait for loads of the steps after it
+    auto step = [&](int s, int u) {
+        __builtin_amdgcn_sched_barrier(0);
+        put((u + 2) % PD);
+        load((u + 2) % PD, s + u + 2 + PD);
+        __builtin_amdgcn_sched_barrier(0);
+        __syncthreads();
+    };
+    int s = 0;
+    for (; s + PD <= nst; s += PD) {
+#pragma unroll
+        for (int u = 0; u < PD; ++u) step(s, u);
+    }
+    if (s < nst) {  // nst is a multiple of kGemmUnroll, PD of kGemmUnroll or twice it
+#pragma unroll
+        for (int u = 0; u < kGemmUnroll; ++u) step(s, u);
+    }
+}
+
+// ------------------------------------------------------------------ multiplying waves
+// acc[i][c] = (row tile i) x (strip c) over nst k steps.  ars: the split operand; aoff[i]: this
+// lane's byte offset of row tile i's first k step.  The next strip's weights are read from LDS
+// while the current one's matrix instructions run (the first strip of step s + 1 too: the
+// loading waves finished it before the barrier ahead of step s).
+template <class T>
+__device__ __forceinline__ void gemm_compute(const uint16_t* ring, __amdgpu_buffer_rsrc_t ars, const uint32_t (&aoff)[T::TR], int nst,
+                                             int wc, int lane, f32x4 (&acc)[T::TR][T::TC]) {
+    bf16x8 av[T::NA][T::TR][3], bv[2][T::PB];
+    f32x4 low[T::NLOW][T::TR][T::TC];
+#pragma unroll
+    for (int q = 0; q < T::NLOW; ++q)
+#pragma unroll
+        for (int i = 0; i < T::TR; ++i)
+#pragma unroll
+            for (int c = 0; c < T::TC; ++c) low[q][i][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+    auto load_a = [&](int set, int s, int i, int p) {  // plane p of row tile i; steps past the last reread it
+        const uint32_t so = static_cast<uint32_t>(min(s, nst - 1)) * (kTileElems * 2);
+        av[set][i][p] = __builtin_bit_cast(bf16x8, gemm_load16(ars, aoff[i] + p * kPlaneElems * 2, so));
+    };
+    const int g = lane >> 4;
+    const uint16_t* src = ring + wc * T::TC * T::PB * kPlaneElems + (16 * g + ((lane & 15) ^ (2 * g))) * 8;
+    int buf = 0;
+    auto load_b = [&](int set, int b, int c, int p) {
+        bv[set][p] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(src + b * T::kStepElems + (c * T::PB + p) * kPlaneElems));
+    };
+#pragma unroll
+    for (int s = 0; s < T::NA - 1; ++s)
+#pragma unroll
+        for (int q = 0; q < 3 * T::TR; ++q) load_a(s, s, q / 3, q % 3);
+    __syncthreads();
+#pragma unroll
+    for (int p = 0; p < T::PB; ++p) load_b(0, 0, 0, p);
+    // The products of a strip, one group of TR matrix instructions each, in order of the operand
+    // planes.  A group takes at most one operand load and one weight read with it: a 1 KB load
+    // occupies the CU's address path for 16 cycles and four waves share it, so nine loads
+    // issued at once held a wave's matrix instructions back by up to 576 cycles per step.
+    constexpr int NP = T::PB == 3 ? 6 : 3, NG = T::TC * NP, NQ = 3 * T::TR;
+    constexpr int pa[6] = {0, 2, T::PB == 3 ? 0 : 1, 1, 1, 0}, pb[6] = {0, 0, T::PB == 3 ? 2 : 0, 1, 0, 1};
+    static_assert(NQ <= NG, "one operand load per group");
+    auto step = [&](int s, int u) {
+        const int nbuf = buf + 1 == kGemmRing ? 0 : buf + 1;
+#pragma unroll
+        for (int c = 0; c < T::TC; ++c) {
+            const int cur = (u * T::TC + c) & 1;
+#pragma unroll
+            for (int g = 0; g < NP; ++g) {
+                const int gi = c * NP + g, q = gi * NQ / NG;
+                if (gi == 0 || q != (gi - 1) * NQ / NG) load_a((u + T::NA - 1) % T::NA, s + u + T::NA - 1, q / 3, q % 3);
+                if (g < T::PB) {
+                    if (c + 1 < T::TC) load_b(cur ^ 1, buf, c + 1, g);
+                    else load_b(cur ^ 1, nbuf, 0, g);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+                auto& d = g == 0 ? acc : low[(g + 1) % T::NLOW];
+#pragma unroll
+                for (int i = 0; i < T::TR; ++i)
+                    d[i][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[u % T::NA][i][pa[g]], bv[cur][pb[g]], d[i][c], 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        buf = nbuf;
+        __syncthreads();
+    };
+    // Register sets come round after U steps; nst is a multiple of kGemmUnroll.
+    constexpr int U = T::NA == 3 ? 3 * kGemmUnroll : kGemmUnroll;
+    int s = 0;
+    for (; s + U <= nst; s += U) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) step(s, u);
+    }
+    if constexpr (U > kGemmUnroll) {
+        if (s < nst) {
+#pragma unroll
+            for (int u = 0; u < kGemmUnroll; ++u) step(s, u);
+            if (s + kGemmUnroll < nst) {
+#pragma unroll
+                for (int u = kGemmUnroll; u < 2 * kGemmUnroll; ++u) step(s, u);
+            }
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < T::TR; ++i)
+#pragma unroll
+        for (int c = 0; c < T::TC; ++c) acc[i][c] += T::NLOW == 2 ? low[0][i][c] + low[1][i][c] : low[0][i][c];
+}
+
+}  // namespace itts

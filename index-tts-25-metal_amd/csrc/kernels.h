@@ -241,7 +241,7 @@ hipError_t launch_beam_advance(const BeamAdvanceArgs& a, hipStream_t s);
 // ------------------------------------------------------------------ prefill
 struct LnRowsArgs {
     const float* x;
-    float* y;
+    uint16_t* y;            // split operand of the next GEMM (gemm_core.h)
     const float* w;
     const float* b;
     int rows;
@@ -249,22 +249,23 @@ struct LnRowsArgs {
 hipError_t launch_ln_rows(const LnRowsArgs& a, hipStream_t s);
 
 // kGemmStore: c[M][N] = dot + bias.  kGemmSwiglu: output columns come in (gate, up) pairs
-// 2i, 2i + 1; c[M][N / 2] gets silu(gate) * up (the Qwen MLP with interleaved weight rows).
+// 2i, 2i + 1; c_split[M][N / 2] gets silu(gate) * up (the Qwen MLP with interleaved weight rows).
 enum GemmEpi : int { kGemmQkv = 0, kGemmResid = 1, kGemmGelu = 2, kGemmStore = 3, kGemmSwiglu = 4 };
 struct GemmArgs {
-    const float* a;         // [M][K]
+    const uint16_t* a;      // [M][K], split (gemm_core.h)
     const void* w;          // [N][K] fp32 or bf16
     const float* bias;      // [N]
     int M, N, K;
     float* c;               // [M][N] (kGemmResid: read-modify-write residual)
+    uint16_t* c_split;      // kGemmGelu [M][N], kGemmSwiglu [M][N / 2]: split operand of the next GEMM
     // kGemmQkv: q rows to c ([M][1280]); K/V to the cache of row_slot[m] at row_pos[m]
     float* kv;
     size_t kv_slot_stride, kv_layer_off, kv_v_off;
     uint32_t kv_cap;
     const uint32_t* row_slot;
     const uint32_t* row_pos;
-    // split-K: at most `splits` K ranges (multiples of 128); launch_gemm picks the row
-    // blocking and the split count from an estimate of the time.  The partial tiles go to
+    // split-K: at most `splits` K ranges (multiples of 128); launch_gemm picks the tile
+    // shape and the split count from an estimate of the time.  The partial tiles go to
     // ws[splits][M][N] and a second kernel adds them in split order.
     int splits;             // 1: no split
     float* ws;
@@ -273,11 +274,11 @@ struct GemmArgs {
     // reduce when there is one
     const float* ln_w;
     const float* ln_b;
-    float* ln_out;
+    uint16_t* ln_out;       // split
 };
 // The workspace holds kGemmWsFloats floats, which bounds splits * M * N.
 constexpr int kGemmMaxSplits = 16;
-constexpr size_t kGemmWsFloats = size_t(512) * 64 * 64;
+constexpr size_t kGemmWsFloats = size_t(8) << 20;
 // The split count launch_gemm would use for this shape (callers pass it in GemmArgs.splits;
 // 1 forbids splitting).
 int gemm_splits(int M, int N, int K);
@@ -290,7 +291,7 @@ struct CausalArgs {
     uint32_t kv_cap;
     const uint32_t* row_slot;
     const uint32_t* row_pos;
-    float* out;             // [M][1280]
+    uint16_t* out;          // [M][1280], split operand of attn.c_proj
     int M;
 };
 hipError_t launch_causal_attention(const CausalArgs& a, hipStream_t s);

@@ -1,15 +1,15 @@
 // Prefill kernels (the P-row prefix forward of gpt.cpp:88-125 with initial=true).
 //
 // * ln_rows: LayerNorm of each 1280-wide row (kernels.metal:618-669), one workgroup per row.
-// * gemm: C[M][N] = A[M][K] * W[N][K]^T + bias on the FP32 matrix cores
-//   (v_mfma_f32_16x16x4f32), replacing the broadcast-bias + MPS GEMM pair of
-//   metal_context.mm:368-410.  A workgroup covers up to 192 rows x 64 columns: the A rows
-//   go through LDS (double-buffered, 32 k per stage), each wave's 16 weight rows straight
-//   into registers one stage pair ahead.  Epilogues: q rows + K/V cache store
-//   (kernels.metal:1250-1266), residual add in place, GELU, plain store, SiLU-gated pairs.
-//   When the tiles alone would leave CUs idle (a 155-row prefix has 20 tiles of a
-//   1280-wide output), K is split over gridDim.z: each split writes its partial tile to a
-//   workspace and gemm_reduce adds the splits in order, then the bias and the epilogue.
+// * gemm: C[M][N] = A[M][K] * W[N][K]^T + bias on the matrix cores, replacing the
+//   broadcast-bias + MPS GEMM pair of metal_context.mm:368-410.  The operands are FP32 values
+//   split into three BF16 numbers and multiplied by BF16 instructions (gemm_core.h); A comes
+//   split from the kernel that produced it (LayerNorm, attention, GELU), weights are split on
+//   the way to LDS.  Epilogues: q rows + K/V cache store (kernels.metal:1250-1266), residual
+//   add in place, GELU, plain store, SiLU-gated pairs.
+//   When the tiles alone would leave CUs idle, K is split over gridDim.z: each split writes
+//   its partial tile to a workspace and gemm_reduce adds the splits in order, then the bias
+//   and the epilogue.
 // * causal_attention: one 8-wave workgroup per (16 query rows, head); the keys move through LDS
 //   64 at a time (K transposed), lane = key for the scores, lane = dimension for the
 //   weighted V sum, online max/sum rescaling (same recurrence as
@@ -17,8 +17,11 @@
 // Rows of several sequences may be stacked (ragged batch prefill): row m belongs to
 // cache slot row_slot[m] at position row_pos[m] and attends to that slot's rows
 // 0..row_pos[m].
+#include <algorithm>
+#include <cmath>
 #include <type_traits>
 
+#include "gemm_core.h"
 #include "kernels.h"
 
 namespace itts {
@@ -32,47 +35,7 @@ __global__ __launch_bounds__(256) void ln_rows_kernel(LnRowsArgs a) {
     for (int i = 0; i < 5; ++i) v[0][i] = a.x[static_cast<size_t>(row) * kWidth + tid + 256 * i];
     ln_block<1, 5>(v, a.w, a.b, red);
 #pragma unroll
-    for (int i = 0; i < 5; ++i) a.y[static_cast<size_t>(row) * kWidth + tid + 256 * i] = v[0][i];
-}
-
-// GEMM tiling.  A workgroup owns up to 192 rows (row tiles of 16) x 64 columns; wave w owns
-// columns 16w .. 16w + 15 of that for every row tile, so the A rows are shared through LDS
-// and each wave streams its own 16 weight rows straight into registers.
-// v_mfma_f32_16x16x4f32 operands: A lane l -> row l & 15, k l >> 4; B lane l -> k l >> 4,
-// column l & 15; D lane l, element r -> row 4 (l >> 4) + r, column l & 15.  Which k the four
-// lane groups carry is free as long as A and B agree: in the c-th of four back-to-back
-// instructions lane group g carries k = k0 + 4g + c, so every lane reads four consecutive k
-// of its row with one 16-byte load (a weight row in global memory, an A row in LDS).
-constexpr int kBN = 64;                // output columns per workgroup
-constexpr int kBK = 64;                // K per LDS stage (four 16-wide MFMA steps)
-constexpr int kMaxRT = 12;             // row tiles of 16 per workgroup (RT: 2, 4, ..., 12)
-constexpr int kAS = kBK + 4;           // A row stride in LDS, 4 x odd: conflict-free 16-byte reads
-constexpr int kGemmThreads = 512;      // eight waves
-
-typedef float floatx4 __attribute__((ext_vector_type(4)));
-
-// Output element (row, col) of the GEMM, v = dot + bias: the epilogue.
-template <int EPI>
-__device__ __forceinline__ void gemm_store(const GemmArgs& a, int row, int col, float v) {
-    if constexpr (EPI == kGemmQkv) {
-        if (col < kWidth) {
-            a.c[static_cast<size_t>(row) * kWidth + col] = v;
-        } else {
-            const int rr = col - kWidth;
-            const bool is_v = rr >= kWidth;
-            const int c = is_v ? rr - kWidth : rr;
-            const size_t off = static_cast<size_t>(a.row_slot[row]) * a.kv_slot_stride + a.kv_layer_off + (is_v ? a.kv_v_off : 0) +
-                               (static_cast<size_t>(c >> 6) * a.kv_cap + a.row_pos[row]) * kHeadDim + (c & 63);
-            a.kv[off] = v;
-        }
-    } else if constexpr (EPI == kGemmResid) {
-        float* p = a.c + static_cast<size_t>(row) * a.N + col;
-        *p = *p + v;
-    } else if constexpr (EPI == kGemmStore) {
-        a.c[static_cast<size_t>(row) * a.N + col] = v;
-    } else {
-        a.c[static_cast<size_t>(row) * a.N + col] = gelu_f(v);
-    }
+    for (int i = 0; i < 5; ++i) split_store(a.y, split_off(row, tid + 256 * i, kWidth), v[0][i]);
 }
 
 // A value held in a register at this point of the program: an empty asm takes it.  The GEMM
@@ -88,52 +51,23 @@ __device__ __forceinline__ void pin_value(T v) {
 // SiLU-gated product of one (gate, up) column pair (kernels.metal:363-374).
 __device__ __forceinline__ float swiglu_f(float g, float u) { return (g / (1.0f + expf(-g))) * u; }
 
-// Four consecutive k of one weight row as floats.
-__device__ __forceinline__ floatx4 gemm_load_b(const float* p) { return *reinterpret_cast<const floatx4*>(p); }
-__device__ __forceinline__ floatx4 gemm_load_b(const uint16_t* p) {
-    typedef uint32_t u32x2v __attribute__((ext_vector_type(2)));
-    const u32x2v v = *reinterpret_cast<const u32x2v*>(p);
-    return floatx4{__uint_as_float(v.x << 16), __uint_as_float(v.x & 0xffff0000u), __uint_as_float(v.y << 16),
-                   __uint_as_float(v.y & 0xffff0000u)};
+// Cache element of K/V column rr (of 2 x 1280) at position pos of a slot.
+__device__ __forceinline__ size_t kv_off(const GemmArgs& a, int rr, uint32_t slot, uint32_t pos) {
+    const bool is_v = rr >= kWidth;
+    const int c = is_v ? rr - kWidth : rr;
+    return static_cast<size_t>(slot) * a.kv_slot_stride + a.kv_layer_off + (is_v ? a.kv_v_off : 0) +
+           (static_cast<size_t>(c >> 6) * a.kv_cap + pos) * kHeadDim + (c & 63);
 }
 
-// One LDS stage (kBK = 64 k): four 16-wide steps over this wave's NT row tiles (tile
-// t0 + 2 t).  The A fragments of step h + 1 are read while step h's instructions run;
-// per step the instructions go c-major (instruction c of every tile, then c + 1), so
-// consecutive instructions use different accumulators.
-template <int NT>
-__device__ __forceinline__ void gemm_stage(const float (*As)[kAS], int t0, int lane, const floatx4 (&b)[4], floatx4 (&acc)[NT]) {
-    floatx4 av[2][NT];
-    const float* base = &As[t0 * 16 + (lane & 15)][4 * (lane >> 4)];
-#pragma unroll
-    for (int t = 0; t < NT; ++t) av[0][t] = *reinterpret_cast<const floatx4*>(base + 32 * t * kAS);
-#pragma unroll
-    for (int h = 0; h < 4; ++h) {
-        if (h < 3) {
-#pragma unroll
-            for (int t = 0; t < NT; ++t) av[(h + 1) & 1][t] = *reinterpret_cast<const floatx4*>(base + 32 * t * kAS + 16 * (h + 1));
-        }
-#pragma unroll
-        for (int c = 0; c < 4; ++c)
-#pragma unroll
-            for (int t = 0; t < NT; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[h & 1][t][c], b[h][c], acc[t], 0, 0, 0);
-    }
-}
-
-// Row block y covers rows [y RT 16, (y + 1) RT 16) of A; split z covers K range
+// Row block y covers row tiles [y RT, (y + 1) RT) of A; split z covers K range
 // [z kchunk, min(K, (z + 1) kchunk)) and, with SPLIT, writes its raw partial tile to
-// a.ws[z][M][N] for gemm_reduce_kernel.  K ranges are multiples of 2 kBK.  Eight waves:
-// wave w owns columns 16 (w % 4) .. + 15 and the row tiles w / 4, w / 4 + 2, ..., so each
-// SIMD runs two waves.  The main loop has no branches (rows past M and loads past the K
-// range are clamped to valid addresses, their results unused), so the compiler's wait
-// counts stay exact and the prefetched loads stay in flight across the matrix instructions.
-template <typename WT, int EPI, bool SPLIT, int RT>
+// a.ws[z][M][N] for gemm_reduce_kernel.  Row tiles past the last are clamped to it (their
+// results are not stored), so the main loop (gemm_core.h) has no branches.
+template <class T, int EPI, bool SPLIT>
 __global__ __launch_bounds__(kGemmThreads) void gemm_kernel(GemmArgs a, int kchunk) {
-    constexpr int BM = RT * 16, NT = RT / 2;
-    constexpr int NP = BM * (kBK / 4), APER = (NP + kGemmThreads - 1) / kGemmThreads;  // A pieces per stage, per thread
-    __shared__ __align__(16) float As[2][BM][kAS];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int strip = wave & 3, t0 = wave >> 2;
+    __shared__ __align__(16) uint8_t lds[T::kLdsBytes];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     // Workgroup L runs on XCD L % 8 (round-robin dispatch).  The logical index j gives each
     // XCD one contiguous range, row blocks fastest, then splits, then column tiles, so the
     // workgroups sharing a column tile's weights mostly share one L2.
@@ -142,233 +76,153 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_kernel(GemmArgs a, int kchu
     const int per = nwg / 8, rem = nwg % 8, xcd = L % 8;
     const int j = (xcd < rem ? xcd * (per + 1) : rem * (per + 1) + (xcd - rem) * per) + L / 8;
     const int by = j % gridDim.y, bz = (j / gridDim.y) % gridDim.z, bx = j / (gridDim.y * gridDim.z);
-    const int m0 = by * BM;
-    const int mrows = min(BM, a.M - m0);
     const int kb = SPLIT ? bz * kchunk : 0;
-    const int ke = SPLIT ? min(a.K, kb + kchunk) : a.K;
-    const int nst = (ke - kb) / kBK;  // even
-
-    // A stage loader: piece f = tid + kGemmThreads i (mod NP) is 4 consecutive k at column
-    // 4 (f % 16) of row f / 16 (pieces past NP repeat earlier ones: the same value is stored
-    // twice); rows past M read row M - 1 (their output rows are not stored).  Native
-    // vector types: arrays of the float4 struct are copied with memcpy, which the compiler
-    // left in scratch memory.
-    int aoff[APER], aoffs[APER];
-#pragma unroll
-    for (int i = 0; i < APER; ++i) {
-        const int f = (tid + kGemmThreads * i) % NP, r = f / (kBK / 4), c = (f % (kBK / 4)) * 4;
-        aoff[i] = min(m0 + r, a.M - 1) * a.K + c;
-        aoffs[i] = r * kAS + c;
+    const int nst = ((SPLIT ? min(a.K, kb + kchunk) : a.K) - kb) / 32;
+    uint16_t* ring = reinterpret_cast<uint16_t*>(lds);
+    const __amdgpu_buffer_rsrc_t ars = gemm_rsrc(a.a, static_cast<uint32_t>(split_elems(a.M, a.K) * 2));
+    const int tiles = (a.M + 15) / 16;
+    if (wave >= 4) {
+        gemm_loader<T>(ring, static_cast<const typename T::W*>(a.w) + static_cast<size_t>(bx) * T::BN * a.K + kb, a.K, nst, tid - 256);
+        return;
     }
-    // B: this lane's weight row (column n of the output) at k offset 4 (lane >> 4).
-    const WT* wrow = static_cast<const WT*>(a.w) + static_cast<size_t>(bx * kBN + strip * 16 + (lane & 15)) * a.K + 4 * (lane >> 4);
-
-    floatx4 acc[NT];
+    constexpr int TR = T::TR, TC = T::TC;
+    const int wr = wave / T::WC, wc = wave % T::WC;
+    const int tile0 = by * T::RT + wr * TR;
+    uint32_t aoff[TR];
 #pragma unroll
-    for (int t = 0; t < NT; ++t) acc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < TR; ++i)
+        aoff[i] = (static_cast<uint32_t>(min(tile0 + i, tiles - 1)) * (a.K / 32) + kb / 32) * (kTileElems * 2) + lane * 16;
+    f32x4 acc[TR][TC];
+#pragma unroll
+    for (int i = 0; i < TR; ++i)
+#pragma unroll
+        for (int c = 0; c < TC; ++c) acc[i][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+    gemm_compute<T>(ring, ars, aoff, nst, wc, lane, acc);
 
-    // Software pipeline over stages s = 0 .. nst - 1 (nst even), unrolled by two so every
-    // ring index is a constant: stage s computes on LDS buffer s % 2 with weights rb[s % 2];
-    // it requests the A rows of stage s + 2 (into ra[s % 2], stored a stage ago) and then
-    // the weights of stage s + 2 (into rb[s % 2], once read), and ends by storing the A
-    // rows of stage s + 1 (requested a stage earlier) into buffer (s + 1) % 2.  Loads
-    // complete in order, so that store never waits for a load requested after it.  Loads
-    // past the last stage reread it (results unused).
-    floatx4 ra[2][APER], rb[2][4];
-    const int klast = ke - kBK;
-    auto kst = [&](int st) { return min(kb + kBK * st, klast); };
-#define ITTS_LOAD_A(set, st)                                                                  \
-    _Pragma("unroll") for (int i = 0; i < APER; ++i) ra[set][i] = *reinterpret_cast<const floatx4*>(a.a + aoff[i] + kst(st))
-#define ITTS_LOAD_B(set, st)                                                                  \
-    _Pragma("unroll") for (int q = 0; q < 4; ++q) rb[set][q] = gemm_load_b(wrow + kst(st) + 16 * q)
-#define ITTS_STORE_A(set, buf)                                                                \
-    _Pragma("unroll") for (int i = 0; i < APER; ++i) *reinterpret_cast<floatx4*>(&As[buf][0][0] + aoffs[i]) = ra[set][i]
-#define ITTS_STAGE(Q)                                                                         \
-    do {                                                                                      \
-        floatx4 bcur[4];                                                                      \
-        _Pragma("unroll") for (int q = 0; q < 4; ++q) bcur[q] = rb[Q][q];                     \
-        ITTS_LOAD_A(Q, s + Q + 2);                                                            \
-        ITTS_LOAD_B(Q, s + Q + 2);                                                            \
-        __builtin_amdgcn_sched_barrier(0);                                                    \
-        gemm_stage<NT>(As[Q], t0, lane, bcur, acc);                                           \
-        __builtin_amdgcn_sched_barrier(0);                                                    \
-        ITTS_STORE_A(1 - Q, 1 - Q);                                                           \
-        __syncthreads();                                                                      \
-    } while (0)
-    ITTS_LOAD_A(0, 0);
-    ITTS_LOAD_B(0, 0);
-    ITTS_LOAD_A(1, 1);
-    ITTS_LOAD_B(1, 1);
-    ITTS_STORE_A(0, 0);
-    __syncthreads();
-    for (int s = 0; s < nst; s += 2) {
-        ITTS_STAGE(0);
-        ITTS_STAGE(1);
-    }
-#undef ITTS_STAGE
-#undef ITTS_STORE_A
-#undef ITTS_LOAD_B
-#undef ITTS_LOAD_A
-
-    const int col = bx * kBN + strip * 16 + (lane & 15);
+    // acc[i][c][r]: row 16 (tile0 + i) + rq + r, column col0 + 16 c
+    const int col0 = bx * T::BN + wc * TC * 16 + (lane & 15);
     const int rq = 4 * (lane >> 4);
     if constexpr (SPLIT) {
         // Every destination's 32-bit element offset formed before the first store (a split's
         // plane is M x N < 2^31 elements): with one register pair reused for each row's
         // address, the compiler let only about two stores be in flight at a time.
         float* ws = a.ws + static_cast<size_t>(bz) * a.M * a.N;
-        uint32_t off[NT][4];
+        uint32_t off[TR][4];
 #pragma unroll
-        for (int t = 0; t < NT; ++t)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                off[t][r] = static_cast<uint32_t>((m0 + (t0 + 2 * t) * 16 + rq + r) * a.N + col);
-                pin_value(off[t][r]);
-            }
-#pragma unroll
-        for (int t = 0; t < NT; ++t)
+        for (int i = 0; i < TR; ++i)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const int row = (t0 + 2 * t) * 16 + rq + r;
-                if (row < mrows) ws[off[t][r]] = acc[t][r];
-            }
-    } else if constexpr (EPI == kGemmSwiglu) {
-        // columns col and col ^ 1 sit in lanes l and l ^ 1, on the same rows
-        const float bias = a.bias[col];
-        float out[NT][4];
-#pragma unroll
-        for (int t = 0; t < NT; ++t)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int row = (t0 + 2 * t) * 16 + rq + r;
-                const float v = acc[t][r] + bias;
-                const float u = __shfl_xor(v, 1, 64);
-                out[t][r] = swiglu_f(v, u);
-                pin_value(out[t][r]);
+                off[i][r] = static_cast<uint32_t>(((tile0 + i) * 16 + rq + r) * a.N + col0);
+                pin_value(off[i][r]);
             }
 #pragma unroll
-        for (int t = 0; t < NT; ++t)
+        for (int i = 0; i < TR; ++i)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int row = (t0 + 2 * t) * 16 + rq + r;
-                if (row < mrows && !(col & 1)) a.c[static_cast<size_t>(m0 + row) * (a.N / 2) + col / 2] = out[t][r];
-            }
-    } else if constexpr (EPI == kGemmResid) {
-        // Every row's residual requested before the first store (rows past the block read the
-        // block's first row): a load under the per-row branch was waited for before the next.
-        const float bias = a.bias[col];
-        float res[NT][4];
+            for (int r = 0; r < 4; ++r)
+                if ((tile0 + i) * 16 + rq + r < a.M) {
 #pragma unroll
-        for (int t = 0; t < NT; ++t)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int row = (t0 + 2 * t) * 16 + rq + r;
-                res[t][r] = a.c[static_cast<size_t>(m0 + (row < mrows ? row : 0)) * a.N + col];
-            }
-        float out[NT][4];
-#pragma unroll
-        for (int t = 0; t < NT; ++t)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                out[t][r] = res[t][r] + (acc[t][r] + bias);
-                pin_value(out[t][r]);
-            }
-#pragma unroll
-        for (int t = 0; t < NT; ++t)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int row = (t0 + 2 * t) * 16 + rq + r;
-                if (row < mrows) a.c[static_cast<size_t>(m0 + row) * a.N + col] = out[t][r];
-            }
-    } else if constexpr (EPI == kGemmQkv) {
-        // K/V columns: every row's cache slot and position requested before the first store, as
-        // above (a workgroup's 64 columns are all q or all K/V: 1280 is a multiple of 64).
-        const float bias = a.bias[col];
-        float out[NT][4];
-#pragma unroll
-        for (int t = 0; t < NT; ++t)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                out[t][r] = acc[t][r] + bias;
-                pin_value(out[t][r]);
-            }
-        if (bx * kBN < kWidth) {
-#pragma unroll
-            for (int t = 0; t < NT; ++t)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int row = (t0 + 2 * t) * 16 + rq + r;
-                    if (row < mrows) a.c[static_cast<size_t>(m0 + row) * kWidth + col] = out[t][r];
+                    for (int c = 0; c < TC; ++c) ws[off[i][r] + 16 * c] = acc[i][c][r];
                 }
-        } else {
-            uint32_t rs[NT][4], rp[NT][4];
+    } else if constexpr (EPI == kGemmGelu || EPI == kGemmSwiglu) {
+        // Split rows for the next GEMM: each wave passes its row tiles through its own part of
+        // LDS (the ring is no longer read), so that a lane holds eight consecutive columns.
+        constexpr int W = EPI == kGemmGelu ? 16 * TC : 8 * TC, S = W + 4;  // columns written; row stride
+        float* buf = reinterpret_cast<float*>(lds) + wave * T::kEpiFloats;
+        const int oc0 = EPI == kGemmGelu ? bx * T::BN + wc * W : (bx * T::BN) / 2 + wc * W;
+        const int on = EPI == kGemmGelu ? a.N : a.N / 2;
+        float bias[TC];
 #pragma unroll
-            for (int t = 0; t < NT; ++t)
+        for (int c = 0; c < TC; ++c) bias[c] = a.bias[col0 + 16 * c];
+#pragma unroll
+        for (int i = 0; i < TR; ++i) {
+#pragma unroll
+            for (int c = 0; c < TC; ++c)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    const int row = (t0 + 2 * t) * 16 + rq + r, rc = m0 + (row < mrows ? row : 0);
-                    rs[t][r] = a.row_slot[rc];
-                    rp[t][r] = a.row_pos[rc];
+                    const float v = acc[i][c][r] + bias[c];
+                    if constexpr (EPI == kGemmGelu) {
+                        buf[(rq + r) * S + 16 * c + (lane & 15)] = gelu_f(v);
+                    } else {  // columns col and col ^ 1 sit in lanes l and l ^ 1, on the same rows
+                        const float u = __shfl_xor(v, 1, 64);
+                        if (!(lane & 1)) buf[(rq + r) * S + 8 * c + (lane & 15) / 2] = swiglu_f(v, u);
+                    }
+                }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            for (int f = lane; f < 16 * (W / 8); f += 64) {
+                const int r = f & 15, q = f >> 4, row = (tile0 + i) * 16 + r;
+                float x[8];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) x[e] = buf[r * S + 8 * q + e];
+                if (row < a.M) split_store_piece(a.c_split, split_off(row, oc0 + 8 * q, on), x);
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+        }
+    } else {
+        float bias[TC];
+#pragma unroll
+        for (int c = 0; c < TC; ++c) bias[c] = a.bias[col0 + 16 * c];
+        // K/V columns (a workgroup's columns are all q or all K/V: 1280 is a multiple of BN)
+        const bool kv_cols = EPI == kGemmQkv && bx * T::BN >= kWidth;
+        const int ldc = EPI == kGemmQkv ? kWidth : a.N;
+#pragma unroll
+        for (int i = 0; i < TR; ++i) {
+            // Every row's residual, or cache slot and position, requested before the first
+            // store (rows past M read row 0): a load under the per-row branch was waited
+            // for before the next.
+            float out[TC][4];
+            uint32_t rs[4] = {}, rp[4] = {};
+            const int row0 = (tile0 + i) * 16 + rq;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int rc = row0 + r < a.M ? row0 + r : 0;
+                if (kv_cols) {
+                    rs[r] = a.row_slot[rc];
+                    rp[r] = a.row_pos[rc];
                 }
 #pragma unroll
-            for (int t = 0; t < NT; ++t)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    pin_value(rs[t][r]);
-                    pin_value(rp[t][r]);
+                for (int c = 0; c < TC; ++c) {
+                    out[c][r] = acc[i][c][r] + bias[c];
+                    if constexpr (EPI == kGemmResid) out[c][r] += a.c[static_cast<size_t>(rc) * a.N + col0 + 16 * c];
                 }
-            const int rr = col - kWidth;
-            const bool is_v = rr >= kWidth;
-            const int c = is_v ? rr - kWidth : rr;
+            }
 #pragma unroll
-            for (int t = 0; t < NT; ++t)
+            for (int r = 0; r < 4; ++r) {
+                pin_value(rs[r]);
+                pin_value(rp[r]);
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int row = (t0 + 2 * t) * 16 + rq + r;
-                    if (row < mrows) {
-                        const size_t off = static_cast<size_t>(rs[t][r]) * a.kv_slot_stride + a.kv_layer_off + (is_v ? a.kv_v_off : 0) +
-                                           (static_cast<size_t>(c >> 6) * a.kv_cap + rp[t][r]) * kHeadDim + (c & 63);
-                        a.kv[off] = out[t][r];
+                for (int c = 0; c < TC; ++c) pin_value(out[c][r]);
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                if (row0 + r < a.M) {
+#pragma unroll
+                    for (int c = 0; c < TC; ++c) {
+                        if (kv_cols) a.kv[kv_off(a, col0 + 16 * c - kWidth, rs[r], rp[r])] = out[c][r];
+                        else a.c[static_cast<size_t>(row0 + r) * ldc + col0 + 16 * c] = out[c][r];
                     }
                 }
         }
-    } else {
-        // Every value (GELU included) formed before the first store, as above.
-        const float bias = a.bias[col];
-        float out[NT][4];
-#pragma unroll
-        for (int t = 0; t < NT; ++t)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                out[t][r] = EPI == kGemmGelu ? gelu_f(acc[t][r] + bias) : acc[t][r] + bias;
-                pin_value(out[t][r]);
-            }
-#pragma unroll
-        for (int t = 0; t < NT; ++t)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int row = (t0 + 2 * t) * 16 + rq + r;
-                if (row < mrows) a.c[static_cast<size_t>(m0 + row) * a.N + col] = out[t][r];
-            }
     }
 }
 
-// Partial 0 + partial 1 + ... of element e in split order.  Every split's load is issued
-// before the first add (SM, a power of two >= the split count, loads per element; indices
-// past the split count reread the last split and their adds are skipped), so the loads
-// overlap instead of forming a chain of round trips.
+// Partial 0 + partial 1 + ... of four consecutive elements from e on, in split order.  Every
+// split's load is issued before the first add (SM, a power of two >= the split count, loads;
+// indices past the split count reread the last split and their adds are skipped), so the
+// loads overlap instead of forming a chain of round trips.
 template <int SM>
-__device__ __forceinline__ float split_sum_n(const GemmArgs& a, size_t e, size_t plane) {
-    float w[SM];
+__device__ __forceinline__ f32x4 split_sum_n(const GemmArgs& a, size_t e, size_t plane) {
+    f32x4 w[SM];
 #pragma unroll
-    for (int z = 0; z < SM; ++z) w[z] = a.ws[static_cast<size_t>(min(z, a.splits - 1)) * plane + e];
-    float d = w[0];
+    for (int z = 0; z < SM; ++z) w[z] = *reinterpret_cast<const f32x4*>(a.ws + static_cast<size_t>(min(z, a.splits - 1)) * plane + e);
+    f32x4 d = w[0];
 #pragma unroll
     for (int z = 1; z < SM; ++z)
         if (z < a.splits) d += w[z];
     return d;
 }
-__device__ __forceinline__ float split_sum(const GemmArgs& a, size_t e, size_t plane) {
+__device__ __forceinline__ f32x4 split_sum(const GemmArgs& a, size_t e, size_t plane) {
     if (a.splits <= 2) return split_sum_n<2>(a, e, plane);
     if (a.splits <= 4) return split_sum_n<4>(a, e, plane);
     if (a.splits <= 8) return split_sum_n<8>(a, e, plane);
@@ -376,38 +230,45 @@ __device__ __forceinline__ float split_sum(const GemmArgs& a, size_t e, size_t p
 }
 
 // Finishes a split-K GEMM: dot = partial 0 + partial 1 + ... in split order, then + bias and
-// the epilogue; one thread per output element.
+// the epilogue; a thread takes 4 columns (kGemmSwiglu: 4 pairs) of one row.  (Eight
+// per thread, one 16-byte store per plane, left a 48-row c_fc 96 workgroups of long GELU chains.)
 template <int EPI>
 __global__ __launch_bounds__(256) void gemm_reduce_kernel(GemmArgs a) {
-    const size_t total = static_cast<size_t>(a.M) * a.N, plane = total;
-    if constexpr (EPI == kGemmSwiglu) {  // one thread per (gate, up) column pair
-        for (size_t e2 = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x; e2 < total / 2;
-             e2 += static_cast<size_t>(gridDim.x) * blockDim.x) {
-            const size_t e = 2 * e2;
-            const float g = split_sum(a, e, plane), u = split_sum(a, e + 1, plane);
-            const int col = static_cast<int>(e % a.N);
-            a.c[e2] = swiglu_f(g + a.bias[col], u + a.bias[col + 1]);
-        }
-        return;
-    }
-    for (size_t e = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x; e < total; e += static_cast<size_t>(gridDim.x) * blockDim.x) {
+    constexpr int W = EPI == kGemmSwiglu ? 8 : 4;
+    const size_t plane = static_cast<size_t>(a.M) * a.N, total = plane / W;
+    for (size_t t = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x; t < total; t += static_cast<size_t>(gridDim.x) * blockDim.x) {
+        const size_t e = t * W;
         const int row = static_cast<int>(e / a.N), col = static_cast<int>(e % a.N);
-        const float bias = a.bias[col];
-        if constexpr (EPI == kGemmQkv) {
-            // the row's cache slot and position requested with the partials, not after them
-            const uint32_t rs = a.row_slot[row], rp = a.row_pos[row];
-            const float v = split_sum(a, e, plane) + bias;
-            if (col < kWidth) {
-                a.c[static_cast<size_t>(row) * kWidth + col] = v;
-            } else {
-                const int rr = col - kWidth;
-                const bool is_v = rr >= kWidth;
-                const int c = is_v ? rr - kWidth : rr;
-                a.kv[static_cast<size_t>(rs) * a.kv_slot_stride + a.kv_layer_off + (is_v ? a.kv_v_off : 0) +
-                     (static_cast<size_t>(c >> 6) * a.kv_cap + rp) * kHeadDim + (c & 63)] = v;
-            }
+        float v[W];
+        uint32_t rs = 0, rp = 0;
+        if (EPI == kGemmQkv && col >= kWidth) {  // requested with the partials, not after them
+            rs = a.row_slot[row];
+            rp = a.row_pos[row];
+        }
+#pragma unroll
+        for (int q = 0; q < W / 4; ++q) {
+            const f32x4 d = split_sum(a, e + 4 * q, plane) + *reinterpret_cast<const f32x4*>(a.bias + col + 4 * q);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[4 * q + i] = d[i];
+        }
+        if constexpr (EPI == kGemmGelu) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[i] = gelu_f(v[i]);
+            split_store4(a.c_split, split_off(row, col, a.N), v);
+        } else if constexpr (EPI == kGemmSwiglu) {
+            float o[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) o[i] = swiglu_f(v[2 * i], v[2 * i + 1]);
+            split_store4(a.c_split, split_off(row, col / 2, a.N / 2), o);
         } else {
-            gemm_store<EPI>(a, row, col, split_sum(a, e, plane) + bias);
+            f32x4 o = {v[0], v[1], v[2], v[3]};
+            if (EPI == kGemmQkv && col >= kWidth) {
+                *reinterpret_cast<f32x4*>(a.kv + kv_off(a, col - kWidth, rs, rp)) = o;
+            } else {
+                f32x4* p = reinterpret_cast<f32x4*>(a.c + static_cast<size_t>(row) * (EPI == kGemmQkv ? kWidth : a.N) + col);
+                if constexpr (EPI == kGemmResid) o = *p + o;
+                *p = o;
+            }
         }
     }
 }
@@ -456,7 +317,7 @@ __global__ __launch_bounds__(256) void gemm_reduce_ln_kernel(GemmArgs a) {
         body(std::integral_constant<int, kGemmMaxSplits>{});
     ln_block<1, 5>(v, a.ln_w, a.ln_b, red);
 #pragma unroll
-    for (int i = 0; i < 5; ++i) a.ln_out[static_cast<size_t>(row) * kWidth + tid + 256 * i] = v[0][i];
+    for (int i = 0; i < 5; ++i) split_store(a.ln_out, split_off(row, tid + 256 * i, kWidth), v[0][i]);
 }
 
 // Causal attention over one head for a block of kQB consecutive rows.  The block's rows are
@@ -577,7 +438,7 @@ __global__ __launch_bounds__(kAttnThreads) void causal_attention_kernel(CausalAr
         }
 #pragma unroll
         for (int i = 0; i < R; ++i)
-            if (pos[i] >= 0) a.out[static_cast<size_t>(m0 + wave + NW * i) * kWidth + h * kHeadDim + lane] = acc[i] / lrun[i];
+            if (pos[i] >= 0) split_store(a.out, split_off(m0 + wave + NW * i, h * kHeadDim + lane, kWidth), acc[i] / lrun[i]);
         r0 = r1;
     }
 }
@@ -603,43 +464,61 @@ int device_cus() {
     return cus;
 }
 
-// How one GEMM is cut: row blocks of RT tiles of 16 (RT even, at most kMaxRT), K cut into
-// `splits` ranges of kchunk (a multiple of 2 kBK).
+// How one GEMM is cut: a tile shape, and K cut into `splits` ranges of kchunk (a multiple of kGemmK).
 struct GemmPlan {
-    int rt, mblocks, splits, kchunk;
+    int tile, mblocks, splits, kchunk;
 };
+// Row tiles of the tile shapes (each 64 columns).  128-column tiles (8 x 8 and 12 x 8) halve
+// the operand reads per product but need more than 256 registers or leave half the CUs idle:
+// slower at every size measured.
+constexpr int kTileRt[] = {1, 2, 4, 8, 12}, kTiles = 5, kGemmBn = 64;
 
-// The plan with the least estimated time, over every RT and split count.  The estimate is
-// a least-squares fit to timings of this kernel on MI355X over RT 2..12 and 1..16 splits
-// for the 1280/5120-wide and the 1024/3072/4096/6144-wide shapes at 64, 155 and 900 rows
-// (median error 2.3%), in microseconds:
-//   4.3 + 0.0039 rounds RT kchunk + 0.86 rounds kchunk / 128
-//       + 0.11 mblocks N K / 1e6 + (split: 2.35 + 2.98 splits M N / 1e6)
-// where rounds = ceil(workgroups / CUs).  The RT kchunk term is the matrix-core work of a
-// workgroup (about 85% of peak); the kchunk / 128 term is a fixed cost per pair of LDS
-// stages (barriers and the LDS reads after them), which is what makes short stages and
-// small RT expensive; the split term is the partial tiles' round trip plus the reduce
-// kernel.  max_splits caps the split count (the workspace holds kGemmWsFloats floats).
-GemmPlan gemm_plan(int M, int N, int K, int max_splits, bool /*bf16*/) {
-    const int rtot = ceil_div(M, 16), ntiles = N / kBN, cus = device_cus();
-    const size_t mn = static_cast<size_t>(M) * N;
-    const int smax = std::max(1, std::min<int>(max_splits, static_cast<int>(std::min<size_t>(kGemmMaxSplits, kGemmWsFloats / std::max<size_t>(1, mn)))));
-    GemmPlan best{kMaxRT, ceil_div(rtot, kMaxRT), 1, K};
+// The plan with the least estimated time, over every tile shape and split count.  The estimate
+// is a least-squares fit to timings of these kernels on MI355X (every tile shape, 1..16 splits,
+// 8 to 1200 rows of the 1280/5120-wide and the 1024..6144-wide shapes, weights from HBM; the
+// plan it picks takes 2.6% longer than the best one on average), in microseconds:
+//   launch + rounds tile + (k steps) (rounds^(2 per CU ? grow : 1) step + crowd max(0, r - free))
+//       + (split: reduce + 1e-6 per_split splits M N)
+// where r = workgroups / CUs and rounds = ceil(r).  `step` is a workgroup's time per 32 k when
+// the chip is mostly idle; `crowd` is what it grows by when every CU is busy (weights and
+// operands then share the L2s, and at 150 rows and more the matrix cores' own rate: 12-tile
+// workgroups on 240 CUs reach 1.0 PFLOP/s of BF16 products, a large BF16 library product 1.13).
+struct GemmCost {
+    double launch, tile, step, crowd, reduce, per_split, grow, free;
+};
+constexpr GemmCost kGemmCost[2][kTiles] = {
+    {   // FP32 weights
+        {2.00, 1.44, 0.260, 0.0455, 2.94, 0.50, 0.555, 0.743},
+        {2.65, 1.46, 0.239, 0.0621, 2.48, 0.68, 0.736, 0.0},
+        {3.61, 1.02, 0.314, 0.111, 2.00, 1.37, 1.0, 0.497},
+        {4.78, 1.29, 0.472, 0.237, 1.00, 1.43, 1.0, 0.5},
+        {4.11, 2.11, 0.585, 0.406, 1.00, 1.06, 1.0, 0.411},
+    },
+    {   // BF16 weights
+        {2.32, 0.935, 0.111, 0.0223, 2.47, 0.50, 0.874, 0.469},
+        {2.39, 0.711, 0.136, 0.0260, 2.22, 1.73, 0.888, 0.494},
+        {3.72, 0.0, 0.162, 0.0603, 1.60, 2.12, 1.0, 0.319},
+        {4.30, 0.608, 0.291, 0.170, 1.00, 1.53, 1.0, 0.534},
+        {3.79, 0.907, 0.358, 0.296, 1.00, 1.46, 1.0, 0.414},
+    }};
+GemmPlan gemm_plan(int M, int N, int K, int max_splits, bool bf16) {
+    const int rtot = ceil_div(M, 16), cus = device_cus();
+    const double mn = static_cast<double>(M) * N;
+    const int smax = std::max(1, std::min<int>(max_splits, static_cast<int>(std::min<double>(kGemmMaxSplits, kGemmWsFloats / mn))));
+    GemmPlan best{kTiles - 1, ceil_div(rtot, kTileRt[kTiles - 1]), 1, K};
     double best_t = 1e30;
-    for (int rt = 2; rt <= kMaxRT; rt += 2) {
-        const int mb = ceil_div(rtot, rt);
-        if (rt > 2 && ceil_div(rtot, rt - 2) == mb) continue;  // a smaller RT covers the rows in as many blocks
+    for (int i = 0; i < kTiles; ++i) {
+        const GemmCost& c = kGemmCost[bf16][i];
+        const int mb = ceil_div(rtot, kTileRt[i]);
         for (int s = 1; s <= smax; ++s) {
-            const int kc = ceil_div(ceil_div(K, s), 2 * kBK) * 2 * kBK;
-            const int sp = ceil_div(K, kc);
-            if (sp != s) continue;
-            const long wgs = static_cast<long>(ntiles) * mb * sp;
-            const double rounds = std::ceil(static_cast<double>(wgs) / cus);
-            double t = 4.3 + 0.0039 * rounds * rt * kc + 0.86 * rounds * kc / (2.0 * kBK) + 0.11 * mb * static_cast<double>(N) * K / 1e6;
-            if (sp > 1) t += 2.35 + 2.98 * sp * static_cast<double>(mn) / 1e6;
+            const int kc = ceil_div(ceil_div(K, s), kGemmK) * kGemmK;
+            if (ceil_div(K, kc) != s) continue;
+            const double r = static_cast<double>(N / kGemmBn) * mb * s / cus, rounds = std::ceil(r);
+            double t = c.launch + rounds * c.tile + kc / 32.0 * (std::pow(rounds, c.grow) * c.step + c.crowd * std::max(0.0, r - c.free));
+            if (s > 1) t += c.reduce + c.per_split * s * mn / 1e6;
             if (t < best_t) {
                 best_t = t;
-                best = GemmPlan{rt, mb, sp, kc};
+                best = GemmPlan{i, mb, s, kc};
             }
         }
     }
@@ -647,14 +526,14 @@ GemmPlan gemm_plan(int M, int N, int K, int max_splits, bool /*bf16*/) {
 }
 
 template <typename WT, int EPI, bool SPLIT>
-void launch_gemm_rt(const GemmArgs& a, const GemmPlan& p, dim3 grid, hipStream_t s) {
-    switch (p.rt) {
-        case 2: hipLaunchKernelGGL((gemm_kernel<WT, EPI, SPLIT, 2>), grid, dim3(kGemmThreads), 0, s, a, p.kchunk); break;
-        case 4: hipLaunchKernelGGL((gemm_kernel<WT, EPI, SPLIT, 4>), grid, dim3(kGemmThreads), 0, s, a, p.kchunk); break;
-        case 6: hipLaunchKernelGGL((gemm_kernel<WT, EPI, SPLIT, 6>), grid, dim3(kGemmThreads), 0, s, a, p.kchunk); break;
-        case 8: hipLaunchKernelGGL((gemm_kernel<WT, EPI, SPLIT, 8>), grid, dim3(kGemmThreads), 0, s, a, p.kchunk); break;
-        case 10: hipLaunchKernelGGL((gemm_kernel<WT, EPI, SPLIT, 10>), grid, dim3(kGemmThreads), 0, s, a, p.kchunk); break;
-        default: hipLaunchKernelGGL((gemm_kernel<WT, EPI, SPLIT, 12>), grid, dim3(kGemmThreads), 0, s, a, p.kchunk); break;
+void launch_gemm_tile(const GemmArgs& a, const GemmPlan& p, hipStream_t s) {
+    const dim3 grid(a.N / kGemmBn, p.mblocks, p.splits), block(kGemmThreads);
+    switch (p.tile) {
+        case 0: hipLaunchKernelGGL((gemm_kernel<GemmTile<WT, 1, 1, 1>, EPI, SPLIT>), grid, block, 0, s, a, p.kchunk); break;
+        case 1: hipLaunchKernelGGL((gemm_kernel<GemmTile<WT, 2, 1, 2>, EPI, SPLIT>), grid, block, 0, s, a, p.kchunk); break;
+        case 2: hipLaunchKernelGGL((gemm_kernel<GemmTile<WT, 4, 1, 4>, EPI, SPLIT>), grid, block, 0, s, a, p.kchunk); break;
+        case 3: hipLaunchKernelGGL((gemm_kernel<GemmTile<WT, 4, 2, 4>, EPI, SPLIT>), grid, block, 0, s, a, p.kchunk); break;
+        default: hipLaunchKernelGGL((gemm_kernel<GemmTile<WT, 4, 3, 4>, EPI, SPLIT>), grid, block, 0, s, a, p.kchunk); break;
     }
 }
 
@@ -662,24 +541,18 @@ void launch_gemm_rt(const GemmArgs& a, const GemmPlan& p, dim3 grid, hipStream_t
 
 int gemm_splits(int M, int N, int K) { return gemm_plan(M, N, K, kGemmMaxSplits, false).splits; }
 
-hipError_t launch_gemm(const GemmArgs& args, int epi, bool bf16, hipStream_t s) {
-    if (args.N % kBN || args.K % (2 * kBK) || args.M < 1 || args.splits < 1 || (args.splits > 1 && !args.ws)) return hipErrorInvalidValue;
-    if ((epi == kGemmStore || epi == kGemmSwiglu) && bf16) return hipErrorInvalidValue;  // FP32 weights only (the Qwen decoder)
-    const GemmPlan p = gemm_plan(args.M, args.N, args.K, args.splits, bf16);
-    GemmArgs a = args;
+static hipError_t launch_gemm_plan(GemmArgs a, int epi, bool bf16, const GemmPlan& p, hipStream_t s) {
     a.splits = p.splits;
-    const dim3 grid(a.N / kBN, p.mblocks, p.splits);
-    const bool ln = args.ln_out != nullptr;
-    if (ln && (epi != kGemmResid || args.N != kWidth)) return hipErrorInvalidValue;
     if (p.splits > 1) {
         // the partial tiles do not depend on the epilogue
-        if (bf16) launch_gemm_rt<uint16_t, kGemmStore, true>(a, p, grid, s);
-        else launch_gemm_rt<float, kGemmStore, true>(a, p, grid, s);
-        if (ln) {
+        if (bf16) launch_gemm_tile<uint16_t, kGemmStore, true>(a, p, s);
+        else launch_gemm_tile<float, kGemmStore, true>(a, p, s);
+        if (a.ln_out) {
             hipLaunchKernelGGL(gemm_reduce_ln_kernel, dim3(a.M), dim3(256), 0, s, a);
             return hipGetLastError();
         }
-        const int rblocks = static_cast<int>(std::min<size_t>((static_cast<size_t>(a.M) * a.N + 255) / 256, 2048));
+        const int w = epi == kGemmSwiglu ? 8 : 4;  // columns of a reduce thread
+        const int rblocks = static_cast<int>(std::min<size_t>((static_cast<size_t>(a.M) * a.N / w + 255) / 256, 2048));
         switch (epi) {
             case kGemmQkv: hipLaunchKernelGGL((gemm_reduce_kernel<kGemmQkv>), dim3(rblocks), dim3(256), 0, s, a); break;
             case kGemmResid: hipLaunchKernelGGL((gemm_reduce_kernel<kGemmResid>), dim3(rblocks), dim3(256), 0, s, a); break;
@@ -690,14 +563,22 @@ hipError_t launch_gemm(const GemmArgs& args, int epi, bool bf16, hipStream_t s) 
         return hipGetLastError();
     }
     switch (epi) {
-        case kGemmQkv: bf16 ? launch_gemm_rt<uint16_t, kGemmQkv, false>(a, p, grid, s) : launch_gemm_rt<float, kGemmQkv, false>(a, p, grid, s); break;
-        case kGemmResid: bf16 ? launch_gemm_rt<uint16_t, kGemmResid, false>(a, p, grid, s) : launch_gemm_rt<float, kGemmResid, false>(a, p, grid, s); break;
-        case kGemmGelu: bf16 ? launch_gemm_rt<uint16_t, kGemmGelu, false>(a, p, grid, s) : launch_gemm_rt<float, kGemmGelu, false>(a, p, grid, s); break;
-        case kGemmStore: launch_gemm_rt<float, kGemmStore, false>(a, p, grid, s); break;
-        default: launch_gemm_rt<float, kGemmSwiglu, false>(a, p, grid, s); break;
+        case kGemmQkv: bf16 ? launch_gemm_tile<uint16_t, kGemmQkv, false>(a, p, s) : launch_gemm_tile<float, kGemmQkv, false>(a, p, s); break;
+        case kGemmResid: bf16 ? launch_gemm_tile<uint16_t, kGemmResid, false>(a, p, s) : launch_gemm_tile<float, kGemmResid, false>(a, p, s); break;
+        case kGemmGelu: bf16 ? launch_gemm_tile<uint16_t, kGemmGelu, false>(a, p, s) : launch_gemm_tile<float, kGemmGelu, false>(a, p, s); break;
+        case kGemmStore: launch_gemm_tile<float, kGemmStore, false>(a, p, s); break;
+        default: launch_gemm_tile<float, kGemmSwiglu, false>(a, p, s); break;
     }
-    if (ln) hipLaunchKernelGGL(ln_rows_kernel, dim3(a.M), dim3(256), 0, s, LnRowsArgs{a.c, a.ln_out, a.ln_w, a.ln_b, a.M});
+    if (a.ln_out) hipLaunchKernelGGL(ln_rows_kernel, dim3(a.M), dim3(256), 0, s, LnRowsArgs{a.c, a.ln_out, a.ln_w, a.ln_b, a.M});
     return hipGetLastError();
+}
+
+hipError_t launch_gemm(const GemmArgs& a, int epi, bool bf16, hipStream_t s) {
+    if (a.N % kGemmBn || a.K % kGemmK || a.M < 1 || a.splits < 1 || (a.splits > 1 && !a.ws)) return hipErrorInvalidValue;
+    if ((epi == kGemmStore || epi == kGemmSwiglu) && bf16) return hipErrorInvalidValue;  // FP32 weights only (the Qwen decoder)
+    if (a.ln_out && (epi != kGemmResid || a.N != kWidth)) return hipErrorInvalidValue;
+    if (split_elems(a.M, a.K) * 2 >= 0x80000000u) return hipErrorInvalidValue;  // 32-bit operand offsets
+    return launch_gemm_plan(a, epi, bf16, gemm_plan(a.M, a.N, a.K, a.splits, bf16), s);
 }
 
 hipError_t launch_causal_attention(const CausalArgs& a, hipStream_t s) {

@@ -41,6 +41,7 @@
 #include <vector>
 
 #include "itts_qwen.h"
+#include "gemm_core.h"
 #include "kernels.h"
 
 namespace itts {
@@ -119,7 +120,7 @@ struct QCausalArgs {
     const float* q;        // [rows][2048]
     const float* kc;
     const float* vc;
-    float* out;            // [rows][2048]
+    uint16_t* out;  // split operand of o_proj            // [rows][2048]
     int rows;
 };
 
@@ -575,8 +576,9 @@ __global__ __launch_bounds__(256) void q_embed_rows_kernel(const float* embed, c
     *reinterpret_cast<float4*>(x + static_cast<size_t>(r) * kD + 4 * t) = v;
 }
 
-// RMSNorm of each 1024-wide row (mit2_rmsnorm_f32_rows_eps, kernels.metal:995-1030).
-__global__ __launch_bounds__(256) void q_rms_rows_kernel(const float* x, const float* w, float* y) {
+// RMSNorm of each 1024-wide row (mit2_rmsnorm_f32_rows_eps, kernels.metal:995-1030), as the next
+// GEMM's split operand.
+__global__ __launch_bounds__(256) void q_rms_rows_kernel(const float* x, const float* w, uint16_t* y) {
     __shared__ float red[4];
     const int r = blockIdx.x, t = threadIdx.x;
     const float4 v = *reinterpret_cast<const float4*>(x + static_cast<size_t>(r) * kD + 4 * t);
@@ -586,8 +588,8 @@ __global__ __launch_bounds__(256) void q_rms_rows_kernel(const float* x, const f
     ss = __builtin_fmaf(v.w, v.w, ss);
     ss = block_sum256(ss, red);
     const float inv = 1.0f / sqrtf(ss / static_cast<float>(kD) + kEps);
-    *reinterpret_cast<float4*>(y + static_cast<size_t>(r) * kD + 4 * t) =
-        make_float4(v.x * inv * g.x, v.y * inv * g.y, v.z * inv * g.z, v.w * inv * g.w);
+    const float n[4] = {v.x * inv * g.x, v.y * inv * g.y, v.z * inv * g.z, v.w * inv * g.w};
+    split_store4(y, split_off(r, 4 * t, kD), n);
 }
 
 // Causal attention of the prompt rows (qwen_attention, kernels.metal:3119-3129, offset 0): one
@@ -641,8 +643,8 @@ __global__ __launch_bounds__(64) void q_causal_attn_kernel(QCausalArgs a) {
         }
         mrun = mnew;
     }
-    a.out[static_cast<size_t>(m) * kQ + h * kHd + lane] = acc1 / lrun;
-    a.out[static_cast<size_t>(m) * kQ + h * kHd + lane + 64] = acc2 / lrun;
+    split_store(a.out, split_off(m, h * kHd + lane, kQ), acc1 / lrun);
+    split_store(a.out, split_off(m, h * kHd + lane + 64, kQ), acc2 / lrun);
 }
 
 #define QWEN_CHECK(x)                                                                                        \
@@ -693,7 +695,8 @@ struct Engine {
     Buf<float2> best;
     Buf<QState> st;
     Buf<uint32_t> toks, ids;
-    Buf<float> X, Xn, QKV, Qp, ATT, FF, ws;
+    Buf<float> X, QKV, Qp, ws;
+    Buf<uint16_t> Xn, ATT, FF;  // split GEMM operands (gemm_core.h)
     int pcap = 0;
     HostStage* pinned = nullptr;
     hipEvent_t up_done = nullptr;  // the last copy out of pinned->up
@@ -818,11 +821,11 @@ struct Engine {
         if (P <= pcap) return;
         const int cap = std::max(P, 256);
         X.alloc(static_cast<size_t>(cap) * kD);
-        Xn.alloc(static_cast<size_t>(cap) * kD);
+        Xn.alloc(split_elems(cap, kD));
         QKV.alloc(static_cast<size_t>(cap) * kQkvN);
         Qp.alloc(static_cast<size_t>(cap) * kQ);
-        ATT.alloc(static_cast<size_t>(cap) * kQ);
-        FF.alloc(static_cast<size_t>(cap) * kF);
+        ATT.alloc(split_elems(cap, kQ));
+        FF.alloc(split_elems(cap, kF));
         if (!ws.p) ws.alloc(kGemmWsFloats);
         pcap = cap;
     }
@@ -837,7 +840,7 @@ struct Engine {
         up_pending = true;
     }
 
-    void gemm(const float* A, const float* Wt, int M, int Nn, int Kk, float* C, int epi) {
+    void gemm(const uint16_t* A, const float* Wt, int M, int Nn, int Kk, float* C, uint16_t* Csplit, int epi) {
         GemmArgs g{};
         g.a = A;
         g.w = Wt;
@@ -846,6 +849,7 @@ struct Engine {
         g.N = Nn;
         g.K = Kk;
         g.c = C;
+        g.c_split = Csplit;
         g.splits = gemm_splits(M, Nn, Kk);
         g.ws = ws.p;
         QWEN_CHECK(launch_gemm(g, epi, false, stream));
@@ -878,18 +882,18 @@ struct Engine {
             const float* w = W(l);
             hipLaunchKernelGGL(q_rms_rows_kernel, dim3(P), dim3(256), 0, s, X.p, N(l) + kNormIn, Xn.p);
             QWEN_CHECK(hipGetLastError());
-            gemm(Xn.p, w, P, kQkvN, kD, QKV.p, kGemmStore);
+            gemm(Xn.p, w, P, kQkvN, kD, QKV.p, nullptr, kGemmStore);
             QPrepArgs pa{QKV.p, P, Qp.p, K(l), Vc(l), N(l) + kNormQ, N(l) + kNormK, inv_freq.p, nullptr};
             hipLaunchKernelGGL(q_prep_kernel, dim3(P, kQH + 2 * kKVH), dim3(64), 0, s, pa);
             QWEN_CHECK(hipGetLastError());
             QCausalArgs ca{Qp.p, K(l), Vc(l), ATT.p, P};
             hipLaunchKernelGGL(q_causal_attn_kernel, dim3(P, kQH), dim3(64), 0, s, ca);
             QWEN_CHECK(hipGetLastError());
-            gemm(ATT.p, w + kOffO, P, kD, kQ, X.p, kGemmResid);
+            gemm(ATT.p, w + kOffO, P, kD, kQ, X.p, nullptr, kGemmResid);
             hipLaunchKernelGGL(q_rms_rows_kernel, dim3(P), dim3(256), 0, s, X.p, N(l) + kNormPost, Xn.p);
             QWEN_CHECK(hipGetLastError());
-            gemm(Xn.p, w + kOffGu, P, 2 * kF, kD, FF.p, kGemmSwiglu);
-            gemm(FF.p, w + kOffD, P, kD, kF, X.p, kGemmResid);
+            gemm(Xn.p, w + kOffGu, P, 2 * kF, kD, nullptr, FF.p, kGemmSwiglu);
+            gemm(FF.p, w + kOffD, P, kD, kF, X.p, nullptr, kGemmResid);
         }
         enqueue_head(X.p + static_cast<size_t>(P - 1) * kD, static_cast<uint32_t>(P));
     }

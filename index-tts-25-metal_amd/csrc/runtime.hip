@@ -28,6 +28,7 @@
 #include <vector>
 
 #include "itts_gpt.h"
+#include "gemm_core.h"
 #include "kernels.h"
 
 namespace itts {
@@ -151,10 +152,10 @@ constexpr uint32_t kNoAllocRows = 512;
 constexpr size_t kScratchActBytes = size_t(kNoAllocRows) * kWidth * 4;
 constexpr size_t kScratchOffX = 0;
 constexpr size_t kScratchOffXn = kScratchOffX + kScratchActBytes;
-constexpr size_t kScratchOffQ = kScratchOffXn + kScratchActBytes;
+constexpr size_t kScratchOffQ = kScratchOffXn + kScratchActBytes / 4 * 6;
 constexpr size_t kScratchOffAtt = kScratchOffQ + kScratchActBytes;
-constexpr size_t kScratchOffFf = kScratchOffAtt + kScratchActBytes;
-constexpr size_t kScratchOffSlot = kScratchOffFf + size_t(kNoAllocRows) * kFfn * 4;
+constexpr size_t kScratchOffFf = kScratchOffAtt + kScratchActBytes / 4 * 6;
+constexpr size_t kScratchOffSlot = kScratchOffFf + size_t(kNoAllocRows) * kFfn * 6;
 constexpr size_t kScratchOffPos = kScratchOffSlot + size_t(kNoAllocRows) * 4;
 constexpr size_t kScratchOffLast = kScratchOffPos + size_t(kNoAllocRows) * 4;
 constexpr size_t kScratchOffWs = kScratchOffLast + 64 * 4;
@@ -196,7 +197,8 @@ ScratchEntry* scratch_entry(int dev) {
 
 // Device buffers of one prefill (enqueue_prefill_layers).
 struct PrefillBufs {
-    float *x, *xn, *q, *att, *ff;
+    float *x, *q;
+    uint16_t *xn, *att, *ff;  // split GEMM operands (gemm_core.h)
     uint32_t *row_slot, *row_pos, *last_rows;
     float* ws;  // split-K workspace, kGemmWsFloats
 };
@@ -227,7 +229,8 @@ struct Engine {
     DevBuf<uint32_t> seg_ids;   // the segments' wrapped text ids
     DevBuf<double> probs;
     // prefill scratch
-    DevBuf<float> px, pxn, pq, patt, pff, pws;
+    DevBuf<float> px, pq, pws;
+    DevBuf<uint16_t> pxn, patt, pff;
     DevBuf<uint32_t> row_slot, row_pos, last_rows;
     // beam search scratch
     DevBuf<float> beam_scores, all_scores;
@@ -733,10 +736,10 @@ struct Engine {
         uint32_t M = 0;
         for (auto r : rows) M += r;
         px.ensure(static_cast<size_t>(M) * kWidth);
-        pxn.ensure(static_cast<size_t>(M) * kWidth);
+        pxn.ensure(split_elems(M, kWidth));
         pq.ensure(static_cast<size_t>(M) * kWidth);
-        patt.ensure(static_cast<size_t>(M) * kWidth);
-        pff.ensure(static_cast<size_t>(M) * kFfn);
+        patt.ensure(split_elems(M, kWidth));
+        pff.ensure(split_elems(M, kFfn));
         row_slot.ensure(M);
         row_pos.ensure(M);
         last_rows.ensure(kMaxBatch);
@@ -760,14 +763,15 @@ struct Engine {
         HIP_CHECK(hipMemcpyAsync(last_rows.p, last.data(), kMaxBatch * 4, hipMemcpyHostToDevice, stream));
         // Host vectors above must outlive the async copies.
         HIP_CHECK(hipStreamSynchronize(stream));
-        enqueue_prefill_layers(PrefillBufs{px.p, pxn.p, pq.p, patt.p, pff.p, row_slot.p, row_pos.p, last_rows.p, pws.p}, nseq, M);
+        enqueue_prefill_layers(PrefillBufs{px.p, pq.p, pxn.p, patt.p, pff.p, row_slot.p, row_pos.p, last_rows.p, pws.p}, nseq, M);
     }
 
     // The prefill forward over M stacked rows whose inputs are in b.x, with each row's
     // sequence slot and position in b.row_slot / b.row_pos and each sequence's last row in
     // b.last_rows; leaves the last rows' logits in logits[0..nseq).
     void enqueue_prefill_layers(const PrefillBufs& b, int nseq, uint32_t M) {
-        float *px_ = b.x, *pxn_ = b.xn, *pq_ = b.q, *patt_ = b.att, *pff_ = b.ff;
+        float *px_ = b.x, *pq_ = b.q;
+        uint16_t *pxn_ = b.xn, *patt_ = b.att, *pff_ = b.ff;
         for (int l = 0; l < layers; ++l) {
             const float* par = params.p + static_cast<size_t>(l) * kParLayer;
             // layers after the first get ln_1 from the previous layer's mlp.c_proj launch
@@ -825,7 +829,7 @@ struct Engine {
             f.K = kWidth;
             f.splits = gemm_splits(static_cast<int>(M), kFfn, kWidth);
             f.ws = b.ws;
-            f.c = pff_;
+            f.c_split = pff_;
             HIP_CHECK(launch_gemm(f, kGemmGelu, bf16, stream));
             GemmArgs f2{};
             f2.a = pff_;
@@ -1023,9 +1027,9 @@ struct Engine {
             ~Drain() { (void)hipStreamSynchronize(s); }
         } drain{stream};
         uint8_t* base = scratch_dev->ptr;
-        const PrefillBufs b{reinterpret_cast<float*>(base + kScratchOffX),      reinterpret_cast<float*>(base + kScratchOffXn),
-                            reinterpret_cast<float*>(base + kScratchOffQ),      reinterpret_cast<float*>(base + kScratchOffAtt),
-                            reinterpret_cast<float*>(base + kScratchOffFf),     reinterpret_cast<uint32_t*>(base + kScratchOffSlot),
+        const PrefillBufs b{reinterpret_cast<float*>(base + kScratchOffX),      reinterpret_cast<float*>(base + kScratchOffQ),
+                            reinterpret_cast<uint16_t*>(base + kScratchOffXn),  reinterpret_cast<uint16_t*>(base + kScratchOffAtt),
+                            reinterpret_cast<uint16_t*>(base + kScratchOffFf),  reinterpret_cast<uint32_t*>(base + kScratchOffSlot),
                             reinterpret_cast<uint32_t*>(base + kScratchOffPos), reinterpret_cast<uint32_t*>(base + kScratchOffLast),
                             reinterpret_cast<float*>(base + kScratchOffWs)};
         struct Flag {  // cleared on every exit, errors included
