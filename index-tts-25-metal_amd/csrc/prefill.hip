@@ -10,10 +10,8 @@
 //   When the tiles alone would leave CUs idle, K is split over gridDim.z: each split writes
 //   its partial tile to a workspace and gemm_reduce adds the splits in order, then the bias
 //   and the epilogue.
-// * causal_attention: one 8-wave workgroup per (16 query rows, head); the keys move through LDS
-//   64 at a time (K transposed), lane = key for the scores, lane = dimension for the
-//   weighted V sum, online max/sum rescaling (same recurrence as
-//   mit2_gpt_causal_attention_sgq_f32, kernels.metal:2249-2292).
+// * causal_attention: 16 query rows of a head per workgroup, both products on the matrix
+//   cores (attn_core.h).
 // Rows of several sequences may be stacked (ragged batch prefill): row m belongs to
 // cache slot row_slot[m] at position row_pos[m] and attends to that slot's rows
 // 0..row_pos[m].
@@ -21,7 +19,7 @@
 #include <cmath>
 #include <type_traits>
 
-#include "gemm_core.h"
+#include "attn_core.h"
 #include "kernels.h"
 
 namespace itts {
@@ -320,127 +318,35 @@ __global__ __launch_bounds__(256) void gemm_reduce_ln_kernel(GemmArgs a) {
     for (int i = 0; i < 5; ++i) split_store(a.ln_out, split_off(row, tid + 256 * i, kWidth), v[0][i]);
 }
 
-// Causal attention over one head for a block of kQB consecutive rows.  The block's rows are
-// taken in runs that share a cache slot (stacked sequences: positions restart at 0 in each
-// slot); for each run the slot's keys 0 .. max position move through LDS kKC at a time.
-// Wave w of 8 owns rows w and w + 8 and keeps their running max, sum and weighted V sum
-// (lane = dimension).  Per row the arithmetic is that of one query at a time: the dot
-// product over dimensions in order from 0, scores scaled by 1/8, max-subtracted exp with
-// the running rescale, the V rows added in key order (kernels.metal:2249-2292).  The loop
-// has no per-row branches: a key past a row's position gets score -inf and weight 0, and a
-// row past its last key sees a rescale of exactly 1, so its state does not change.
-constexpr int kQB = 16, kKC = 64, kAttnThreads = 512, kAttnRows = kQB / (kAttnThreads / 64);
-
-__global__ __launch_bounds__(kAttnThreads) void causal_attention_kernel(CausalArgs a) {
-    typedef float f4 __attribute__((ext_vector_type(4)));
-    constexpr int NW = kAttnThreads / 64, R = kAttnRows;
-    __shared__ f4 Kt[kHeadDim / 4][kKC];                 // [dimension group][key]
-    __shared__ float Vs[kKC][kHeadDim + 4];
-    __shared__ f4 qs[kQB][kHeadDim / 4];
-    __shared__ f4 ps[NW][R][kKC / 4];                    // [wave][row of the wave][key group]
-    __shared__ uint32_t rslot[kQB], rpos[kQB];
-    const int m0 = blockIdx.x * kQB, h = blockIdx.y;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int nq = min(kQB, a.M - m0);
-    if (tid < kQB * kHeadDim / 4) {
-        const int r = tid >> 4, c = tid & 15;
-        qs[r][c] = *reinterpret_cast<const f4*>(a.q + static_cast<size_t>(m0 + min(r, nq - 1)) * kWidth + h * kHeadDim + 4 * c);
-    }
-    if (tid < kQB) {
-        rslot[tid] = tid < nq ? a.row_slot[m0 + tid] : 0u;
-        rpos[tid] = tid < nq ? a.row_pos[m0 + tid] : 0u;
-    }
-    __syncthreads();
-
+// Causal attention over one head for 16 consecutive rows (attn_core.h).  The rows are taken in
+// runs that share a cache slot (stacked sequences: positions restart at 0 in each slot): for
+// each run the slot's keys 0 .. max position, with the other runs' rows seeing none of them
+// (score -inf, weight 0, a rescale of exactly 1).  Later rows have more keys: they start first.
+__global__ __launch_bounds__(64 * kAttnWaves) void causal_attention_kernel(CausalArgs a) {
+    __shared__ AttnLds<kHeadDim> lds;
+    const int m0 = (gridDim.x - 1 - blockIdx.x) * kAttnTile, h = blockIdx.y;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int nq = min(kAttnTile, a.M - m0);
+    const int qr = min(lane & 15, nq - 1);
+    const int slot_q = static_cast<int>(a.row_slot[m0 + qr]), pos_q = static_cast<int>(a.row_pos[m0 + qr]);
+    SplitFrag q[kHeadDim / 32];
+    attn_query<kHeadDim>(a.q + static_cast<size_t>(m0 + qr) * kWidth + h * kHeadDim, lane, q);
+    AttnState<kHeadDim> st;
     for (int r0 = 0; r0 < nq;) {
-        const uint32_t slot = rslot[r0];
-        int r1 = r0 + 1;
-        while (r1 < nq && rslot[r1] == slot) ++r1;
-        int kn = 0;
-        for (int r = r0; r < r1; ++r) kn = max(kn, static_cast<int>(rpos[r]) + 1);
+        const int slot = __builtin_amdgcn_readlane(slot_q, r0);
+        const uint32_t same = static_cast<uint32_t>(__ballot(slot_q == slot)) & ((1u << nq) - 1u) & ~((1u << r0) - 1u);
+        const int r1 = r0 + __popc(same);                                // a slot's rows are consecutive
+        const int kn = __builtin_amdgcn_readlane(pos_q, r1 - 1) + 1;     // and in order
         const float* kb = a.kv + static_cast<size_t>(slot) * a.kv_slot_stride + a.kv_layer_off + static_cast<size_t>(h) * a.kv_cap * kHeadDim;
-        const float* vb = kb + a.kv_v_off;
-        // chunk loads, keys past kn clamped to kn - 1 (masked below):
-        //   K piece j: key tid % 64, dimension group tid / 64 + 8 j (LDS writes conflict-free)
-        //   V piece j: key tid / 16 + 32 j, dimension group tid % 16 (256-byte rows)
-        f4 kr[2], vr[2];
-        auto load_chunk = [&](int c0) {
-#pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                const int kk = min(c0 + lane, kn - 1), kv = min(c0 + (tid >> 4) + 32 * j, kn - 1);
-                kr[j] = *reinterpret_cast<const f4*>(kb + static_cast<size_t>(kk) * kHeadDim + 4 * (wave + NW * j));
-                vr[j] = *reinterpret_cast<const f4*>(vb + static_cast<size_t>(kv) * kHeadDim + 4 * (tid & 15));
-            }
-        };
-        int pos[R];
-        float mrun[R], lrun[R], acc[R];
-#pragma unroll
-        for (int i = 0; i < R; ++i) {
-            const int r = wave + NW * i;
-            pos[i] = r >= r0 && r < r1 ? static_cast<int>(rpos[r]) : -1;  // -1: not in this run
-            mrun[i] = -INFINITY;
-            lrun[i] = 0.0f;
-            acc[i] = 0.0f;
-        }
-        load_chunk(0);
-        for (int c0 = 0; c0 < kn; c0 += kKC) {
-            __syncthreads();  // the previous chunk's readers are done
-#pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                Kt[wave + NW * j][lane] = kr[j];
-                *reinterpret_cast<f4*>(&Vs[(tid >> 4) + 32 * j][4 * (tid & 15)]) = vr[j];
-            }
-            __syncthreads();
-            if (c0 + kKC < kn) load_chunk(c0 + kKC);
-            __builtin_amdgcn_sched_barrier(0);
-            // scores: lane = key
-            float d[R];
-#pragma unroll
-            for (int i = 0; i < R; ++i) d[i] = 0.0f;
-#pragma unroll
-            for (int g = 0; g < kHeadDim / 4; ++g) {
-                const f4 k4 = Kt[g][lane];
-#pragma unroll
-                for (int i = 0; i < R; ++i) {
-                    const f4 q4 = qs[wave + NW * i][g];
-                    d[i] = __builtin_fmaf(q4.x, k4.x, d[i]);
-                    d[i] = __builtin_fmaf(q4.y, k4.y, d[i]);
-                    d[i] = __builtin_fmaf(q4.z, k4.z, d[i]);
-                    d[i] = __builtin_fmaf(q4.w, k4.w, d[i]);
-                }
-            }
-#pragma unroll
-            for (int i = 0; i < R; ++i) {
-                const bool valid = c0 + lane <= pos[i];
-                const float s = valid ? d[i] * 0.125f : -INFINITY;
-                const float cm = wave_max(s);
-                const float mnew = fmaxf(mrun[i], cm);
-                const float corr = mrun[i] == -INFINITY ? 0.0f : expf(mrun[i] - mnew);
-                const float p = valid ? expf(s - mnew) : 0.0f;
-                lrun[i] = lrun[i] * corr + wave_sum(p);
-                acc[i] *= corr;
-                mrun[i] = mnew;
-                reinterpret_cast<float*>(ps[wave][i])[lane] = p;
-            }
-            // acc += p_k V[k], keys in order; lane = dimension
-            const int nkc = min(kKC, kn - c0);
-            for (int k4 = 0; k4 < (nkc + 3) / 4; ++k4) {
-                f4 pv[R];
-#pragma unroll
-                for (int i = 0; i < R; ++i) pv[i] = ps[wave][i][k4];
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const float v = Vs[4 * k4 + e][lane];
-#pragma unroll
-                    for (int i = 0; i < R; ++i) acc[i] = __builtin_fmaf(pv[i][e], v, acc[i]);
-                }
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < R; ++i)
-            if (pos[i] >= 0) split_store(a.out, split_off(m0 + wave + NW * i, h * kHeadDim + lane, kWidth), acc[i] / lrun[i]);
+        const int pos = qr >= r0 && qr < r1 ? pos_q : -1;
+        for (int c0 = wave * kAttnKeys; c0 < kn; c0 += kAttnWaves * kAttnKeys)
+            attn_chunk<kHeadDim>(st, q, kb, kb + a.kv_v_off, c0, kn, pos, 0.125f, lane);
         r0 = r1;
     }
+    float out[4];
+    attn_merge<kHeadDim>(lds, st, wave, lane, out);
+    const int r = tid >> 4;
+    if (r < nq) split_store4(a.out, split_off(m0 + r, h * kHeadDim + 4 * (tid & 15), kWidth), out);
 }
 
 }  // namespace
@@ -582,7 +488,7 @@ hipError_t launch_gemm(const GemmArgs& a, int epi, bool bf16, hipStream_t s) {
 }
 
 hipError_t launch_causal_attention(const CausalArgs& a, hipStream_t s) {
-    hipLaunchKernelGGL(causal_attention_kernel, dim3((a.M + kQB - 1) / kQB, kHeads), dim3(kAttnThreads), 0, s, a);
+    hipLaunchKernelGGL(causal_attention_kernel, dim3(ceil_div(a.M, kAttnTile), kHeads), dim3(64 * kAttnWaves), 0, s, a);
     return hipGetLastError();
 }
 

@@ -41,7 +41,7 @@
 #include <vector>
 
 #include "itts_qwen.h"
-#include "gemm_core.h"
+#include "attn_core.h"
 #include "kernels.h"
 
 namespace itts {
@@ -592,59 +592,23 @@ __global__ __launch_bounds__(256) void q_rms_rows_kernel(const float* x, const f
     split_store4(y, split_off(r, 4 * t, kD), n);
 }
 
-// Causal attention of the prompt rows (qwen_attention, kernels.metal:3119-3129, offset 0): one
-// wave per (row, query head); 64 keys per pass with lane = key for the scores, lanes = the
-// dimension pairs (l, l + 64) for the weighted V sum; online max / sum rescaling.
-__global__ __launch_bounds__(64) void q_causal_attn_kernel(QCausalArgs a) {
-    const int m = blockIdx.x, h = blockIdx.y, lane = threadIdx.x, kvh = h >> 1;
-    __shared__ __align__(16) float qs[kHd];
-    qs[lane] = a.q[static_cast<size_t>(m) * kQ + h * kHd + lane];
-    qs[lane + 64] = a.q[static_cast<size_t>(m) * kQ + h * kHd + lane + 64];
-    __syncthreads();
-    const float* kb = a.kc + static_cast<size_t>(kvh) * kCap * kHd;
-    const float* vb = a.vc + static_cast<size_t>(kvh) * kCap * kHd;
-    float mrun = -INFINITY, lrun = 0.0f, acc1 = 0.0f, acc2 = 0.0f;
-    for (int c0 = 0; c0 <= m; c0 += 64) {
-        const int key = c0 + lane;
-        const bool valid = key <= m;
-        float s = -INFINITY;
-        if (valid) {
-            const float4* kr = reinterpret_cast<const float4*>(kb + static_cast<size_t>(key) * kHd);
-            const float4* q4 = reinterpret_cast<const float4*>(qs);
-            float d = 0.0f;
-#pragma unroll 8
-            for (int i = 0; i < kHd / 4; ++i) d = dot4(q4[i], kr[i], d);
-            s = d * kScale;
-        }
-        const float cm = wave_max(s);
-        const float mnew = fmaxf(mrun, cm);
-        const float corr = mrun == -INFINITY ? 0.0f : expf(mrun - mnew);
-        const float p = valid ? expf(s - mnew) : 0.0f;
-        lrun = lrun * corr + wave_sum(p);
-        acc1 *= corr;
-        acc2 *= corr;
-        const int nk = min(64, m + 1 - c0);
-        for (int k0 = 0; k0 < nk; k0 += 16) {
-            float v1[16], v2[16];
-#pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                const bool ok = k0 + i < nk;
-                const size_t off = static_cast<size_t>(c0 + (ok ? k0 + i : 0)) * kHd + lane;
-                v1[i] = ok ? vb[off] : 0.0f;
-                v2[i] = ok ? vb[off + 64] : 0.0f;
-            }
-#pragma unroll
-            for (int i = 0; i < 16; ++i)
-                if (k0 + i < nk) {
-                    const float pk = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(p), k0 + i));
-                    acc1 = __builtin_fmaf(pk, v1[i], acc1);
-                    acc2 = __builtin_fmaf(pk, v2[i], acc2);
-                }
-        }
-        mrun = mnew;
-    }
-    split_store(a.out, split_off(m, h * kHd + lane, kQ), acc1 / lrun);
-    split_store(a.out, split_off(m, h * kHd + lane + 64, kQ), acc2 / lrun);
+// Causal attention of the prompt rows (qwen_attention, kernels.metal:3119-3129, offset 0): 16 rows
+// of one query head per workgroup (attn_core.h), the last rows (most keys) first.
+__global__ __launch_bounds__(64 * kAttnWaves) void q_causal_attn_kernel(QCausalArgs a) {
+    __shared__ AttnLds<kHd> lds;
+    const int m0 = (gridDim.x - 1 - blockIdx.x) * kAttnTile, h = blockIdx.y;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int nq = min(kAttnTile, a.rows - m0);
+    const int qr = m0 + min(lane & 15, nq - 1), kn = m0 + nq;
+    SplitFrag q[kHd / 32];
+    attn_query<kHd>(a.q + static_cast<size_t>(qr) * kQ + h * kHd, lane, q);
+    const size_t head = static_cast<size_t>(h >> 1) * kCap * kHd;
+    AttnState<kHd> st;
+    for (int c0 = wave * kAttnKeys; c0 < kn; c0 += kAttnWaves * kAttnKeys) attn_chunk<kHd>(st, q, a.kc + head, a.vc + head, c0, kn, qr, kScale, lane);
+    float out[8];
+    attn_merge<kHd>(lds, st, wave, lane, out);
+    const int r = tid >> 4;
+    if (r < nq) split_store_piece(a.out, split_off(m0 + r, h * kHd + 8 * (tid & 15), kQ), out);
 }
 
 #define QWEN_CHECK(x)                                                                                        \
@@ -887,7 +851,7 @@ struct Engine {
             hipLaunchKernelGGL(q_prep_kernel, dim3(P, kQH + 2 * kKVH), dim3(64), 0, s, pa);
             QWEN_CHECK(hipGetLastError());
             QCausalArgs ca{Qp.p, K(l), Vc(l), ATT.p, P};
-            hipLaunchKernelGGL(q_causal_attn_kernel, dim3(P, kQH), dim3(64), 0, s, ca);
+            hipLaunchKernelGGL(q_causal_attn_kernel, dim3((P + kAttnTile - 1) / kAttnTile, kQH), dim3(64 * kAttnWaves), 0, s, ca);
             QWEN_CHECK(hipGetLastError());
             gemm(ATT.p, w + kOffO, P, kD, kQ, X.p, nullptr, kGemmResid);
             hipLaunchKernelGGL(q_rms_rows_kernel, dim3(P), dim3(256), 0, s, X.p, N(l) + kNormPost, Xn.p);

@@ -108,6 +108,30 @@ def test_prefill_and_steps_small(small):
     assert dec.cached_tokens() == orc.cached_tokens()
 
 
+def bf16_round(a):
+    u = np.ascontiguousarray(a, np.float32).view(np.uint32)
+    return ((u + 0x7FFF + ((u >> 16) & 1)) & 0xFFFF0000).astype(np.uint32).view(np.float32)
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+def test_prefill_tile_edges_match_oracle(itts, oracle, dtype):
+    """Prefixes of 1..193 rows, either side of every edge of the prefill kernels' tiles (16-row
+    operand tiles and attention tiles, 32-key chunks over four waves, row blocks of 16 to 192):
+    last-row logits within 2e-5 of the oracle's largest logit, as FP32 sums of up to 5120
+    products over two layers give, whichever instruction forms the products."""
+    w = itts.make_synthetic_weights(layers=2, seed=31, ln_random=True)
+    dec = itts.GptDecoder(w, kv_capacity=256, weight_dtype=dtype)
+    if dtype == "bf16":  # the five matrices rounded as the decoder rounds them (nearest even)
+        matrices = ("attn.c_attn.weight", "attn.c_proj.weight", "mlp.c_fc.weight", "mlp.c_proj.weight", "mel_head.weight")
+        w = {k: bf16_round(v) if k.endswith(matrices) else v for k, v in w.items()}
+    orc = oracle.OracleGpt(w, kv_capacity=256)
+    r = np.random.default_rng(9)
+    for rows in (1, 2, 15, 16, 17, 31, 32, 33, 64, 65, 127, 129, 192, 193):
+        prefix = (0.5 * r.standard_normal((rows, 1280))).astype(np.float32)
+        got, ref = dec.prefill(prefix), orc.prefill(prefix)
+        assert np.max(np.abs(got - ref)) <= 2e-5 * np.max(np.abs(ref)), (rows, np.max(np.abs(got - ref)), np.max(np.abs(ref)))
+
+
 @pytest.mark.parametrize("n_text", [1, 13, 29, 61, 93, 125, 157, 253, 480])
 def test_prefill_row_counts_match_oracle(small, itts, n_text):
     """Prefill logits and the next step against the oracle for prefixes of 36..515 rows: the
