@@ -10,22 +10,23 @@
 // codec's erf form, erf from the Abramowitz-Stegun 7.1.26 polynomial (kernels.metal:3133-3137);
 // "same" convolutions pad kernel/2 zeros on each side (kernels.metal:1397-1426, 1516-1541).
 //
-// Kernels:
+// Kernels (43 launches per decode):
 //   * codec_lookup: one workgroup per code, the 8-wide codebook row times out_project.
-//   * codec_gemm<EPI>: C = A W^T + bias on the FP32 matrix cores (v_mfma_f32_32x32x2f32),
-//     64 x 64 tile per 256-thread workgroup, A with a row stride of its own.  Grids below
-//     about 512 workgroups split K (partial sums, then codec_reduce adds them in split order
-//     and applies the epilogue), since a decode of a few dozen codes gives only a handful of
-//     output tiles.  A "same"
-//     convolution of kernel k over time-major rows is this GEMM with K = k * Cin: row t of A
-//     is the k consecutive input rows t .. t + k - 1 of the zero-padded input (contiguous
-//     in memory, so A is the padded input read with row stride Cin), and the weights are
-//     stored [Cout][k][Cin].  Epilogues: bias; bias + GELU; residual + gamma * (. + bias).
-//   * codec_dwconv_ln: depthwise conv7 + LayerNorm of one 384-wide row per wave.
-//   * codec_ln: LayerNorm of one 384-wide row per wave.
-//   * codec_upsample: nearest x2 in time into the zero-padded input of the last conv.
-// A decode of a given length is captured once as a HIP graph and replayed (about 60 launches,
-// which bound short decodes); the padding rows are written by kernels, not memsets.
+//   * codec_gemm<EPI>: C = A W^T + bias on the matrix cores with split operands (gemm_core.h); every
+//     A is written split by the kernel before.  A "same" convolution of kernel k over time-major
+//     rows is this GEMM with K = k * Cin: row t of A is the k consecutive input rows t .. t + k - 1
+//     of the zero-padded input, so a lane's operand row moves down one row per tap, and the
+//     weights are stored [Cout][k][Cin].
+//   * The conv3 over the doubled rows reads row t twice: out[2t] = w0 y[t-1] + (w1 + w2) y[t] and
+//     out[2t+1] = (w0 + w1) y[t] + w2 y[t+1].  It is one two-tap GEMM over y with 2048 columns
+//     (even, then odd output rows, the odd ones a row further down): two thirds of the
+//     products, and no doubled input.
+//   * codec_rows: everything between two GEMMs of the ConvNeXt stack in one launch: the split sums,
+//     bias, gamma and residual (or the first LayerNorm) of a row and its neighbours, then the
+//     depthwise conv7 and LayerNorm (or the final LayerNorm).  Each row is formed by the
+//     workgroups of four row pairs instead of a launch of its own.
+// A decode of a given length is captured once as a HIP graph and replayed (the launches bound
+// short decodes); the padding rows are written by kernels, not memsets.
 #include <type_traits>
 #include <algorithm>
 #include <cmath>
@@ -37,7 +38,7 @@
 #include <unordered_map>
 #include <vector>
 
-#include "common.h"
+#include "gemm_core.h"
 #include "itts_gpt.h"
 
 namespace itts {
@@ -49,12 +50,12 @@ constexpr int kCF = 2048;        // ConvNeXt hidden width
 constexpr int kCBlocks = 12;
 constexpr int kCK = 7;           // embed / depthwise kernel
 constexpr int kUpK = 3;          // up conv kernel
+constexpr int kUpN = 2 * kCW;    // up conv as a GEMM: even and odd output rows
+constexpr int kUpTaps = 2;
 constexpr int kCodebook = 8192;
 constexpr int kCodeDim = 8;
 constexpr int kMaxCodes = 5000;  // codec.cpp:58
 constexpr float kCodecEps = 1e-6f;
-
-typedef float floatx16 __attribute__((ext_vector_type(16)));
 
 // 0.5 x (1 + erf(x / sqrt 2)), erf by Abramowitz & Stegun 7.1.26 (|error| <= 1.5e-7), the form
 // the reference's codec GELU evaluates.
@@ -66,179 +67,141 @@ __device__ __forceinline__ float codec_gelu(float x) {
     return 0.5f * x * (1.0f + erf);
 }
 
-// Row r of the embed conv's zero-padded input (T + 2 pad rows): rows pad .. pad + T - 1 are the
-// projected codebook rows of the codes, the others zero.
+// Row r of the embed conv's zero-padded input (T + 2 pad rows), split: rows pad .. pad + T - 1 are
+// the projected codebook rows of the codes, the others zero.  The two padding rows of the up
+// conv's input (0 and T + 1 of ypad) are cleared here too.
 __global__ __launch_bounds__(256) void codec_lookup_kernel(const uint32_t* codes, const float* cb, const float* w, const float* b,
-                                                           float* out, int T, int pad) {
+                                                           uint16_t* out, uint16_t* ypad, int T, int pad) {
     const int r = blockIdx.x, tid = threadIdx.x;
+    const float zero[4] = {0.f, 0.f, 0.f, 0.f};
+    if (r < 2) split_store4(ypad, split_off(r * (T + 1), 4 * tid, kCW), zero);
     if (r < pad || r >= T + pad) {
-#pragma unroll
-        for (int i = 0; i < kCW / 256; ++i) out[static_cast<size_t>(r) * kCW + tid + 256 * i] = 0.0f;
+        split_store4(out, split_off(r, 4 * tid, kCW), zero);
         return;
     }
-    const int t = r;
-    __shared__ float e[kCodeDim];
-    if (tid < kCodeDim) e[tid] = cb[static_cast<size_t>(codes[r - pad]) * kCodeDim + tid];
-    __syncthreads();
+    const float* e = cb + static_cast<size_t>(codes[r - pad]) * kCodeDim;
+    const f32x4 e0 = *reinterpret_cast<const f32x4*>(e), e1 = *reinterpret_cast<const f32x4*>(e + 4);
+    float v[4];
 #pragma unroll
-    for (int i = 0; i < kCW / 256; ++i) {
-        const int o = tid + 256 * i;
-        const float* wr = w + static_cast<size_t>(o) * kCodeDim;
+    for (int i = 0; i < 4; ++i) {
+        const int o = 4 * tid + i;
+        const f32x4 w0 = *reinterpret_cast<const f32x4*>(w + static_cast<size_t>(o) * kCodeDim);
+        const f32x4 w1 = *reinterpret_cast<const f32x4*>(w + static_cast<size_t>(o) * kCodeDim + 4);
         float acc = 0.0f;
 #pragma unroll
-        for (int j = 0; j < kCodeDim; ++j) acc = __builtin_fmaf(wr[j], e[j], acc);
-        out[static_cast<size_t>(t) * kCW + o] = acc + b[o];
+        for (int j = 0; j < 4; ++j) acc = __builtin_fmaf(w0[j], e0[j], acc);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc = __builtin_fmaf(w1[j], e1[j], acc);
+        v[i] = acc + b[o];
     }
+    split_store4(out, split_off(r, 4 * tid, kCW), v);
 }
 
-enum CodecEpi : int { kEpiBias = 0, kEpiGelu = 1, kEpiScaleResid = 2 };
+// kEpiPartial: raw sums of K range z to ws[z].  kEpiGelu: GELU, split.  kEpiShift: + bias, split,
+// one row down (the up conv's padded input).  kEpiUp: + bias, columns n >= 1024 to the odd rows.
+enum CodecEpi : int { kEpiPartial = 0, kEpiGelu = 1, kEpiShift = 2, kEpiUp = 3 };
 
 struct CodecGemm {
-    const float* a;      // A rows, lda floats apart (rows may overlap: a convolution window)
-    int lda;
+    const uint16_t* a;   // split operand (of a convolution: the padded rows, kCW wide)
+    int a_rows;          // rows of it
     const float* w;      // [N][K]
     const float* bias;   // [N]
-    const float* gamma;  // kEpiScaleResid: [N]
-    float* c;            // [M][ldc]; kEpiScaleResid: read-modify-write residual
-    int ldc;
+    float* c;            // kEpiUp output
+    uint16_t* cs;        // kEpiGelu, kEpiShift output
     int M, N, K;
-    float* ws;           // split-K partial sums [splits][M][N] (splits > 1)
-    int kchunk;          // K per split (a multiple of GK)
+    float* ws;           // partial sums [splits][M][N]
+    int kchunk;          // K per split
 };
 
-constexpr int GM = 64, GN = 64, GK = 32, GP = 4;
-
-__device__ __forceinline__ float codec_epilogue(int epi, float v, float gamma, const float* p) {
-    if (epi == kEpiBias) return v;
-    if (epi == kEpiGelu) return codec_gelu(v);
-    return *p + v * gamma;  // codec.cpp:46: x + scale(h, gamma)
-}
-
-// One 64 x 64 tile of C over K range [z kchunk, (z + 1) kchunk): 2 x 2 waves of 32 x 32 MFMA
-// tiles, 32 K per LDS stage with the next stage prefetched into registers.  PARTIAL: the raw
-// sums go to ws[z]; otherwise bias and the epilogue are applied in place.
-template <int EPI, bool PARTIAL>
-__global__ __launch_bounds__(256) void codec_gemm_kernel(CodecGemm g) {
-    __shared__ float As[GK][GM + GP];
-    __shared__ float Bs[GK][GN + GP];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = wave >> 1, wn = wave & 1;
-    const int m0 = blockIdx.y * GM, n0 = blockIdx.x * GN;
-    const int k_begin = blockIdx.z * g.kchunk, k_end = min(g.K, k_begin + g.kchunk);
-    const int lrow = tid >> 2, lk = (tid & 3) * 4;  // loader: K pieces lk and lk + 16 of one row
-    const bool arow_ok = m0 + lrow < g.M;
-    const float* arow = g.a + static_cast<size_t>(arow_ok ? m0 + lrow : 0) * g.lda + lk;
-    const float* wrow = g.w + static_cast<size_t>(n0 + lrow) * g.K + lk;
-    const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
-    float4 ra0 = zero, ra1 = zero, rb0, rb1;
-    auto load = [&](int k0) {
-        if (arow_ok) {
-            ra0 = *reinterpret_cast<const float4*>(arow + k0);
-            ra1 = *reinterpret_cast<const float4*>(arow + k0 + 16);
-        }
-        rb0 = *reinterpret_cast<const float4*>(wrow + k0);
-        rb1 = *reinterpret_cast<const float4*>(wrow + k0 + 16);
-    };
-    floatx16 acc;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) acc[i] = 0.0f;
-    load(k_begin);
-    for (int k0 = k_begin; k0 < k_end; k0 += GK) {
-        As[lk + 0][lrow] = ra0.x;
-        As[lk + 1][lrow] = ra0.y;
-        As[lk + 2][lrow] = ra0.z;
-        As[lk + 3][lrow] = ra0.w;
-        As[lk + 16][lrow] = ra1.x;
-        As[lk + 17][lrow] = ra1.y;
-        As[lk + 18][lrow] = ra1.z;
-        As[lk + 19][lrow] = ra1.w;
-        Bs[lk + 0][lrow] = rb0.x;
-        Bs[lk + 1][lrow] = rb0.y;
-        Bs[lk + 2][lrow] = rb0.z;
-        Bs[lk + 3][lrow] = rb0.w;
-        Bs[lk + 16][lrow] = rb1.x;
-        Bs[lk + 17][lrow] = rb1.y;
-        Bs[lk + 18][lrow] = rb1.z;
-        Bs[lk + 19][lrow] = rb1.w;
-        __syncthreads();
-        if (k0 + GK < k_end) load(k0 + GK);
-#pragma unroll
-        for (int kk = 0; kk < GK; kk += 2) {
-            const float av = As[kk + (lane >> 5)][wm * 32 + (lane & 31)];
-            const float bv = Bs[kk + (lane >> 5)][wn * 32 + (lane & 31)];
-            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(av, bv, acc, 0, 0, 0);
-        }
-        __syncthreads();
+template <class T, int EPI, bool CONV>
+__global__ __launch_bounds__(kGemmThreads) void codec_gemm_kernel(CodecGemm g) {
+    __shared__ __align__(16) uint8_t lds[T::kLdsBytes];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const auto [bx, by, bz] = gemm_place();
+    const int kb = bz * g.kchunk, nst = (min(g.K, kb + g.kchunk) - kb) / 32;
+    uint16_t* ring = reinterpret_cast<uint16_t*>(lds);
+    if (wave >= 4) {
+        gemm_loader<T>(ring, g.w + static_cast<size_t>(bx) * T::BN * g.K + kb, g.K, nst, tid - 256);
+        return;
     }
-    // D layout of v_mfma_f32_32x32x2f32: lane l, element i -> row 8(i/4) + 4(l/32) + i%4, col l%32.
-    const int col = n0 + wn * 32 + (lane & 31);
-    auto row_of = [&](int i) { return m0 + wm * 32 + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3); };
-    if constexpr (PARTIAL) {
-        // Every destination formed before the first store: with one register pair reused for
-        // each row's address, the compiler waited for each store to complete before forming
-        // the next address.
-        size_t dst[16];  // element offsets into ws (rows past M are formed, never stored to)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            dst[i] = (static_cast<size_t>(blockIdx.z) * g.M + row_of(i)) * g.N + col;
-            asm volatile("" ::"v"(dst[i]));
-        }
-#pragma unroll
-        for (int i = 0; i < 16; ++i)
-            if (row_of(i) < g.M) g.ws[dst[i]] = acc[i];
+    constexpr int TR = T::TR, TC = T::TC;
+    const int wr = wave / T::WC, wc = wave % T::WC;
+    const int tile0 = by * T::RT + wr * TR;
+    const int akt = CONV ? kCW / 32 : g.K / 32;  // k steps of an operand row
+    const __amdgpu_buffer_rsrc_t ars = gemm_rsrc(g.a, static_cast<uint32_t>(split_elems(g.a_rows, akt * 32) * 2));
+    f32x4 acc[TR][TC];
+    if constexpr (CONV) {
+        // k step s is step s % 32 of tap s / 32, which reads a row further down; rows past the
+        // operand's buffer read as zero (result rows past M only)
+        const int row0 = tile0 * 16 + (lane & 15) + (bx * T::BN >= kCW ? 1 : 0);  // (the up conv's odd rows)
+        gemm_compute<T>(
+            ring, ars,
+            [&](int i, int s) {
+                const int sg = kb / 32 + s, row = row0 + 16 * i + (sg >> 5);
+                return GemmOff{static_cast<uint32_t>(row >> 4) * (kCW / 32 * kTileElems * 2) + ((row & 15) + (lane & 48)) * 16,
+                               static_cast<uint32_t>(sg & 31) * (kTileElems * 2)};
+            },
+            nst, wc, lane, acc);
     } else {
-        // Bias and gamma read once, every row's residual requested before the first store (rows
-        // past M reread row M - 1, in bounds, and store nothing), and every value formed before
-        // the first store.  Read per element behind the stores into C, which may alias them,
-        // each was a memory round trip; and a use of a load inside a row's branch made the
-        // compiler wait there for every access in flight, the earlier rows' stores included.
-        const float bias = g.bias[col], gamma = EPI == kEpiScaleResid ? g.gamma[col] : 0.0f;
-        float res[16], out[16];
+        const int tiles = (g.M + 15) / 16;
+        uint32_t off[TR];
 #pragma unroll
-        for (int i = 0; i < 16; ++i)
-            res[i] = EPI == kEpiScaleResid ? g.c[static_cast<size_t>(min(row_of(i), g.M - 1)) * g.ldc + col] : 0.0f;
+        for (int i = 0; i < TR; ++i) off[i] = (static_cast<uint32_t>(min(tile0 + i, tiles - 1)) * akt + kb / 32) * (kTileElems * 2) + lane * 16;
+        gemm_compute<T>(
+            ring, ars, [&](int i, int s) { return GemmOff{off[i], static_cast<uint32_t>(s) * (kTileElems * 2)}; }, nst, wc, lane, acc);
+    }
+    const int cw = bx * T::BN + wc * TC * 16, col0 = cw + (lane & 15);
+    if constexpr (EPI == kEpiPartial) {
+        gemm_store_partial<T>(g.ws + static_cast<size_t>(bz) * g.M * g.N, g.M, g.N, tile0, col0, lane, acc);
+    } else {
+        float bias[TC];
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            out[i] = codec_epilogue(EPI, acc[i] + bias, gamma, &res[i]);
-            asm volatile("" ::"v"(out[i]));  // formed here, not sunk into the row's branch
-        }
+        for (int c = 0; c < TC; ++c) bias[c] = g.bias[col0 + 16 * c];
+        if constexpr (EPI == kEpiGelu) {
+            gemm_store_split<T, false>(lds, wave, lane, g.cs, g.M, g.N, 0, tile0, cw,
+                                       [&](int i, int c, int r) { return codec_gelu(acc[i][c][r] + bias[c]); });
+        } else if constexpr (EPI == kEpiShift) {
+            gemm_store_split<T, false>(lds, wave, lane, g.cs, g.M, g.N, 1, tile0, cw, [&](int i, int c, int r) { return acc[i][c][r] + bias[c]; });
+        } else {
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const int row = row_of(i);
-            if (row < g.M) g.c[static_cast<size_t>(row) * g.ldc + col] = out[i];
+            for (int i = 0; i < TR; ++i) {
+                const int row = (tile0 + i) * 16 + 4 * (lane >> 4);
+#pragma unroll
+                for (int c = 0; c < TC; ++c)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        acc[i][c][r] += bias[c];
+                        pin_value(acc[i][c][r]);
+                    }
+                const int odd = cw >= kCW ? 1 : 0;
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (row + r < g.M) {
+                        float* p = g.c + (2 * static_cast<size_t>(row + r) + odd) * kCW + (col0 & (kCW - 1));
+#pragma unroll
+                        for (int c = 0; c < TC; ++c) p[16 * c] = acc[i][c][r];
+                    }
+            }
         }
     }
 }
 
-// Split-K: C = epilogue(sum over splits z = 0, 1, ... of ws[z] + bias), in split order, so
-// the result does not depend on which split finished first.
-template <int EPI>
-__global__ __launch_bounds__(256) void codec_reduce_kernel(CodecGemm g, int splits) {
-    const size_t i = static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x, total = static_cast<size_t>(g.M) * g.N;
-    if (i >= total) return;
-    const int row = static_cast<int>(i / g.N), col = static_cast<int>(i % g.N);
-    float* p = g.c + static_cast<size_t>(row) * g.ldc + col;
-    const float bias = g.bias[col], gamma = EPI == kEpiScaleResid ? g.gamma[col] : 0.0f;
-    const float res = EPI == kEpiScaleResid ? *p : 0.0f;
-    // every split's partial requested before the first add (SM >= splits; indices past the split
-    // count reread the last split and are not added): a loop of dependent adds over loads issued
-    // one at a time made each split a memory round trip
-    auto sum = [&](auto sm) {
-        constexpr int SM = decltype(sm)::value;
-        float w[SM];
+// The up conv's splits, added in split order, + bias; a thread takes four columns.
+template <int SM>
+__global__ __launch_bounds__(256) void codec_up_reduce_kernel(CodecGemm g, int splits) {
+    const size_t e = (static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x) * 4, plane = static_cast<size_t>(g.M) * kUpN;
+    if (e >= plane) return;
+    const size_t row = e / kUpN;
+    const int n = static_cast<int>(e % kUpN);
+    f32x4 w[SM];
 #pragma unroll
-        for (int z = 0; z < SM; ++z) w[z] = g.ws[static_cast<size_t>(min(z, splits - 1)) * total + i];
-        float s = 0.0f;
+    for (int z = 0; z < SM; ++z) w[z] = *reinterpret_cast<const f32x4*>(g.ws + static_cast<size_t>(min(z, splits - 1)) * plane + e);
+    f32x4 d = w[0];
 #pragma unroll
-        for (int z = 0; z < SM; ++z)
-            if (z < splits) s += w[z];
-        return s;
-    };
-    const float s = splits <= 4 ? sum(std::integral_constant<int, 4>{})
-                    : splits <= 8 ? sum(std::integral_constant<int, 8>{})
-                    : splits <= 16 ? sum(std::integral_constant<int, 16>{})
-                                   : sum(std::integral_constant<int, 32>{});
-    *p = codec_epilogue(EPI, s + bias, gamma, &res);
+    for (int z = 1; z < SM; ++z)
+        if (z < splits) d += w[z];
+    *reinterpret_cast<f32x4*>(g.c + (2 * row + (n >= kCW ? 1 : 0)) * kCW + (n & (kCW - 1))) = d + *reinterpret_cast<const f32x4*>(g.bias + n);
 }
 
 // LayerNorm of a 384-wide row held as 6 values per lane (columns lane + 64 i): mean, then
@@ -266,58 +229,92 @@ __device__ __forceinline__ void ln384(float (&v)[6], const float* gw, const floa
     }
 }
 
-// Depthwise conv7 (same padding) of row t, then LayerNorm: one wave per row, 4 rows per workgroup.
-__global__ __launch_bounds__(256) void codec_dwconv_ln_kernel(const float* x, const float* dw, const float* db, const float* gw,
-                                                              const float* gb, float* out, int T) {
-    const int lane = threadIdx.x & 63, t = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (t >= T) return;
-    // All 42 loads first (rows clamped into [0, T), taps outside it zeroed), so they are in
-    // flight together instead of one tap's branch at a time.
-    float xv[kCK][6];
+// Rows between the GEMMs.  x row = LayerNorm(split sum + bias) (FIRST: after the embed conv) or
+// x_in + gamma * (split sum + bias) (after pwconv2); then, with DW, the depthwise conv7 of x (same
+// padding) and LayerNorm, else LayerNorm alone; split.  A workgroup of eight waves owns two rows:
+// with DW each wave forms one of the eight rows they read (three before, three after, zeros
+// outside [0, T)), so the neighbours' split sums are read again (from L2) instead of a launch
+// between them; the owned rows go to x_out, which is not x_in (the neighbours read that).
+struct CodecRows {
+    const float* ws;
+    int splits, T;
+    const float *bias, *gamma, *x_in;
+    float* x_out;
+    const float *fw, *fb;    // FIRST: its LayerNorm
+    const float *dw, *db;    // depthwise conv
+    const float *lw, *lb;    // the LayerNorm at the end
+    uint16_t* out;
+};
+constexpr int kRowsOwn = 2, kRowsWaves = 8;
+
+template <bool FIRST, bool DW>
+__global__ __launch_bounds__(64 * kRowsWaves) void codec_rows_kernel(CodecRows a) {
+    __shared__ float xs[kRowsWaves][kCH];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int halo = DW ? kCK / 2 : 0;
+    const int t0 = blockIdx.x * kRowsOwn, t = t0 + wave - halo;
+    const bool live = t >= 0 && t < a.T && wave < kRowsOwn + 2 * halo;
+    float v[6];
 #pragma unroll
-    for (int k = 0; k < kCK; ++k) {
-        const int src = t + k - kCK / 2;
-        const int row = min(max(src, 0), T - 1);
+    for (int i = 0; i < 6; ++i) v[i] = 0.0f;
+    if (live) {
+        const size_t row = static_cast<size_t>(t) * kCH + lane, plane = static_cast<size_t>(a.T) * kCH;
+        float res[6], bias[6], gamma[6];
 #pragma unroll
-        for (int i = 0; i < 6; ++i) xv[k][i] = x[static_cast<size_t>(row) * kCH + lane + 64 * i];
-        if (src < 0 || src >= T) {
+        for (int i = 0; i < 6; ++i) {
+            bias[i] = a.bias[lane + 64 * i];
+            res[i] = FIRST ? 0.0f : a.x_in[row + 64 * i];
+            gamma[i] = FIRST ? 1.0f : a.gamma[lane + 64 * i];
+        }
+        // every split's partial of a group requested before its first add; in split order
+        auto sum = [&](auto sm) {
+            constexpr int SM = decltype(sm)::value;
+            for (int z0 = 0; z0 < a.splits; z0 += SM) {
+                float w[SM][6];
 #pragma unroll
-            for (int i = 0; i < 6; ++i) xv[k][i] = 0.0f;
+                for (int z = 0; z < SM; ++z)
+#pragma unroll
+                    for (int i = 0; i < 6; ++i) w[z][i] = a.ws[static_cast<size_t>(min(z0 + z, a.splits - 1)) * plane + row + 64 * i];
+#pragma unroll
+                for (int z = 0; z < SM; ++z)
+                    if (z0 + z < a.splits) {
+#pragma unroll
+                        for (int i = 0; i < 6; ++i) v[i] += w[z][i];
+                    }
+            }
+        };
+        if (a.splits <= 2) sum(std::integral_constant<int, 2>{});
+        else if (a.splits <= 4) sum(std::integral_constant<int, 4>{});
+        else sum(std::integral_constant<int, 8>{});
+#pragma unroll
+        for (int i = 0; i < 6; ++i) v[i] = FIRST ? v[i] + bias[i] : res[i] + (v[i] + bias[i]) * gamma[i];  // codec.cpp:46: x + scale(h, gamma)
+        if constexpr (FIRST) ln384(v, a.fw, a.fb, lane);
+        if (DW && wave >= halo && wave < halo + kRowsOwn) {
+#pragma unroll
+            for (int i = 0; i < 6; ++i) a.x_out[row + 64 * i] = v[i];
         }
     }
-    float v[6];
+    int ot = t;
+    if constexpr (DW) {
 #pragma unroll
-    for (int i = 0; i < 6; ++i) {
-        const int c = lane + 64 * i;
-        float acc = db[c];
+        for (int i = 0; i < 6; ++i) xs[wave][lane + 64 * i] = v[i];
+        __syncthreads();
+        ot = t0 + wave;
+        if (wave >= kRowsOwn || ot >= a.T) return;
 #pragma unroll
-        for (int k = 0; k < kCK; ++k) acc += xv[k][i] * dw[c * kCK + k];
-        v[i] = acc;
+        for (int i = 0; i < 6; ++i) {
+            const int c = lane + 64 * i;
+            float acc = a.db[c];
+#pragma unroll
+            for (int k = 0; k < kCK; ++k) acc += xs[wave + k][c] * a.dw[c * kCK + k];
+            v[i] = acc;
+        }
+    } else if (!live) {
+        return;
     }
-    ln384(v, gw, gb, lane);
+    ln384(v, a.lw, a.lb, lane);
 #pragma unroll
-    for (int i = 0; i < 6; ++i) out[static_cast<size_t>(t) * kCH + lane + 64 * i] = v[i];
-}
-
-// LayerNorm of each 384-wide row (in place allowed): one wave per row.
-__global__ __launch_bounds__(256) void codec_ln_kernel(const float* x, const float* gw, const float* gb, float* out, int T) {
-    const int lane = threadIdx.x & 63, t = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (t >= T) return;
-    float v[6];
-#pragma unroll
-    for (int i = 0; i < 6; ++i) v[i] = x[static_cast<size_t>(t) * kCH + lane + 64 * i];
-    ln384(v, gw, gb, lane);
-#pragma unroll
-    for (int i = 0; i < 6; ++i) out[static_cast<size_t>(t) * kCH + lane + 64 * i] = v[i];
-}
-
-// upad row 1 + j = y row floor(j * 0.5) (the reference's scale in/out = 0.5) for j < 2T; rows
-// 0 and 2T + 1 are the conv's zero padding.
-__global__ __launch_bounds__(256) void codec_upsample_kernel(const float* y, float* upad, int T) {
-    const int j = blockIdx.x;  // 0 .. 2T + 1
-    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (j > 0 && j <= 2 * T) v = reinterpret_cast<const float4*>(y + static_cast<size_t>((j - 1) / 2) * kCW)[threadIdx.x];
-    reinterpret_cast<float4*>(upad + static_cast<size_t>(j) * kCW)[threadIdx.x] = v;  // 256 threads x float4 = 1024 floats
+    for (int i = 0; i < 6; ++i) split_store(a.out, split_off(ot, lane + 64 * i, kCH), v[i]);
 }
 
 #define CODEC_CHECK(x)                                                                                                  \
@@ -351,12 +348,9 @@ struct Buf {
     }
 };
 
-// Splits of K that bring a small grid up to about 512 workgroups, each split at least 256 deep.
-inline int codec_splits(int M, int N, int K) {
-    const int tiles = (N / GN) * ((M + GM - 1) / GM);
-    int s = std::max(1, std::min((512 + tiles - 1) / tiles, K / 256));
-    return std::min(s, 32);
-}
+// At most this many K splits of a GEMM whose partial sums the next kernel adds anyway.
+constexpr int kCodecSplits = 32;
+constexpr size_t kCodecWsFloats = size_t(16) << 20;  // and at most this many partial sums, except of one split
 
 }  // namespace
 
@@ -373,7 +367,8 @@ struct CodecEngine {
     struct Block {
         Buf<float> dw, db, lw, lb, w1, b1, w2, b2, gamma;
     } blk[kCBlocks];
-    Buf<float> xpad, x, hn, f, y, upad, out, ws;
+    Buf<uint16_t> xpad, hn, f, ypad;  // split GEMM operands (gemm_core.h)
+    Buf<float> x[2], out, ws;
     Buf<uint32_t> dcodes;
     // Decodes of one length replay a captured graph (ITTS_CODEC_GRAPHS=0: eager launches).  A
     // buffer that moves bumps `generation`, and graphs captured before are dropped.
@@ -381,16 +376,13 @@ struct CodecEngine {
     uint64_t generation = 0, graph_generation = 0;
     std::unordered_map<int, hipGraphExec_t> graphs;
 
-    static int used_splits(int M, int N, int K, int* kchunk) {
-        const int splits = codec_splits(M, N, K);
-        *kchunk = ((K + splits - 1) / splits + GK - 1) / GK * GK;
-        return (K + *kchunk - 1) / *kchunk;
+    static GemmPlan plan(int M, int N, int K, int max_splits, bool reduce) {
+        const size_t mn = static_cast<size_t>(M) * N;
+        return gemm_plan(M, N, K, std::max(1, std::min<int>(max_splits, static_cast<int>(kCodecWsFloats / mn))), false, reduce);
     }
-    static size_t ws_need(int M, int N, int K) {
-        int kc = 0;
-        const int used = used_splits(M, N, K, &kc);
-        return used > 1 ? static_cast<size_t>(used) * M * N : 0;
-    }
+    static GemmPlan embed_plan(int T) { return plan(T, kCH, kCK * kCW, kCodecSplits, false); }
+    static GemmPlan pw2_plan(int T) { return plan(T, kCH, kCF, kCodecSplits, false); }
+    static GemmPlan up_plan(int T) { return plan(T, kUpN, kUpTaps * kCW, 8, true); }
     template <class B>
     void grow(B& b, size_t n) {
         if (b.ensure(n)) ++generation;
@@ -399,33 +391,25 @@ struct CodecEngine {
     void reserve(int T) {
         const size_t pad = kCK / 2;
         grow(dcodes, T);
-        grow(xpad, (T + 2 * pad) * kCW);
-        grow(x, static_cast<size_t>(T) * kCH);
-        grow(hn, static_cast<size_t>(T) * kCH);
-        grow(f, static_cast<size_t>(T) * kCF);
-        grow(y, static_cast<size_t>(T) * kCW);
-        grow(upad, static_cast<size_t>(2 * T + 2) * kCW);
+        grow(xpad, split_elems(T + 2 * pad, kCW));
+        for (auto& b : x) grow(b, static_cast<size_t>(T) * kCH);
+        grow(hn, split_elems(T, kCH));
+        grow(f, split_elems(T, kCF));
+        grow(ypad, split_elems(T + 2, kCW));
         grow(out, static_cast<size_t>(2 * T) * kCW);
-        size_t w = std::max({ws_need(T, kCH, kCK * kCW), ws_need(T, kCF, kCH), ws_need(T, kCH, kCF), ws_need(T, kCW, kCH),
-                             ws_need(2 * T, kCW, kUpK * kCW)});
-        grow(ws, std::max<size_t>(w, 1));
+        grow(ws, static_cast<size_t>(T) * std::max({embed_plan(T).splits * kCH, pw2_plan(T).splits * kCH, up_plan(T).splits * kUpN}));
     }
 
-    template <int EPI>
-    void gemm(CodecGemm g) {
-        if (g.N % GN || g.K % GK || g.M < 1) throw std::logic_error("codec GEMM shape");
-        const int used = used_splits(g.M, g.N, g.K, &g.kchunk);
-        const dim3 grid(g.N / GN, (g.M + GM - 1) / GM, used);
-        if (used == 1) {
-            hipLaunchKernelGGL((codec_gemm_kernel<EPI, false>), grid, dim3(256), 0, stream, g);
-        } else {
-            if (ws.n < static_cast<size_t>(used) * g.M * g.N) throw std::logic_error("codec split-K workspace not reserved");
-            g.ws = ws.p;
-            hipLaunchKernelGGL((codec_gemm_kernel<EPI, true>), grid, dim3(256), 0, stream, g);
-            CODEC_CHECK(hipGetLastError());
-            const size_t total = static_cast<size_t>(g.M) * g.N;
-            hipLaunchKernelGGL(codec_reduce_kernel<EPI>, dim3(static_cast<unsigned>((total + 255) / 256)), dim3(256), 0, stream, g, used);
-        }
+    template <int EPI, bool CONV>
+    void gemm(CodecGemm g, const GemmPlan& p) {
+        if (g.N % kGemmBn || g.K % kGemmK || g.M < 1) throw std::logic_error("codec GEMM shape");
+        if (EPI == kEpiPartial && ws.n < static_cast<size_t>(p.splits) * g.M * g.N) throw std::logic_error("codec split-K workspace not reserved");
+        if (EPI != kEpiPartial && p.splits != 1) throw std::logic_error("codec GEMM splits");
+        g.ws = ws.p;
+        g.kchunk = p.kchunk;
+        gemm_tile<float>(p.tile, [&](auto t) {
+            hipLaunchKernelGGL((codec_gemm_kernel<decltype(t), EPI, CONV>), dim3(g.N / kGemmBn, p.mblocks, p.splits), dim3(kGemmThreads), 0, stream, g);
+        });
         CODEC_CHECK(hipGetLastError());
     }
     std::string last_error;
@@ -481,8 +465,23 @@ struct CodecEngine {
         fin_b.upload(vec(get(d + ".final_layer_norm.bias", {kCH}), kCH));
         dec_w.upload(vec(get("codec.decoder.1.weight", {kCW, kCH}), static_cast<size_t>(kCW) * kCH));
         dec_b.upload(vec(get("codec.decoder.1.bias", {kCW}), kCW));
-        up_w.upload(conv_w(get("codec.up.weight", {kCW, kCW, kUpK}), kCW, kCW, kUpK));
-        up_b.upload(vec(get("codec.up.bias", {kCW}), kCW));
+        // even rows: taps w0 | w1 + w2 (rows t - 1, t); odd rows: w0 + w1 | w2 (rows t, t + 1)
+        const float* uw = get("codec.up.weight", {kCW, kCW, kUpK});
+        const float* ub = get("codec.up.bias", {kCW});
+        std::vector<float> up(static_cast<size_t>(kUpN) * kUpTaps * kCW), upb(kUpN);
+        for (int o = 0; o < kCW; ++o) {
+            float *ev = &up[static_cast<size_t>(o) * kUpTaps * kCW], *od = &up[static_cast<size_t>(kCW + o) * kUpTaps * kCW];
+            for (int i = 0; i < kCW; ++i) {
+                const float* w = uw + (static_cast<size_t>(o) * kCW + i) * kUpK;
+                ev[i] = w[0];
+                ev[kCW + i] = w[1] + w[2];
+                od[i] = w[0] + w[1];
+                od[kCW + i] = w[2];
+            }
+            upb[o] = upb[kCW + o] = ub[o];
+        }
+        up_w.upload(up);
+        up_b.upload(upb);
         const char* env = std::getenv("ITTS_CODEC_GRAPHS");
         use_graphs = !(env && std::strcmp(env, "0") == 0);
         CODEC_CHECK(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
@@ -500,25 +499,44 @@ struct CodecEngine {
     void enqueue(int T) {
         const int pad = kCK / 2;
         hipStream_t s = stream;
-        hipLaunchKernelGGL(codec_lookup_kernel, dim3(T + 2 * pad), dim3(256), 0, s, dcodes.p, cb.p, op_w.p, op_b.p, xpad.p, T, pad);
+        hipLaunchKernelGGL(codec_lookup_kernel, dim3(T + 2 * pad), dim3(256), 0, s, dcodes.p, cb.p, op_w.p, op_b.p, xpad.p, ypad.p, T, pad);
         CODEC_CHECK(hipGetLastError());
-        const int rows4 = (T + 3) / 4;
-        gemm<kEpiBias>({xpad.p, kCW, emb_w.p, emb_b.p, nullptr, x.p, kCH, T, kCH, kCK * kCW, nullptr, 0});
-        hipLaunchKernelGGL(codec_ln_kernel, dim3(rows4), dim3(256), 0, s, x.p, n0_w.p, n0_b.p, x.p, T);
+        const dim3 rows((T + kRowsOwn - 1) / kRowsOwn), threads(64 * kRowsWaves);
+        const GemmPlan pe = embed_plan(T), p2 = pw2_plan(T), pu = up_plan(T), p1 = plan(T, kCF, kCH, 1, false), pd = plan(T, kCW, kCH, 1, false);
+        gemm<kEpiPartial, true>({xpad.p, T + 2 * pad, emb_w.p, nullptr, nullptr, nullptr, T, kCH, kCK * kCW, nullptr, 0}, pe);
+        hipLaunchKernelGGL((codec_rows_kernel<true, true>), rows, threads, 0, s,
+                           CodecRows{ws.p, pe.splits, T, emb_b.p, nullptr, nullptr, x[0].p, n0_w.p, n0_b.p, blk[0].dw.p, blk[0].db.p, blk[0].lw.p,
+                                     blk[0].lb.p, hn.p});
         CODEC_CHECK(hipGetLastError());
         for (int i = 0; i < kCBlocks; ++i) {
             const Block& b = blk[i];
-            hipLaunchKernelGGL(codec_dwconv_ln_kernel, dim3(rows4), dim3(256), 0, s, x.p, b.dw.p, b.db.p, b.lw.p, b.lb.p, hn.p, T);
+            gemm<kEpiGelu, false>({hn.p, T, b.w1.p, b.b1.p, nullptr, f.p, T, kCF, kCH, nullptr, 0}, p1);
+            gemm<kEpiPartial, false>({f.p, T, b.w2.p, nullptr, nullptr, nullptr, T, kCH, kCF, nullptr, 0}, p2);
+            CodecRows r{ws.p, p2.splits, T, b.b2.p, b.gamma.p, x[i & 1].p, x[1 - (i & 1)].p, nullptr, nullptr, nullptr, nullptr, fin_w.p, fin_b.p, hn.p};
+            if (i + 1 < kCBlocks) {
+                const Block& n = blk[i + 1];
+                r.dw = n.dw.p;
+                r.db = n.db.p;
+                r.lw = n.lw.p;
+                r.lb = n.lb.p;
+                hipLaunchKernelGGL((codec_rows_kernel<false, true>), rows, threads, 0, s, r);
+            } else {
+                hipLaunchKernelGGL((codec_rows_kernel<false, false>), rows, threads, 0, s, r);
+            }
             CODEC_CHECK(hipGetLastError());
-            gemm<kEpiGelu>({hn.p, kCH, b.w1.p, b.b1.p, nullptr, f.p, kCF, T, kCF, kCH, nullptr, 0});
-            gemm<kEpiScaleResid>({f.p, kCF, b.w2.p, b.b2.p, b.gamma.p, x.p, kCH, T, kCH, kCF, nullptr, 0});
         }
-        hipLaunchKernelGGL(codec_ln_kernel, dim3(rows4), dim3(256), 0, s, x.p, fin_w.p, fin_b.p, hn.p, T);
+        gemm<kEpiShift, false>({hn.p, T, dec_w.p, dec_b.p, nullptr, ypad.p, T, kCW, kCH, nullptr, 0}, pd);
+        const CodecGemm u{ypad.p, T + 2, up_w.p, up_b.p, out.p, nullptr, T, kUpN, kUpTaps * kCW, ws.p, 0};
+        if (pu.splits == 1) {
+            gemm<kEpiUp, true>(u, pu);
+            return;
+        }
+        gemm<kEpiPartial, true>(u, pu);
+        const dim3 ug(static_cast<unsigned>((static_cast<size_t>(T) * kUpN / 4 + 255) / 256));
+        if (pu.splits <= 2) hipLaunchKernelGGL(codec_up_reduce_kernel<2>, ug, dim3(256), 0, s, u, pu.splits);
+        else if (pu.splits <= 4) hipLaunchKernelGGL(codec_up_reduce_kernel<4>, ug, dim3(256), 0, s, u, pu.splits);
+        else hipLaunchKernelGGL(codec_up_reduce_kernel<8>, ug, dim3(256), 0, s, u, pu.splits);
         CODEC_CHECK(hipGetLastError());
-        gemm<kEpiBias>({hn.p, kCH, dec_w.p, dec_b.p, nullptr, y.p, kCW, T, kCW, kCH, nullptr, 0});
-        hipLaunchKernelGGL(codec_upsample_kernel, dim3(2 * T + 2), dim3(256), 0, s, y.p, upad.p, T);
-        CODEC_CHECK(hipGetLastError());
-        gemm<kEpiBias>({upad.p, kCW, up_w.p, up_b.p, nullptr, out.p, kCW, 2 * T, kCW, kUpK * kCW, nullptr, 0});
     }
 
     void drop_graphs() {

@@ -215,13 +215,16 @@ __device__ __forceinline__ void gemm_loader(uint16_t* ring, const typename T::W*
 }
 
 // ------------------------------------------------------------------ multiplying waves
-// acc[i][c] = (row tile i) x (strip c) over nst k steps.  ars: the split operand; aoff[i]: this
-// lane's byte offset of row tile i's first k step.  The next strip's weights are read from LDS
+// acc[i][c] = (row tile i) x (strip c) over nst k steps.  ars: the split operand; aoff(i, s): this
+// lane's byte offset of row tile i at k step s (of nst), and the part of it that is uniform.  The next strip's weights are read from LDS
 // while the current one's matrix instructions run (the first strip of step s + 1 too: the
 // loading waves finished it before the barrier ahead of step s).
-template <class T>
-__device__ __forceinline__ void gemm_compute(const uint16_t* ring, __amdgpu_buffer_rsrc_t ars, const uint32_t (&aoff)[T::TR], int nst,
-                                             int wc, int lane, f32x4 (&acc)[T::TR][T::TC]) {
+struct GemmOff {
+    uint32_t lane, uniform;
+};
+template <class T, class AOff>
+__device__ __forceinline__ void gemm_compute(const uint16_t* ring, __amdgpu_buffer_rsrc_t ars, AOff aoff, int nst, int wc, int lane,
+                                             f32x4 (&acc)[T::TR][T::TC]) {
     bf16x8 av[T::NA][T::TR][3], bv[2][T::PB];
     f32x4 low[T::NLOW][T::TR][T::TC];
 #pragma unroll
@@ -231,9 +234,13 @@ __device__ __forceinline__ void gemm_compute(const uint16_t* ring, __amdgpu_buff
 #pragma unroll
             for (int c = 0; c < T::TC; ++c) low[q][i][c] = f32x4{0.f, 0.f, 0.f, 0.f};
     auto load_a = [&](int set, int s, int i, int p) {  // plane p of row tile i; steps past the last reread it
-        const uint32_t so = static_cast<uint32_t>(min(s, nst - 1)) * (kTileElems * 2);
-        av[set][i][p] = __builtin_bit_cast(bf16x8, gemm_load16(ars, aoff[i] + p * kPlaneElems * 2, so));
+        const GemmOff o = aoff(i, min(s, nst - 1));
+        av[set][i][p] = __builtin_bit_cast(bf16x8, gemm_load16(ars, o.lane + p * kPlaneElems * 2, o.uniform));
     };
+#pragma unroll
+    for (int i = 0; i < T::TR; ++i)
+#pragma unroll
+        for (int c = 0; c < T::TC; ++c) acc[i][c] = f32x4{0.f, 0.f, 0.f, 0.f};
     const int g = lane >> 4;
     const uint16_t* src = ring + wc * T::TC * T::PB * kPlaneElems + (16 * g + ((lane & 15) ^ (2 * g))) * 8;
     int buf = 0;
@@ -299,6 +306,115 @@ __device__ __forceinline__ void gemm_compute(const uint16_t* ring, __amdgpu_buff
     for (int i = 0; i < T::TR; ++i)
 #pragma unroll
         for (int c = 0; c < T::TC; ++c) acc[i][c] += T::NLOW == 2 ? low[0][i][c] + low[1][i][c] : low[0][i][c];
+}
+
+// ------------------------------------------------------------------ placement and results
+// A value held in a register at this point of the program: an empty asm takes it.  The
+// epilogues form every output (and read every loaded operand) before the first row's store
+// this way; left to the compiler, each row's arithmetic sank into that row's branch, where the
+// use of a load still in flight made it wait for every memory access outstanding, the
+// earlier rows' stores included (one store completion per row).
+template <typename T>
+__device__ __forceinline__ void pin_value(T v) {
+    asm volatile("" ::"v"(v));
+}
+
+// Workgroup L runs on XCD L % 8 (round-robin dispatch).  The logical index j gives each XCD one
+// contiguous range, row blocks (y) fastest, then splits (z), then column tiles (x), so the
+// workgroups sharing a column tile's weights mostly share one L2.
+struct GemmPlace {
+    int x, y, z;
+};
+__device__ __forceinline__ GemmPlace gemm_place() {
+    const int nwg = gridDim.x * gridDim.y * gridDim.z;
+    const int L = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
+    const int per = nwg / 8, rem = nwg % 8, xcd = L % 8;
+    const int j = (xcd < rem ? xcd * (per + 1) : rem * (per + 1) + (xcd - rem) * per) + L / 8;
+    return {j / static_cast<int>(gridDim.y * gridDim.z), j % static_cast<int>(gridDim.y), (j / static_cast<int>(gridDim.y)) % static_cast<int>(gridDim.z)};
+}
+
+// A wave's results lie at rows 16 (tile0 + i) + rq + r (rq = 4 (lane / 16)), columns col0 + 16 c:
+// acc[i][c][r].  Raw partial sums to ws[M][N].  Every destination's 32-bit element offset is
+// formed before the first store (M x N < 2^31): with one register pair reused for each row's
+// address, the compiler let only about two stores be in flight at a time.
+template <class T>
+__device__ __forceinline__ void gemm_store_partial(float* ws, int M, int N, int tile0, int col0, int lane, const f32x4 (&acc)[T::TR][T::TC]) {
+    const int rq = 4 * (lane >> 4);
+    uint32_t off[T::TR][4];
+#pragma unroll
+    for (int i = 0; i < T::TR; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            off[i][r] = static_cast<uint32_t>(((tile0 + i) * 16 + rq + r) * N + col0);
+            pin_value(off[i][r]);
+        }
+#pragma unroll
+    for (int i = 0; i < T::TR; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            if ((tile0 + i) * 16 + rq + r < M) {
+#pragma unroll
+                for (int c = 0; c < T::TC; ++c) ws[off[i][r] + 16 * c] = acc[i][c][r];
+            }
+}
+
+// Results as split rows of the next GEMM's operand ([.][on], from row row_off on): each wave
+// passes its row tiles through its own part of LDS (the ring is no longer read), so that a lane
+// holds eight consecutive columns.  f(i, c, r) is the value of acc[i][c][r]; with PAIRS, of a
+// column pair, given in its even lane, and `oc0` counts pairs.
+template <class T, bool PAIRS, class F>
+__device__ __forceinline__ void gemm_store_split(uint8_t* lds, int wave, int lane, uint16_t* out, int M, int on, int row_off, int tile0, int oc0,
+                                                 F f) {
+    constexpr int W = PAIRS ? 8 * T::TC : 16 * T::TC, S = W + 4;  // columns written; row stride
+    float* buf = reinterpret_cast<float*>(lds) + wave * T::kEpiFloats;
+    const int rq = 4 * (lane >> 4);
+#pragma unroll
+    for (int i = 0; i < T::TR; ++i) {
+#pragma unroll
+        for (int c = 0; c < T::TC; ++c)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float v = f(i, c, r);
+                if constexpr (PAIRS) {
+                    if (!(lane & 1)) buf[(rq + r) * S + 8 * c + (lane & 15) / 2] = v;
+                } else {
+                    buf[(rq + r) * S + 16 * c + (lane & 15)] = v;
+                }
+            }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        for (int q = lane; q < 2 * W; q += 64) {
+            const int r = q & 15, e0 = 8 * (q >> 4), row = (tile0 + i) * 16 + r;
+            float x[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) x[e] = buf[r * S + e0 + e];
+            if (row < M) split_store_piece(out, split_off(row + row_off, oc0 + e0, on), x);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    }
+}
+
+// How one GEMM is cut: a tile shape, its row blocks, and K cut into `splits` ranges of kchunk (a
+// multiple of kGemmK).  `reduce`: the splits are added by a kernel of their own (else by one that
+// runs anyway).
+struct GemmPlan {
+    int tile, mblocks, splits, kchunk;
+};
+GemmPlan gemm_plan(int M, int N, int K, int max_splits, bool bf16, bool reduce);
+// Row tiles of the tile shapes (each 64 columns).  128-column tiles (8 x 8 and 12 x 8) halve
+// the operand reads per product but need more than 256 registers or leave half the CUs idle:
+// slower at every size measured.
+constexpr int kTileRt[] = {1, 2, 4, 8, 12}, kTiles = 5, kGemmBn = 64;
+template <typename WT, class F>
+void gemm_tile(int tile, F f) {  // f(GemmTile<...>{}) for the plan's tile shape
+    switch (tile) {
+        case 0: f(GemmTile<WT, 1, 1, 1>{}); break;
+        case 1: f(GemmTile<WT, 2, 1, 2>{}); break;
+        case 2: f(GemmTile<WT, 4, 1, 4>{}); break;
+        case 3: f(GemmTile<WT, 4, 2, 4>{}); break;
+        default: f(GemmTile<WT, 4, 3, 4>{}); break;
+    }
 }
 
 }  // namespace itts

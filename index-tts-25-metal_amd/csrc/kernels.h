@@ -264,10 +264,10 @@ struct GemmArgs {
     uint32_t kv_cap;
     const uint32_t* row_slot;
     const uint32_t* row_pos;
-    // split-K: at most `splits` K ranges (multiples of 128); launch_gemm picks the tile
+    // split-K: at most `splits` K ranges (1 forbids splitting); launch_gemm picks the tile
     // shape and the split count from an estimate of the time.  The partial tiles go to
     // ws[splits][M][N] and a second kernel adds them in split order.
-    int splits;             // 1: no split
+    int splits;
     float* ws;
     // kGemmResid with ln_out (N = 1280): also ln_out[m] = LayerNorm(c[m]; ln_w, ln_b), the
     // next LayerNorm of the residual stream (kernels.metal:618-669), folded into the split-K
@@ -279,9 +279,6 @@ struct GemmArgs {
 // The workspace holds kGemmWsFloats floats, which bounds splits * M * N.
 constexpr int kGemmMaxSplits = 16;
 constexpr size_t kGemmWsFloats = size_t(8) << 20;
-// The split count launch_gemm would use for this shape (callers pass it in GemmArgs.splits;
-// 1 forbids splitting).
-int gemm_splits(int M, int N, int K);
 hipError_t launch_gemm(const GemmArgs& a, int epi, bool bf16, hipStream_t s);
 
 struct CausalArgs {

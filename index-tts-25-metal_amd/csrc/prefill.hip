@@ -36,16 +36,6 @@ __global__ __launch_bounds__(256) void ln_rows_kernel(LnRowsArgs a) {
     for (int i = 0; i < 5; ++i) split_store(a.y, split_off(row, tid + 256 * i, kWidth), v[0][i]);
 }
 
-// A value held in a register at this point of the program: an empty asm takes it.  The GEMM
-// epilogues form every output (and read every loaded operand) before the first row's store
-// this way; left to the compiler, each row's arithmetic sank into that row's branch, where the
-// use of a load still in flight made it wait for every memory access outstanding, the
-// earlier rows' stores included (one store completion per row).
-template <typename T>
-__device__ __forceinline__ void pin_value(T v) {
-    asm volatile("" ::"v"(v));
-}
-
 // SiLU-gated product of one (gate, up) column pair (kernels.metal:363-374).
 __device__ __forceinline__ float swiglu_f(float g, float u) { return (g / (1.0f + expf(-g))) * u; }
 
@@ -66,14 +56,7 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_kernel(GemmArgs a, int kchu
     __shared__ __align__(16) uint8_t lds[T::kLdsBytes];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    // Workgroup L runs on XCD L % 8 (round-robin dispatch).  The logical index j gives each
-    // XCD one contiguous range, row blocks fastest, then splits, then column tiles, so the
-    // workgroups sharing a column tile's weights mostly share one L2.
-    const int nwg = gridDim.x * gridDim.y * gridDim.z;
-    const int L = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
-    const int per = nwg / 8, rem = nwg % 8, xcd = L % 8;
-    const int j = (xcd < rem ? xcd * (per + 1) : rem * (per + 1) + (xcd - rem) * per) + L / 8;
-    const int by = j % gridDim.y, bz = (j / gridDim.y) % gridDim.z, bx = j / (gridDim.y * gridDim.z);
+    const auto [bx, by, bz] = gemm_place();
     const int kb = SPLIT ? bz * kchunk : 0;
     const int nst = ((SPLIT ? min(a.K, kb + kchunk) : a.K) - kb) / 32;
     uint16_t* ring = reinterpret_cast<uint16_t*>(lds);
@@ -86,76 +69,30 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_kernel(GemmArgs a, int kchu
     constexpr int TR = T::TR, TC = T::TC;
     const int wr = wave / T::WC, wc = wave % T::WC;
     const int tile0 = by * T::RT + wr * TR;
-    uint32_t aoff[TR];
+    uint32_t off[TR];
 #pragma unroll
-    for (int i = 0; i < TR; ++i)
-        aoff[i] = (static_cast<uint32_t>(min(tile0 + i, tiles - 1)) * (a.K / 32) + kb / 32) * (kTileElems * 2) + lane * 16;
+    for (int i = 0; i < TR; ++i) off[i] = (static_cast<uint32_t>(min(tile0 + i, tiles - 1)) * (a.K / 32) + kb / 32) * (kTileElems * 2) + lane * 16;
     f32x4 acc[TR][TC];
-#pragma unroll
-    for (int i = 0; i < TR; ++i)
-#pragma unroll
-        for (int c = 0; c < TC; ++c) acc[i][c] = f32x4{0.f, 0.f, 0.f, 0.f};
-    gemm_compute<T>(ring, ars, aoff, nst, wc, lane, acc);
+    gemm_compute<T>(
+        ring, ars, [&](int i, int s) { return GemmOff{off[i], static_cast<uint32_t>(s) * (kTileElems * 2)}; }, nst, wc, lane, acc);
 
     // acc[i][c][r]: row 16 (tile0 + i) + rq + r, column col0 + 16 c
     const int col0 = bx * T::BN + wc * TC * 16 + (lane & 15);
     const int rq = 4 * (lane >> 4);
     if constexpr (SPLIT) {
-        // Every destination's 32-bit element offset formed before the first store (a split's
-        // plane is M x N < 2^31 elements): with one register pair reused for each row's
-        // address, the compiler let only about two stores be in flight at a time.
-        float* ws = a.ws + static_cast<size_t>(bz) * a.M * a.N;
-        uint32_t off[TR][4];
-#pragma unroll
-        for (int i = 0; i < TR; ++i)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                off[i][r] = static_cast<uint32_t>(((tile0 + i) * 16 + rq + r) * a.N + col0);
-                pin_value(off[i][r]);
-            }
-#pragma unroll
-        for (int i = 0; i < TR; ++i)
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-                if ((tile0 + i) * 16 + rq + r < a.M) {
-#pragma unroll
-                    for (int c = 0; c < TC; ++c) ws[off[i][r] + 16 * c] = acc[i][c][r];
-                }
+        gemm_store_partial<T>(a.ws + static_cast<size_t>(bz) * a.M * a.N, a.M, a.N, tile0, col0, lane, acc);
     } else if constexpr (EPI == kGemmGelu || EPI == kGemmSwiglu) {
-        // Split rows for the next GEMM: each wave passes its row tiles through its own part of
-        // LDS (the ring is no longer read), so that a lane holds eight consecutive columns.
-        constexpr int W = EPI == kGemmGelu ? 16 * TC : 8 * TC, S = W + 4;  // columns written; row stride
-        float* buf = reinterpret_cast<float*>(lds) + wave * T::kEpiFloats;
-        const int oc0 = EPI == kGemmGelu ? bx * T::BN + wc * W : (bx * T::BN) / 2 + wc * W;
-        const int on = EPI == kGemmGelu ? a.N : a.N / 2;
         float bias[TC];
 #pragma unroll
         for (int c = 0; c < TC; ++c) bias[c] = a.bias[col0 + 16 * c];
-#pragma unroll
-        for (int i = 0; i < TR; ++i) {
-#pragma unroll
-            for (int c = 0; c < TC; ++c)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const float v = acc[i][c][r] + bias[c];
-                    if constexpr (EPI == kGemmGelu) {
-                        buf[(rq + r) * S + 16 * c + (lane & 15)] = gelu_f(v);
-                    } else {  // columns col and col ^ 1 sit in lanes l and l ^ 1, on the same rows
-                        const float u = __shfl_xor(v, 1, 64);
-                        if (!(lane & 1)) buf[(rq + r) * S + 8 * c + (lane & 15) / 2] = swiglu_f(v, u);
-                    }
-                }
-            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            for (int f = lane; f < 16 * (W / 8); f += 64) {
-                const int r = f & 15, q = f >> 4, row = (tile0 + i) * 16 + r;
-                float x[8];
-#pragma unroll
-                for (int e = 0; e < 8; ++e) x[e] = buf[r * S + 8 * q + e];
-                if (row < a.M) split_store_piece(a.c_split, split_off(row, oc0 + 8 * q, on), x);
-            }
-            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-            __builtin_amdgcn_wave_barrier();
+        if constexpr (EPI == kGemmGelu) {
+            gemm_store_split<T, false>(lds, wave, lane, a.c_split, a.M, a.N, 0, tile0, bx * T::BN + wc * TC * 16,
+                                       [&](int i, int c, int r) { return gelu_f(acc[i][c][r] + bias[c]); });
+        } else {  // columns col and col ^ 1 sit in lanes l and l ^ 1, on the same rows
+            gemm_store_split<T, true>(lds, wave, lane, a.c_split, a.M, a.N / 2, 0, tile0, (bx * T::BN + wc * TC * 16) / 2, [&](int i, int c, int r) {
+                const float v = acc[i][c][r] + bias[c];
+                return swiglu_f(v, __shfl_xor(v, 1, 64));
+            });
         }
     } else {
         float bias[TC];
@@ -370,15 +307,6 @@ int device_cus() {
     return cus;
 }
 
-// How one GEMM is cut: a tile shape, and K cut into `splits` ranges of kchunk (a multiple of kGemmK).
-struct GemmPlan {
-    int tile, mblocks, splits, kchunk;
-};
-// Row tiles of the tile shapes (each 64 columns).  128-column tiles (8 x 8 and 12 x 8) halve
-// the operand reads per product but need more than 256 registers or leave half the CUs idle:
-// slower at every size measured.
-constexpr int kTileRt[] = {1, 2, 4, 8, 12}, kTiles = 5, kGemmBn = 64;
-
 // The plan with the least estimated time, over every tile shape and split count.  The estimate
 // is a least-squares fit to timings of these kernels on MI355X (every tile shape, 1..16 splits,
 // 8 to 1200 rows of the 1280/5120-wide and the 1024..6144-wide shapes, weights from HBM; the
@@ -407,21 +335,22 @@ constexpr GemmCost kGemmCost[2][kTiles] = {
         {4.30, 0.608, 0.291, 0.170, 1.00, 1.53, 1.0, 0.534},
         {3.79, 0.907, 0.358, 0.296, 1.00, 1.46, 1.0, 0.414},
     }};
-GemmPlan gemm_plan(int M, int N, int K, int max_splits, bool bf16) {
+}  // namespace
+
+GemmPlan gemm_plan(int M, int N, int K, int max_splits, bool bf16, bool reduce) {
     const int rtot = ceil_div(M, 16), cus = device_cus();
     const double mn = static_cast<double>(M) * N;
-    const int smax = std::max(1, std::min<int>(max_splits, static_cast<int>(std::min<double>(kGemmMaxSplits, kGemmWsFloats / mn))));
     GemmPlan best{kTiles - 1, ceil_div(rtot, kTileRt[kTiles - 1]), 1, K};
     double best_t = 1e30;
     for (int i = 0; i < kTiles; ++i) {
         const GemmCost& c = kGemmCost[bf16][i];
         const int mb = ceil_div(rtot, kTileRt[i]);
-        for (int s = 1; s <= smax; ++s) {
+        for (int s = 1; s <= max_splits; ++s) {
             const int kc = ceil_div(ceil_div(K, s), kGemmK) * kGemmK;
             if (ceil_div(K, kc) != s) continue;
             const double r = static_cast<double>(N / kGemmBn) * mb * s / cus, rounds = std::ceil(r);
             double t = c.launch + rounds * c.tile + kc / 32.0 * (std::pow(rounds, c.grow) * c.step + c.crowd * std::max(0.0, r - c.free));
-            if (s > 1) t += c.reduce + c.per_split * s * mn / 1e6;
+            if (s > 1) t += (reduce ? c.reduce : 0.0) + c.per_split * s * mn / 1e6;
             if (t < best_t) {
                 best_t = t;
                 best = GemmPlan{i, mb, s, kc};
@@ -431,21 +360,15 @@ GemmPlan gemm_plan(int M, int N, int K, int max_splits, bool bf16) {
     return best;
 }
 
+namespace {
+
 template <typename WT, int EPI, bool SPLIT>
 void launch_gemm_tile(const GemmArgs& a, const GemmPlan& p, hipStream_t s) {
-    const dim3 grid(a.N / kGemmBn, p.mblocks, p.splits), block(kGemmThreads);
-    switch (p.tile) {
-        case 0: hipLaunchKernelGGL((gemm_kernel<GemmTile<WT, 1, 1, 1>, EPI, SPLIT>), grid, block, 0, s, a, p.kchunk); break;
-        case 1: hipLaunchKernelGGL((gemm_kernel<GemmTile<WT, 2, 1, 2>, EPI, SPLIT>), grid, block, 0, s, a, p.kchunk); break;
-        case 2: hipLaunchKernelGGL((gemm_kernel<GemmTile<WT, 4, 1, 4>, EPI, SPLIT>), grid, block, 0, s, a, p.kchunk); break;
-        case 3: hipLaunchKernelGGL((gemm_kernel<GemmTile<WT, 4, 2, 4>, EPI, SPLIT>), grid, block, 0, s, a, p.kchunk); break;
-        default: hipLaunchKernelGGL((gemm_kernel<GemmTile<WT, 4, 3, 4>, EPI, SPLIT>), grid, block, 0, s, a, p.kchunk); break;
-    }
+    const dim3 grid(a.N / kGemmBn, p.mblocks, p.splits);
+    gemm_tile<WT>(p.tile, [&](auto t) { hipLaunchKernelGGL((gemm_kernel<decltype(t), EPI, SPLIT>), grid, dim3(kGemmThreads), 0, s, a, p.kchunk); });
 }
 
 }  // namespace
-
-int gemm_splits(int M, int N, int K) { return gemm_plan(M, N, K, kGemmMaxSplits, false).splits; }
 
 static hipError_t launch_gemm_plan(GemmArgs a, int epi, bool bf16, const GemmPlan& p, hipStream_t s) {
     a.splits = p.splits;
@@ -484,7 +407,8 @@ hipError_t launch_gemm(const GemmArgs& a, int epi, bool bf16, hipStream_t s) {
     if ((epi == kGemmStore || epi == kGemmSwiglu) && bf16) return hipErrorInvalidValue;  // FP32 weights only (the Qwen decoder)
     if (a.ln_out && (epi != kGemmResid || a.N != kWidth)) return hipErrorInvalidValue;
     if (split_elems(a.M, a.K) * 2 >= 0x80000000u) return hipErrorInvalidValue;  // 32-bit operand offsets
-    return launch_gemm_plan(a, epi, bf16, gemm_plan(a.M, a.N, a.K, a.splits, bf16), s);
+    const int fit = static_cast<int>(std::min<size_t>(kGemmMaxSplits, kGemmWsFloats / (static_cast<size_t>(a.M) * a.N)));
+    return launch_gemm_plan(a, epi, bf16, gemm_plan(a.M, a.N, a.K, std::max(1, std::min(a.splits, fit)), bf16, true), s);
 }
 
 hipError_t launch_causal_attention(const CausalArgs& a, hipStream_t s) {

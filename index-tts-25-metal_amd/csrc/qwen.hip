@@ -814,7 +814,7 @@ struct Engine {
         g.K = Kk;
         g.c = C;
         g.c_split = Csplit;
-        g.splits = gemm_splits(M, Nn, Kk);
+        g.splits = kGemmMaxSplits;
         g.ws = ws.p;
         QWEN_CHECK(launch_gemm(g, epi, false, stream));
     }

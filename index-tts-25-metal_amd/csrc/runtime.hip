@@ -783,7 +783,7 @@ struct Engine {
             g.M = static_cast<int>(M);
             g.N = kQkv;
             g.K = kWidth;
-            g.splits = gemm_splits(static_cast<int>(M), kQkv, kWidth);
+            g.splits = kGemmMaxSplits;
             g.ws = b.ws;
             g.c = pq_;
             g.kv = kv.p;
@@ -813,7 +813,7 @@ struct Engine {
             p.M = static_cast<int>(M);
             p.N = kWidth;
             p.K = kWidth;
-            p.splits = gemm_splits(static_cast<int>(M), kWidth, kWidth);
+            p.splits = kGemmMaxSplits;
             p.ws = b.ws;
             p.c = px_;
             p.ln_w = par + kParLn2W;  // ln_2 of the new residual rows
@@ -827,7 +827,7 @@ struct Engine {
             f.M = static_cast<int>(M);
             f.N = kFfn;
             f.K = kWidth;
-            f.splits = gemm_splits(static_cast<int>(M), kFfn, kWidth);
+            f.splits = kGemmMaxSplits;
             f.ws = b.ws;
             f.c_split = pff_;
             HIP_CHECK(launch_gemm(f, kGemmGelu, bf16, stream));
@@ -838,7 +838,7 @@ struct Engine {
             f2.M = static_cast<int>(M);
             f2.N = kWidth;
             f2.K = kFfn;
-            f2.splits = gemm_splits(static_cast<int>(M), kWidth, kFfn);
+            f2.splits = kGemmMaxSplits;
             f2.ws = b.ws;
             f2.c = px_;
             if (l + 1 < layers) {  // ln_1 of the next layer
