@@ -36,7 +36,7 @@ DEVICE_FLAGS = [
     f"-I{INCLUDE}",
     f"-I{CSRC}",
 ]
-SOURCES = ["decode.hip", "step.hip", "step_batch.hip", "sampler.hip", "beam.hip", "prefill.hip", "util.hip", "runtime.hip",
+SOURCES = ["decode.hip", "step.hip", "step_bf16.hip", "step_batch.hip", "sampler.hip", "beam.hip", "prefill.hip", "util.hip", "runtime.hip",
            "codec.hip", "libm_check.hip", "qwen.hip"]
 # Per-file device flags.  step.hip: the persistent step kernel is scheduled with LLVM's max-ILP
 # strategy, 578.4 -> 567.9 us per step at 752 cached rows (one box, three alternating runs); the
@@ -45,7 +45,7 @@ SOURCES = ["decode.hip", "step.hip", "step_batch.hip", "sampler.hip", "beam.hip"
 # (one box, alternating).  Measured and not applied: max-ILP for prefill.hip (155-row prefill
 # 3.23 -> 3.29 ms) and qwen.hip (step 835 -> 846 us), no change for sampler.hip and beam.hip.
 _MAX_ILP = ["-mllvm", "--amdgpu-sched-strategy=max-ilp"]
-SOURCE_FLAGS = {"step.hip": _MAX_ILP, "codec.hip": _MAX_ILP}
+SOURCE_FLAGS = {"step.hip": _MAX_ILP, "step_bf16.hip": _MAX_ILP, "codec.hip": _MAX_ILP}
 HOST_SOURCES = ["bundle.cpp"]  # host-only C++ (g++)
 HOST_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-Wall", f"-I{INCLUDE}", f"-I{CSRC}"]
 

@@ -181,6 +181,8 @@ constexpr int kStepStampsPerLayer = 8;
 bool step_fits(int grid);
 hipError_t step_occupancy(bool bf16, int* blocks_per_cu);
 hipError_t launch_step(const StepArgs& a, int grid, bool bf16, hipStream_t s);
+hipError_t step_occupancy_bf16(int* blocks_per_cu);  // (step_bf16.hip)
+hipError_t launch_step_bf16(const StepArgs& a, int grid, hipStream_t s);
 // Persistent step for 2..kStepBatchMax sequences (FP32 weights, no beam row-owner table).
 constexpr int kStepBatchMax = 4;
 bool step_batch_fits(int grid, int nseq);

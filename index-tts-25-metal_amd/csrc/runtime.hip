@@ -119,9 +119,21 @@ void unregister_step_user(int dev) {
     --g_step_users[dev];
 }
 
-hipError_t launch_step_serialized(const StepArgs& a, int nseq, int grid, bool bf16, int dev, hipStream_t s) {
+// One persistent step that is waited for before the lock is released (a BF16 decoder's step()).
+// Such decoders are not counted as users: with the lock held no other decoder can launch a
+// grid, and those launched before are drained first, so the other decoders keep launching
+// unchained.
+template <class F>
+void exclusive_step(int dev, F run) {
     std::lock_guard<std::mutex> lock(g_step_mu);
-    if (g_step_users[dev] <= 1) return nseq == 1 ? launch_step(a, grid, bf16, s) : launch_step_batch(a, nseq, grid, s);
+    auto it = g_step_users.find(dev);
+    if (it != g_step_users.end() && it->second > 0) HIP_CHECK(hipDeviceSynchronize());
+    run();
+}
+
+hipError_t launch_step_serialized(const StepArgs& a, int nseq, int grid, int dev, hipStream_t s) {
+    std::lock_guard<std::mutex> lock(g_step_mu);
+    if (g_step_users[dev] <= 1) return nseq == 1 ? launch_step(a, grid, false, s) : launch_step_batch(a, nseq, grid, s);
     auto& last = g_step_last;
     auto it = last.find(dev);
     if (it == last.end()) {
@@ -133,7 +145,7 @@ hipError_t launch_step_serialized(const StepArgs& a, int nseq, int grid, bool bf
         const hipError_t err = hipStreamWaitEvent(s, it->second, 0);
         if (err != hipSuccess) return err;
     }
-    const hipError_t err = nseq == 1 ? launch_step(a, grid, bf16, s) : launch_step_batch(a, nseq, grid, s);
+    const hipError_t err = nseq == 1 ? launch_step(a, grid, false, s) : launch_step_batch(a, nseq, grid, s);
     if (err != hipSuccess) return err;
     return hipEventRecord(it->second, s);
 }
@@ -289,7 +301,7 @@ struct Engine {
         // later steps in flight copies into the pinned ring), and no persistent grid of this
         // decoder may outlive its registration: drain the stream before anything is freed.
         if (stream) (void)hipStreamSynchronize(stream);
-        if (step_ok) unregister_step_user(step_dev);
+        if (step_ok && !bf16) unregister_step_user(step_dev);
         for (auto& kvp : graphs) (void)hipGraphExecDestroy(kvp.second);
         for (auto& e : ev)
             if (e) (void)hipEventDestroy(e);
@@ -469,24 +481,24 @@ struct Engine {
 
     // The persistent step runs when one 512-thread workgroup fits per CU (the grid is one
     // workgroup per CU, all resident together), there is a workgroup per attention head
-    // (step_fits: head h's merge runs on workgroup h), weights are FP32 and the cache holds
-    // at most 4096 rows (at most 32 splits, kAttnMaxChunk rows each).
+    // (step_fits: head h's merge runs on workgroup h) and the cache holds at most 4096 rows
+    // (at most 32 splits, kAttnMaxChunk rows each).
     void init_step() {
         const char* pe = std::getenv("ITTS_GPT_PERSISTENT");
-        if ((pe && std::strcmp(pe, "0") == 0) || bf16 || cap > 4096) return;
+        if ((pe && std::strcmp(pe, "0") == 0) || cap > 4096) return;
         int dev = 0, cus = 0, occ = 0;
         HIP_CHECK(hipGetDevice(&dev));
         step_dev = dev;
         HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-        HIP_CHECK(step_occupancy(false, &occ));
+        HIP_CHECK(step_occupancy(bf16, &occ));
         if (occ < 1 || !step_fits(cus)) return;
-        // Batches and beams of 2..4 sequences in one launch (step_batch.hip) only when
+        // Batches and beams of 2..4 sequences of FP32 weights in one launch (step_batch.hip) only when
         // ITTS_GPT_PERSISTENT_BATCH=1: the multi-kernel path's batched GEMVs (five-wave
         // workgroups, LayerNorms formed in the GEMV) measure as fast at 2 sequences and faster
         // from 3 on (3: 932 against 1015 us per step, 4: 1036 against 1207; beam-3 3070
         // against 2824 beam tokens/s), with bitwise the same logits.
         const char* pb = std::getenv("ITTS_GPT_PERSISTENT_BATCH");
-        const bool batch = max_batch >= 2 && pb && std::strcmp(pb, "1") == 0;
+        const bool batch = !bf16 && max_batch >= 2 && pb && std::strcmp(pb, "1") == 0;
         for (int nb = 2; batch && nb <= kStepBatchMax; ++nb) {
             int bocc = 0;
             HIP_CHECK(step_batch_occupancy(nb, &bocc));
@@ -501,7 +513,7 @@ struct Engine {
         const char* fs = std::getenv("ITTS_GPT_FUSED_SAMPLER");
         fused_sampling = fs && std::strcmp(fs, "1") == 0;
         step_grid = cus;
-        register_step_user(dev);
+        if (!bf16) register_step_user(dev);
         step_ok = true;
     }
 
@@ -555,8 +567,11 @@ struct Engine {
     // 2..kStepBatchMax in one launch (step_batch.hip; with the beam row-owner table when every
     // slot it may name is below kStepBatchMax).  Other batches take the multi-kernel path,
     // whose batched GEMVs read the weights once for all of them.
-    bool persistent(int nseq, bool use_table) const {
+    // With BF16 weights it takes the single steps whose logits go to the host (step(): 690 -> 600
+    // us a call at 250 cached rows); generate()'s documented path there is the multi-kernel graph.
+    bool persistent(int nseq, bool use_table, bool sampler = true) const {
         if (!step_ok || nseq < 1 || nseq > kStepBatchMax) return false;
+        if (bf16 && sampler) return false;
         if (use_table) return nseq >= 2 && step_batch_ok[nseq] && beam_slots <= static_cast<uint32_t>(kStepBatchMax);
         return nseq == 1 || step_batch_ok[nseq];
     }
@@ -568,7 +583,8 @@ struct Engine {
             s.tail = step_tail.p;
             s.sample = sample_base(kModeDecode);
         }
-        HIP_CHECK(launch_step_serialized(s, nseq, step_grid, bf16, step_dev, stream));
+        if (bf16) HIP_CHECK(launch_step(s, step_grid, true, stream));  // inside exclusive_step
+        else HIP_CHECK(launch_step_serialized(s, nseq, step_grid, step_dev, stream));
     }
 
     // ---------------------------------------------------------------- forward pieces
@@ -687,7 +703,7 @@ struct Engine {
 
     // Runs one step (forward [+ sampler]) as a replay of its captured graph, or eagerly.
     void run_step(int nseq, int nb, bool sampler, bool use_table) {
-        if (persistent(nseq, use_table)) {
+        if (persistent(nseq, use_table, sampler)) {
             timing.decode_path = ITTS_PATH_STEP;
             const bool fuse = sampler && nseq == 1 && fused_sampling;
             launch_persistent(nseq, use_table, fuse);
@@ -904,9 +920,13 @@ struct Engine {
         s.position = position;
         pinned_state[0] = s;
         upload_states(1);
-        run_step(1, 1, false, false);
-        HIP_CHECK(hipMemcpyAsync(out_logits, logits.p, kMelVocab * 4, hipMemcpyDeviceToHost, stream));
-        HIP_CHECK(hipStreamSynchronize(stream));
+        auto run = [&] {
+            run_step(1, 1, false, false);
+            HIP_CHECK(hipMemcpyAsync(out_logits, logits.p, kMelVocab * 4, hipMemcpyDeviceToHost, stream));
+            HIP_CHECK(hipStreamSynchronize(stream));
+        };
+        if (bf16 && persistent(1, false, false)) exclusive_step(step_dev, run);
+        else run();
         check_step_error();
         cached++;
     }
@@ -1301,7 +1321,7 @@ struct Engine {
             HIP_CHECK(hipMemsetAsync(stamps.p, 0, stamps.n * 8, stream));
             StepArgs a = step_args(0, nseq);
             a.stamps = stamps.p;
-            HIP_CHECK(launch_step_serialized(a, nseq, step_grid, bf16, step_dev, stream));
+            HIP_CHECK(launch_step_serialized(a, nseq, step_grid, step_dev, stream));
             HIP_CHECK(hipMemcpyAsync(host.data(), stamps.p, stamps.n * 8, hipMemcpyDeviceToHost, stream));
             HIP_CHECK(hipStreamSynchronize(stream));
             check_step_error();

@@ -55,7 +55,20 @@ namespace itts {
 namespace {
 using namespace stepc;
 
+// This file is compiled twice: for FP32 weights and, through step_bf16.hip, for BF16 weights.  (Two
+// kernels in one file changed the FP32 kernel's inlining and its step by 3 us.)
+#ifdef ITTS_STEP_BF16
+using StepWeight = uint16_t;
+#else
+using StepWeight = float;
+#endif
+
 constexpr int kRing = 24;          // chunks in the LDS ring
+// BF16 weights: a chunk is half the bytes, so twice the slots keep as many in flight, and the
+// producers end their phases closer together.  Step at 60 / 1010 cached rows, call to logits on
+// the host: 2 slots 625 / 682 us, 3 600 / 648, 4 589 / 643, 6 613 / 680; with 4 slots, first poll
+// after 4 * 64 clocks 623 / 668, 8 608 / 657, 14 597 / 647, 20 592 / 642, 24 588 / 637.
+constexpr int kSlotsBf16 = 4, kPollDelayBf16 = 24;
 
 // This workgroup's share of the step, identical in every wave.
 struct Plan {
@@ -127,15 +140,18 @@ struct Smem {
 // Source of the 5 lines of chunk r of layer l of this workgroup's stream (l == layers:
 // chunk r of its mel_head rows): a wave-uniform base, the chunk's extent in bytes from it,
 // and the lane's byte offset of each line.  Line k of a chunk lands at ring line k, lane i's
-// 16 bytes at +16 i.
-__device__ __forceinline__ void chunk_src(const StepArgs& a, const Plan& P, const float* W, int l, int r, int lane,
+// 16 bytes at +16 i.  WT: the weights' type (BF16: a line is 512 bytes, 8 per lane; the 16-byte
+// loads of run_loader overlap, their upper halves unused).  Returns whether the chunk holds
+// weights (not cached rows).
+template <typename WT>
+__device__ __forceinline__ bool chunk_src(const StepArgs& a, const Plan& P, const WT* W, int l, int r, int lane,
                                           const float*& base, uint32_t& extent, uint32_t (&off)[kLines]) {
     if (l >= a.layers) {
-        base = W + a.off_head + static_cast<size_t>(P.h0 + r) * kWidth;
+        base = reinterpret_cast<const float*>(W + a.off_head + static_cast<size_t>(P.h0 + r) * kWidth);
     } else {
-        const float* wl = W + static_cast<size_t>(l) * a.layer_stride;
+        const WT* wl = W + static_cast<size_t>(l) * a.layer_stride;
         if (r < P.o_att) {
-            base = wl + static_cast<size_t>(P.q0 + r) * kWidth;
+            base = reinterpret_cast<const float*>(wl + static_cast<size_t>(P.q0 + r) * kWidth);
         } else if (r < P.o_proj) {
             // attention tile chunks: K chunks 0..kc-1 then V chunks, 20 cached rows each,
             // lane l covers row 4 k + l / 16 of line k, 16 bytes (l % 16) of it
@@ -158,29 +174,32 @@ __device__ __forceinline__ void chunk_src(const StepArgs& a, const Plan& P, cons
                 if (row >= R) row = 0;                                 // clamped: loaded, never read
                 off[k] = static_cast<uint32_t>((row * kHeadDim + (lane & 15) * 4) * 4);
             }
-            return;
+            return false;
         } else if (r < P.o_fc) {
-            base = wl + static_cast<size_t>(kQkv) * kWidth + static_cast<size_t>(P.p0 + r - P.o_proj) * kWidth;
+            base = reinterpret_cast<const float*>(wl + static_cast<size_t>(kQkv) * kWidth + static_cast<size_t>(P.p0 + r - P.o_proj) * kWidth);
         } else if (r < P.o_fc2) {
-            base = wl + static_cast<size_t>(kQkv + kWidth) * kWidth + static_cast<size_t>(P.f0 + r - P.o_fc) * kWidth;
+            base = reinterpret_cast<const float*>(wl + static_cast<size_t>(kQkv + kWidth) * kWidth + static_cast<size_t>(P.f0 + r - P.o_fc) * kWidth);
         } else {
             const int q = r - P.o_fc2;  // mlp.c_proj rows are 5120 wide: 4 chunks each
-            base = wl + static_cast<size_t>(kQkv + kWidth + kFfn) * kWidth + static_cast<size_t>(P.g0 + (q >> 2)) * kFfn +
-                   (q & 3) * kChunkF;
+            base = reinterpret_cast<const float*>(wl + static_cast<size_t>(kQkv + kWidth + kFfn) * kWidth + static_cast<size_t>(P.g0 + (q >> 2)) * kFfn +
+                   (q & 3) * kChunkF);
         }
     }
-    extent = kChunkF * 4;
+    extent = kChunkF * static_cast<int>(sizeof(WT));
 #pragma unroll
-    for (int k = 0; k < kLines; ++k) off[k] = static_cast<uint32_t>((k * 256 + lane * 4) * 4);
+    for (int k = 0; k < kLines; ++k) off[k] = static_cast<uint32_t>((k * 256 + lane * 4) * static_cast<int>(sizeof(WT)));
+    return true;
 }
 
 // The batch-1 stream: chunk_src over this workgroup's Plan.
+template <typename WT>
 __device__ __forceinline__ void run_loader(const StepArgs& a, const Plan& P, float* ring, Ctl& ctl, int lw, int lane) {
-    const float* __restrict__ W = static_cast<const float*>(a.w);
-    stepc::run_loader<kRing>(a, P.layer_chunks, P.hn, ring, ctl, lw, lane,
-                             [&](int l, int r, const float*& base, uint32_t& extent, uint32_t(&off)[kLines]) {
-                                 chunk_src(a, P, W, l, r, lane, base, extent, off);
-                             });
+    const WT* __restrict__ W = static_cast<const WT*>(a.w);
+    constexpr bool kBf16 = sizeof(WT) == 2;
+    stepc::run_loader<kRing, kBf16, kBf16 ? kSlotsBf16 : kSlots>(a, P.layer_chunks, P.hn, ring, ctl, lw, lane,
+                                                               [&](int l, int r, const float*& base, uint32_t& extent, uint32_t(&off)[kLines]) {
+                                                                   return chunk_src<WT>(a, P, W, l, r, lane, base, extent, off);
+                                                               });
 }
 
 // ------------------------------------------------------------------ compute waves
@@ -425,6 +444,8 @@ __device__ inline void sampling_tail(const StepArgs& a, Ctl& ctl, StepTailLds& l
 }
 
 __global__ __launch_bounds__(kST) void step_kernel(StepArgs a) {
+    using WT = StepWeight;
+    constexpr int kDelay = sizeof(WT) == 2 ? kPollDelayBf16 : kPollDelay;
     __shared__ StepTailLds lds;
     __shared__ Ctl ctl;
     float* ring = lds.step.ring;
@@ -450,7 +471,7 @@ __global__ __launch_bounds__(kST) void step_kernel(StepArgs a) {
     // start back by 6-10 us).
     if (wave >= kCW) {
         wait_go(ctl, a.err);
-        run_loader(a, P, ring, ctl, __builtin_amdgcn_readfirstlane(wave - kCW), lane);
+        run_loader<WT>(a, P, ring, ctl, __builtin_amdgcn_readfirstlane(wave - kCW), lane);
         sampling_tail(a, ctl, lds, a.epoch + 8u * static_cast<uint32_t>(a.layers) + kEpLogit);
         return;
     }
@@ -498,7 +519,7 @@ __global__ __launch_bounds__(kST) void step_kernel(StepArgs a) {
                 use[i] = l > 0;
             }
             XRead<5> xr;
-            if (l > 0) poll_delay();
+            if (l > 0) poll_delay<kDelay>();
             xr.issue(XB, idx, use, ep(l, kEpXh));
             LnParDot ln;
             ln.load(par + kParLn1W, par + kParLn1B, lane);
@@ -781,7 +802,7 @@ __global__ __launch_bounds__(kST) void step_kernel(StepArgs a) {
                 use[i] = true;
             }
             XRead<5> xr;
-            poll_delay();
+            poll_delay<kDelay>();
             xr.issue(XB, idx, use, ep(l, kEpAttn));
             LaneBias<kGProj, false> bias;
             bias.load(par + kParProjB + P.p0, P.pn, wave, lane);
@@ -817,7 +838,7 @@ __global__ __launch_bounds__(kST) void step_kernel(StepArgs a) {
                 use[i] = true;
             }
             XRead<5> xr;
-            poll_delay();
+            poll_delay<kDelay>();
             xr.issue(XB, idx, use, ep(l, kEpHmid));
             LnParDot ln;
             ln.load(par + kParLn2W, par + kParLn2B, lane);
@@ -859,7 +880,7 @@ __global__ __launch_bounds__(kST) void step_kernel(StepArgs a) {
                 use[i] = true;
             }
             XRead<NF> xr;
-            poll_delay();
+            poll_delay<kDelay>();
             xr.issue(XB, idx, use, ep(l, kEpFf));
             LaneBias<kGFc2, true> bias;
             bias.load(par + kParFc2B + P.g0, P.gn, wave, lane);
@@ -897,7 +918,7 @@ __global__ __launch_bounds__(kST) void step_kernel(StepArgs a) {
             use[i] = true;
         }
         XRead<5> xr;
-        poll_delay();
+        poll_delay<kDelay>();
         xr.issue(XB, idx, use, ep(a.layers, kEpXh));
         LnPar lf;
         lf.load(a.head + kHeadLnfW, a.head + kHeadLnfB, tid);
@@ -940,19 +961,24 @@ __global__ __launch_bounds__(kST) void step_kernel(StepArgs a) {
 
 }  // namespace
 
-bool step_fits(int grid) { return grid >= kHeads; }
-
-// FP32 weights only (the loaders copy 16-byte FP32 lines); BF16 decoders keep the
-// multi-kernel path.
-hipError_t step_occupancy(bool bf16, int* blocks_per_cu) {
-    if (bf16) return hipErrorInvalidValue;
-    return hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks_per_cu, step_kernel, kST, 0);
-}
-
-hipError_t launch_step(const StepArgs& a, int grid, bool bf16, hipStream_t s) {
-    if (bf16) return hipErrorInvalidValue;
+#ifdef ITTS_STEP_BF16
+hipError_t step_occupancy_bf16(int* blocks_per_cu) { return hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks_per_cu, step_kernel, kST, 0); }
+hipError_t launch_step_bf16(const StepArgs& a, int grid, hipStream_t s) {
     hipLaunchKernelGGL(step_kernel, dim3(grid), dim3(kST), 0, s, a);
     return hipGetLastError();
 }
+#else
+bool step_fits(int grid) { return grid >= kHeads; }
+
+hipError_t step_occupancy(bool bf16, int* blocks_per_cu) {
+    return bf16 ? step_occupancy_bf16(blocks_per_cu) : hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks_per_cu, step_kernel, kST, 0);
+}
+
+hipError_t launch_step(const StepArgs& a, int grid, bool bf16, hipStream_t s) {
+    if (bf16) return launch_step_bf16(a, grid, s);
+    hipLaunchKernelGGL(step_kernel, dim3(grid), dim3(kST), 0, s, a);
+    return hipGetLastError();
+}
+#endif
 
 }  // namespace itts

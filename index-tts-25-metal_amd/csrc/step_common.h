@@ -108,7 +108,10 @@ __device__ __forceinline__ void xread(const uint64_t* base, const int (&idx)[N],
     r.wait(base, idx, e, out, err, failed);
 }
 
-__device__ __forceinline__ void poll_delay() { __builtin_amdgcn_s_sleep(kPollDelay); }
+template <int D = kPollDelay>
+__device__ __forceinline__ void poll_delay() {
+    __builtin_amdgcn_s_sleep(D);
+}
 
 // A wave-uniform value through an empty asm: conditions derived from it are formed where
 // they are used instead of being hoisted out of the layer loop into spilled registers.
@@ -301,7 +304,10 @@ __device__ __forceinline__ void ln_to_xrow(const float* row, int lane, float mea
 // the younger kSlots - 1 chunks in flight.
 // RING: chunks in the ring; src(l, r, base, extent, off) gives chunk r of layer l (l == layers:
 // chunk r of the head rows) as chunk_src does; layer_chunks and head_chunks size the stream.
-template <int RING, class Src>
+// BF16: src says whether the chunk is one of BF16 weights (half the bytes, lane offsets of 8
+// bytes); its lanes' four values are widened on the way into the ring, which stays FP32, so the
+// compute waves are the same.  SLOTS: chunks staged in registers per loader wave.
+template <int RING, bool BF16 = false, int SLOTS = kSlots, class Src>
 __device__ __forceinline__ void run_loader(const StepArgs& a, int layer_chunks, int head_chunks, float* ring, Ctl& ctl, int lw, int lane,
                                            Src src) {
     const float* __restrict__ W = static_cast<const float*>(a.w);
@@ -317,12 +323,14 @@ __device__ __forceinline__ void run_loader(const StepArgs& a, int layer_chunks, 
     };
     norm();
     typedef float v4f __attribute__((ext_vector_type(4)));  // plain vector type: the slots stay in registers
-    v4f slot[kSlots][kLines];
-    auto load = [&](v4f(&d)[kLines], int j) {
+    v4f slot[SLOTS][kLines];
+    bool half[SLOTS] = {};  // the slot holds BF16 weights
+    auto load = [&](v4f(&d)[kLines], bool& hw, int j) {
         const float* base = W;
         uint32_t extent = kChunkF * 4, off[kLines];
         if (j < owned) {
-            src(cl, cr, base, extent, off);
+            if constexpr (BF16) hw = src(cl, cr, base, extent, off);
+            else src(cl, cr, base, extent, off);
             cr += kLW;
             norm();
         } else {
@@ -341,11 +349,11 @@ __device__ __forceinline__ void run_loader(const StepArgs& a, int layer_chunks, 
         for (int k = 0; k < kLines; ++k) d[k] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(rs, static_cast<int>(off[k]), 0, kCachePolicyNt));
     };
 #pragma unroll
-    for (int s = 0; s < kSlots; ++s) load(slot[s], s);
+    for (int s = 0; s < SLOTS; ++s) load(slot[s], half[s], s);
     uint32_t lim = RING;  // chunks below lim may be written: min(need) + RING
-    for (int j0 = 0; j0 < owned; j0 += kSlots) {
+    for (int j0 = 0; j0 < owned; j0 += SLOTS) {
 #pragma unroll
-        for (int s = 0; s < kSlots; ++s) {
+        for (int s = 0; s < SLOTS; ++s) {
             const int j = j0 + s;
             if (j < owned) {
                 const uint32_t c = static_cast<uint32_t>(lw + kLW * j);
@@ -365,10 +373,17 @@ __device__ __forceinline__ void run_loader(const StepArgs& a, int layer_chunks, 
                 }
                 float* dst = ring + (c % RING) * kChunkF + lane * 4;
 #pragma unroll
-                for (int k = 0; k < kLines; ++k) *reinterpret_cast<v4f*>(dst + k * 256) = slot[s][k];
+                for (int k = 0; k < kLines; ++k) {
+                    v4f v = slot[s][k];
+                    if (BF16 && half[s]) {
+                        const uint32_t x = __float_as_uint(v.x), y = __float_as_uint(v.y);
+                        v = v4f{__uint_as_float(x << 16), __uint_as_float(x & 0xffff0000u), __uint_as_float(y << 16), __uint_as_float(y & 0xffff0000u)};
+                    }
+                    *reinterpret_cast<v4f*>(dst + k * 256) = v;
+                }
                 if (lane == 0) lds_st(&ctl.done[lw], c + 1);
             }
-            load(slot[s], j + kSlots);
+            load(slot[s], half[s], j + SLOTS);
         }
     }
 }

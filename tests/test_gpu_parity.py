@@ -4,6 +4,8 @@ Tolerances (north star): teacher-forced logits max-abs <= 1e-3 and relative (L2)
 greedy codes exact; processors (mask and values) and sampled tokens bit-exact given the
 same logits and RNG state.
 """
+import os
+
 import numpy as np
 import pytest
 
@@ -577,6 +579,32 @@ def test_persistent_step_bitwise_equals_multikernel(both_paths, itts, n_text):
         b = multi.step(code, i + 2)
         assert multi.last_timing()["decode_path"] == "multi"
         assert np.array_equal(a, b), f"step {i}: max diff {np.max(np.abs(a - b))}"
+
+
+@pytest.mark.parametrize("rows", [1, 19, 20, 63, 64, 65, 767, 769, 1023])
+def test_persistent_bf16_step_bitwise_equals_multikernel(itts, small_weights, rows):
+    """With BF16 weights the persistent step's loaders widen the weights on their way into the
+    ring: the logits are those of the multi-kernel path bit for bit, at cached row counts either
+    side of the attention tiles' edges (20-row chunks, 64-row splits, 12 splits, wider tiles)."""
+    decs = {}
+    old = os.environ.get("ITTS_GPT_PERSISTENT")
+    try:
+        for v, path in (("0", "multi"), ("1", "step")):
+            os.environ["ITTS_GPT_PERSISTENT"] = v
+            decs[path] = itts.GptDecoder(small_weights, kv_capacity=1100, weight_dtype="bf16")
+    finally:
+        if old is None:
+            del os.environ["ITTS_GPT_PERSISTENT"]
+        else:
+            os.environ["ITTS_GPT_PERSISTENT"] = old
+    prefix = (0.5 * np.random.default_rng(rows).standard_normal((rows, 1280))).astype(np.float32)
+    got = {}
+    for path, d in decs.items():
+        got[path] = [d.prefill(prefix)] + [d.step(c, i + 2) for i, c in enumerate((17, 4000, 8191))]
+        assert d.last_timing()["decode_path"] == path
+        d.close()
+    for a, b in zip(got["multi"], got["step"]):
+        assert same_bits(a, b)
 
 
 def test_persistent_step_past_2048_rows_bitwise_equals_multikernel(itts, small_weights):
