@@ -187,6 +187,27 @@ __global__ __launch_bounds__(kGemmThreads) void codec_gemm_kernel(CodecGemm g) {
     }
 }
 
+// The same for up to 16 RT rows of an operand that is not a convolution's (gemm_core.h, gemm_small).
+template <int RT, int EPI>
+__global__ __launch_bounds__(64 * kSmallWaves) void codec_gemm_small_kernel(CodecGemm g) {
+    __shared__ GemmSmallLds<RT> lds;
+    const int kb = blockIdx.y * g.kchunk, nst = (min(g.K, kb + g.kchunk) - kb) / 32;
+    float sum[2];
+    gemm_small<float, RT>(lds, g.w + static_cast<size_t>(blockIdx.x) * 16 * g.K + kb, g.K, nst,
+                          gemm_rsrc(g.a, static_cast<uint32_t>(split_elems(g.M, g.K) * 2)), kb / 32 * (kTileElems * 2),
+                          g.K / 32 * (kTileElems * 2), (g.M + 15) / 16, sum);
+    const int col = blockIdx.x * 16 + (threadIdx.x & 15);
+    const float bias = EPI == kEpiPartial ? 0.0f : g.bias[col];
+#pragma unroll
+    for (int q = 0; q < (RT > 2 ? 2 : 1); ++q) {
+        const int row = (threadIdx.x >> 4) + 32 * q;
+        if (row >= g.M) continue;
+        if constexpr (EPI == kEpiPartial) g.ws[(static_cast<size_t>(blockIdx.y) * g.M + row) * g.N + col] = sum[q];
+        else if constexpr (EPI == kEpiGelu) split_store(g.cs, split_off(row, col, g.N), codec_gelu(sum[q] + bias));
+        else split_store(g.cs, split_off(row + 1, col, g.N), sum[q] + bias);
+    }
+}
+
 // The up conv's splits, added in split order, + bias; a thread takes four columns.
 template <int SM>
 __global__ __launch_bounds__(256) void codec_up_reduce_kernel(CodecGemm g, int splits) {
@@ -210,18 +231,14 @@ __device__ __forceinline__ void ln384(float (&v)[6], const float* gw, const floa
     float s = 0.0f;
 #pragma unroll
     for (int i = 0; i < 6; ++i) s += v[i];
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) s += __shfl_xor(s, o, 64);
-    const float mean = s / float(kCH);
+    const float mean = wave_sum(s) / float(kCH);
     float q = 0.0f;
 #pragma unroll
     for (int i = 0; i < 6; ++i) {
         const float d = v[i] - mean;
         q += d * d;
     }
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) q += __shfl_xor(q, o, 64);
-    const float inv = 1.0f / sqrtf(q / float(kCH) + kCodecEps);
+    const float inv = 1.0f / sqrtf(wave_sum(q) / float(kCH) + kCodecEps);
 #pragma unroll
     for (int i = 0; i < 6; ++i) {
         const int c = lane + 64 * i;
@@ -254,6 +271,16 @@ __global__ __launch_bounds__(64 * kRowsWaves) void codec_rows_kernel(CodecRows a
     const int halo = DW ? kCK / 2 : 0;
     const int t0 = blockIdx.x * kRowsOwn, t = t0 + wave - halo;
     const bool live = t >= 0 && t < a.T && wave < kRowsOwn + 2 * halo;
+    // the depthwise weights of the owned rows' waves, requested with the split sums
+    float dw[6][kCK], db[6];
+    if (DW && wave < kRowsOwn) {
+#pragma unroll
+        for (int i = 0; i < 6; ++i) {
+            db[i] = a.db[lane + 64 * i];
+#pragma unroll
+            for (int k = 0; k < kCK; ++k) dw[i][k] = a.dw[(lane + 64 * i) * kCK + k];
+        }
+    }
     float v[6];
 #pragma unroll
     for (int i = 0; i < 6; ++i) v[i] = 0.0f;
@@ -304,9 +331,9 @@ __global__ __launch_bounds__(64 * kRowsWaves) void codec_rows_kernel(CodecRows a
 #pragma unroll
         for (int i = 0; i < 6; ++i) {
             const int c = lane + 64 * i;
-            float acc = a.db[c];
+            float acc = db[i];
 #pragma unroll
-            for (int k = 0; k < kCK; ++k) acc += xs[wave + k][c] * a.dw[c * kCK + k];
+            for (int k = 0; k < kCK; ++k) acc += xs[wave + k][c] * dw[i][k];
             v[i] = acc;
         }
     } else if (!live) {
@@ -381,7 +408,6 @@ struct CodecEngine {
         return gemm_plan(M, N, K, std::max(1, std::min<int>(max_splits, static_cast<int>(kCodecWsFloats / mn))), false, reduce);
     }
     static GemmPlan embed_plan(int T) { return plan(T, kCH, kCK * kCW, kCodecSplits, false); }
-    static GemmPlan pw2_plan(int T) { return plan(T, kCH, kCF, kCodecSplits, false); }
     static GemmPlan up_plan(int T) { return plan(T, kUpN, kUpTaps * kCW, 8, true); }
     template <class B>
     void grow(B& b, size_t n) {
@@ -397,9 +423,38 @@ struct CodecEngine {
         grow(f, split_elems(T, kCF));
         grow(ypad, split_elems(T + 2, kCW));
         grow(out, static_cast<size_t>(2 * T) * kCW);
-        grow(ws, static_cast<size_t>(T) * std::max({embed_plan(T).splits * kCH, pw2_plan(T).splits * kCH, up_plan(T).splits * kUpN}));
+        grow(ws, static_cast<size_t>(T) * std::max({embed_plan(T).splits * kCH, cut(T, kCH, kCF, kCodecSplits).splits() * kCH, up_plan(T).splits * kUpN}));
     }
 
+    template <int EPI>
+    void gemm_few(CodecGemm g, const GemmSmallPlan& p) {
+        if (EPI == kEpiPartial && ws.n < static_cast<size_t>(p.splits) * g.M * g.N) throw std::logic_error("codec split-K workspace not reserved");
+        g.ws = ws.p;
+        g.kchunk = p.kchunk;
+        const dim3 grid(g.N / 16, p.splits), block(64 * kSmallWaves);
+        switch ((g.M + 15) / 16) {
+            case 1: hipLaunchKernelGGL((codec_gemm_small_kernel<1, EPI>), grid, block, 0, stream, g); break;
+            case 2: hipLaunchKernelGGL((codec_gemm_small_kernel<2, EPI>), grid, block, 0, stream, g); break;
+            case 3: hipLaunchKernelGGL((codec_gemm_small_kernel<3, EPI>), grid, block, 0, stream, g); break;
+            default: hipLaunchKernelGGL((codec_gemm_small_kernel<4, EPI>), grid, block, 0, stream, g); break;
+        }
+        CODEC_CHECK(hipGetLastError());
+    }
+
+    // A plan's cut with what launches it: few rows of a plain operand take the small kernel.
+    struct Cut {
+        GemmSmallPlan few;
+        GemmPlan tiles;
+        int splits() const { return few.splits ? few.splits : tiles.splits; }
+    };
+    static Cut cut(int M, int N, int K, int max_splits) {
+        return {gemm_small_plan(M, N, K, max_splits, false), plan(M, N, K, max_splits, false)};
+    }
+    template <int EPI>
+    void gemm(const CodecGemm& g, const Cut& c) {
+        if (c.few.splits) gemm_few<EPI>(g, c.few);
+        else gemm<EPI, false>(g, c.tiles);
+    }
     template <int EPI, bool CONV>
     void gemm(CodecGemm g, const GemmPlan& p) {
         if (g.N % kGemmBn || g.K % kGemmK || g.M < 1) throw std::logic_error("codec GEMM shape");
@@ -502,7 +557,8 @@ struct CodecEngine {
         hipLaunchKernelGGL(codec_lookup_kernel, dim3(T + 2 * pad), dim3(256), 0, s, dcodes.p, cb.p, op_w.p, op_b.p, xpad.p, ypad.p, T, pad);
         CODEC_CHECK(hipGetLastError());
         const dim3 rows((T + kRowsOwn - 1) / kRowsOwn), threads(64 * kRowsWaves);
-        const GemmPlan pe = embed_plan(T), p2 = pw2_plan(T), pu = up_plan(T), p1 = plan(T, kCF, kCH, 1, false), pd = plan(T, kCW, kCH, 1, false);
+        const GemmPlan pe = embed_plan(T), pu = up_plan(T);
+        const Cut p1 = cut(T, kCF, kCH, 1), p2 = cut(T, kCH, kCF, kCodecSplits), pd = cut(T, kCW, kCH, 1);
         gemm<kEpiPartial, true>({xpad.p, T + 2 * pad, emb_w.p, nullptr, nullptr, nullptr, T, kCH, kCK * kCW, nullptr, 0}, pe);
         hipLaunchKernelGGL((codec_rows_kernel<true, true>), rows, threads, 0, s,
                            CodecRows{ws.p, pe.splits, T, emb_b.p, nullptr, nullptr, x[0].p, n0_w.p, n0_b.p, blk[0].dw.p, blk[0].db.p, blk[0].lw.p,
@@ -510,9 +566,9 @@ struct CodecEngine {
         CODEC_CHECK(hipGetLastError());
         for (int i = 0; i < kCBlocks; ++i) {
             const Block& b = blk[i];
-            gemm<kEpiGelu, false>({hn.p, T, b.w1.p, b.b1.p, nullptr, f.p, T, kCF, kCH, nullptr, 0}, p1);
-            gemm<kEpiPartial, false>({f.p, T, b.w2.p, nullptr, nullptr, nullptr, T, kCH, kCF, nullptr, 0}, p2);
-            CodecRows r{ws.p, p2.splits, T, b.b2.p, b.gamma.p, x[i & 1].p, x[1 - (i & 1)].p, nullptr, nullptr, nullptr, nullptr, fin_w.p, fin_b.p, hn.p};
+            gemm<kEpiGelu>({hn.p, T, b.w1.p, b.b1.p, nullptr, f.p, T, kCF, kCH, nullptr, 0}, p1);
+            gemm<kEpiPartial>({f.p, T, b.w2.p, nullptr, nullptr, nullptr, T, kCH, kCF, nullptr, 0}, p2);
+            CodecRows r{ws.p, p2.splits(), T, b.b2.p, b.gamma.p, x[i & 1].p, x[1 - (i & 1)].p, nullptr, nullptr, nullptr, nullptr, fin_w.p, fin_b.p, hn.p};
             if (i + 1 < kCBlocks) {
                 const Block& n = blk[i + 1];
                 r.dw = n.dw.p;
@@ -525,7 +581,7 @@ struct CodecEngine {
             }
             CODEC_CHECK(hipGetLastError());
         }
-        gemm<kEpiShift, false>({hn.p, T, dec_w.p, dec_b.p, nullptr, ypad.p, T, kCW, kCH, nullptr, 0}, pd);
+        gemm<kEpiShift>({hn.p, T, dec_w.p, dec_b.p, nullptr, ypad.p, T, kCW, kCH, nullptr, 0}, pd);
         const CodecGemm u{ypad.p, T + 2, up_w.p, up_b.p, out.p, nullptr, T, kUpN, kUpTaps * kCW, ws.p, 0};
         if (pu.splits == 1) {
             gemm<kEpiUp, true>(u, pu);

@@ -16,6 +16,8 @@
 // Non-finite inputs: an infinity (or a value past the largest BF16) turns into NaN products, so
 // a result that would have been infinite may come out NaN; NaN stays NaN.
 #pragma once
+#include <algorithm>
+
 #include "common.h"
 
 namespace itts {
@@ -393,6 +395,120 @@ __device__ __forceinline__ void gemm_store_split(uint8_t* lds, int wave, int lan
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         __builtin_amdgcn_wave_barrier();
     }
+}
+
+// ------------------------------------------------------------------ few rows
+// Up to four row tiles: a workgroup of eight waves takes 16 columns and its K range whole,
+// wave w the k steps w, w + 8, ... of it, each with its weights straight from memory to the
+// matrix operand (no LDS, no barrier until the end), two to five steps requested at once.  With so few
+// rows the weights are read once either way and the time is the memory's: 64-column tiles
+// need K splits (and a kernel to add them) to reach every CU, and their steps wait on one
+// another.  More rows: the operand, read by every workgroup, becomes the larger stream.
+constexpr int kSmallWaves = 8;
+constexpr int kSmallK = 32 * kSmallWaves;  // K ranges are multiples of this
+template <int RT>
+struct GemmSmallLds {
+    float sum[kSmallWaves][RT][16][17];
+};
+// Thread t ends with the sum (over the waves, in order) of row t / 16, column t % 16 for
+// t < 256 RT / (RT > 2 ? 2 : 1); with RT > 2, also of row t / 16 + 32 in `out[1]`.  w: the
+// workgroup's first weight row at its first k; a_row_bytes: bytes of a row tile of the operand.
+template <typename WT, int RT>
+__device__ __forceinline__ void gemm_small(GemmSmallLds<RT>& lds, const WT* w, int K, int nst, __amdgpu_buffer_rsrc_t ars, uint32_t a0,
+                                           uint32_t a_row_bytes, int tiles, float (&out)[2]) {
+    constexpr int NL = sizeof(WT) == 4 ? 2 : 1;
+    constexpr int kBatch = RT == 1 ? 5 : 2;  // two workgroups per CU up to two row tiles
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), g = lane >> 4, c = lane & 15;
+    const __amdgpu_buffer_rsrc_t rs = gemm_rsrc(w, static_cast<uint32_t>((static_cast<size_t>(15) * K + nst * 32) * sizeof(WT)));
+    const uint32_t boff = static_cast<uint32_t>((static_cast<size_t>(c) * K + 8 * g) * sizeof(WT));
+    uint32_t aoff[RT];
+#pragma unroll
+    for (int i = 0; i < RT; ++i) aoff[i] = a0 + static_cast<uint32_t>(min(i, tiles - 1)) * a_row_bytes + lane * 16;
+    f32x4 acc[RT], low[2][RT];
+#pragma unroll
+    for (int i = 0; i < RT; ++i) acc[i] = low[0][i] = low[1][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int s0 = wave; s0 < nst; s0 += kSmallWaves * kBatch) {
+        u32x4 b[kBatch][NL];
+        bf16x8 a[kBatch][RT][3];
+#pragma unroll
+        for (int u = 0; u < kBatch; ++u) {  // steps past the last: out of range, zeros, no memory access
+            const int s = s0 + kSmallWaves * u;
+            const uint32_t o = s < nst ? boff + static_cast<uint32_t>(s) * 32 * sizeof(WT) : 0x40000000u;
+#pragma unroll
+            for (int q = 0; q < NL; ++q) b[u][q] = gemm_load16(rs, o + 16 * q, 0);
+        }
+#pragma unroll
+        for (int u = 0; u < kBatch; ++u) {
+            const int s = s0 + kSmallWaves * u;
+#pragma unroll
+            for (int i = 0; i < RT; ++i)
+#pragma unroll
+                for (int p = 0; p < 3; ++p)
+                    a[u][i][p] = __builtin_bit_cast(
+                        bf16x8, gemm_load16(ars, s < nst ? aoff[i] + static_cast<uint32_t>(s) * (kTileElems * 2) + p * kPlaneElems * 2 : 0x7ffffff0u, 0));
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < kBatch; ++u) {
+            u32x4 h, m, l;
+            if constexpr (NL == 2) {
+                float x[8];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) x[i] = __uint_as_float(b[u][i >> 2][i & 3]);
+                split_piece(x, h, m, l);
+            } else {
+                h = b[u][0];
+            }
+            const bf16x8 bh = __builtin_bit_cast(bf16x8, h), bm = __builtin_bit_cast(bf16x8, m), bl = __builtin_bit_cast(bf16x8, l);
+            auto mul = [&](int p, bf16x8 y, f32x4 (&d)[RT]) {
+#pragma unroll
+                for (int i = 0; i < RT; ++i) d[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u][i][p], y, d[i], 0, 0, 0);
+            };
+            mul(0, bh, acc);
+            mul(2, bh, low[0]);
+            mul(1, bh, low[1]);
+            if constexpr (NL == 2) {
+                mul(0, bl, low[0]);
+                mul(0, bm, low[1]);
+                mul(1, bm, low[0]);
+            }
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < RT; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) lds.sum[wave][i][4 * g + r][c] = acc[i][r] + (low[0][i][r] + low[1][i][r]);
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < (RT > 2 ? 2 : 1); ++q) {
+        const int row = (tid >> 4) + 32 * q, i = row >> 4;
+        float v = 0.0f;
+        if (i < RT) {
+#pragma unroll
+            for (int z = 0; z < kSmallWaves; ++z) v += lds.sum[z][i][row & 15][tid & 15];
+        }
+        out[q] = v;
+    }
+}
+// Its cut, or splits 0 where the 64-column tiles are faster.  Measured on MI355X in both kernels
+// (one GEMM with what follows it, weights from HBM, us, 64-column tiles -> this):
+//   at most one workgroup per CU and 1280 k each: 3840 x 1280 at 20 rows 11.0 -> 8.1, at 60 rows
+//   13.1 -> 11.4; 1280 x 1280 at 32 / 60 rows 8.1 -> 6.9 / 9.5 -> 8.2; 1024 x 3072 at 48 rows 10.5 -> 9.8;
+//   5120 x 1280, 320 workgroups: 8 rows 12.9 -> 11.0, but 20 rows 13.5 -> 15.3 (some CUs have two,
+//   and every one reads the whole operand); 1280 x 5120 at 20 rows 12.7 -> 17.8;
+//   BF16 weights (the operand outweighs them sooner): 3840 x 1280 at 32 rows 7.9 -> 6.5, at 63 rows
+//   8.5 -> 9.4.
+struct GemmSmallPlan {
+    int splits, kchunk;
+};
+inline GemmSmallPlan gemm_small_plan(int M, int N, int K, int max_splits, bool bf16) {
+    const int rt = (M + 15) / 16, tiles = N / 16;
+    if (rt > (bf16 ? 2 : 4)) return {0, 0};
+    const int want = std::max(1, std::min(max_splits, 256 / tiles));
+    const int units = (K + kSmallK - 1) / kSmallK, per = (units + want - 1) / want;
+    const GemmSmallPlan p{(units + per - 1) / per, per * kSmallK};
+    if (p.kchunk > 1280 || tiles * p.splits > (rt == 1 ? 400 : 256)) return {0, 0};
+    return p;
 }
 
 // How one GEMM is cut: a tile shape, its row blocks, and K cut into `splits` ranges of kchunk (a

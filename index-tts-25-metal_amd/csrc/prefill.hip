@@ -142,6 +142,41 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_kernel(GemmArgs a, int kchu
     }
 }
 
+// The same for up to 16 RT rows (gemm_core.h, gemm_small).
+template <typename WT, int RT, int EPI, bool SPLIT>
+__global__ __launch_bounds__(64 * kSmallWaves) void gemm_small_kernel(GemmArgs a, int kchunk) {
+    __shared__ GemmSmallLds<RT> lds;
+    const int kb = SPLIT ? blockIdx.y * kchunk : 0, nst = ((SPLIT ? min(a.K, kb + kchunk) : a.K) - kb) / 32;
+    const uint32_t row_bytes = a.K / 32 * (kTileElems * 2);
+    float sum[2];
+    gemm_small<WT, RT>(lds, static_cast<const WT*>(a.w) + static_cast<size_t>(blockIdx.x) * 16 * a.K + kb, a.K, nst,
+                       gemm_rsrc(a.a, static_cast<uint32_t>(split_elems(a.M, a.K) * 2)), kb / 32 * (kTileElems * 2), row_bytes, (a.M + 15) / 16, sum);
+    const int col = blockIdx.x * 16 + (threadIdx.x & 15);
+    const float bias = SPLIT ? 0.0f : a.bias[col];
+#pragma unroll
+    for (int q = 0; q < (RT > 2 ? 2 : 1); ++q) {
+        const int row = (threadIdx.x >> 4) + 32 * q;
+        const bool live = row < a.M;
+        const float v = sum[q] + bias;
+        if constexpr (SPLIT) {
+            if (live) a.ws[(static_cast<size_t>(blockIdx.y) * a.M + row) * a.N + col] = sum[q];
+        } else if constexpr (EPI == kGemmGelu) {
+            if (live) split_store(a.c_split, split_off(row, col, a.N), gelu_f(v));
+        } else if constexpr (EPI == kGemmSwiglu) {
+            const float u = __shfl_xor(v, 1, 64);
+            if (live && !(col & 1)) split_store(a.c_split, split_off(row, col / 2, a.N / 2), swiglu_f(v, u));
+        } else if constexpr (EPI == kGemmQkv) {
+            if (!live) continue;
+            if (col < kWidth) a.c[static_cast<size_t>(row) * kWidth + col] = v;
+            else a.kv[kv_off(a, col - kWidth, a.row_slot[row], a.row_pos[row])] = v;
+        } else {
+            if (!live) continue;
+            float* p = a.c + static_cast<size_t>(row) * a.N + col;
+            *p = EPI == kGemmResid ? *p + v : v;
+        }
+    }
+}
+
 // Partial 0 + partial 1 + ... of four consecutive elements from e on, in split order.  Every
 // split's load is issued before the first add (SM, a power of two >= the split count, loads;
 // indices past the split count reread the last split and their adds are skipped), so the
@@ -370,45 +405,79 @@ void launch_gemm_tile(const GemmArgs& a, const GemmPlan& p, hipStream_t s) {
 
 }  // namespace
 
-static hipError_t launch_gemm_plan(GemmArgs a, int epi, bool bf16, const GemmPlan& p, hipStream_t s) {
-    a.splits = p.splits;
-    if (p.splits > 1) {
-        // the partial tiles do not depend on the epilogue
-        if (bf16) launch_gemm_tile<uint16_t, kGemmStore, true>(a, p, s);
-        else launch_gemm_tile<float, kGemmStore, true>(a, p, s);
-        if (a.ln_out) {
-            hipLaunchKernelGGL(gemm_reduce_ln_kernel, dim3(a.M), dim3(256), 0, s, a);
-            return hipGetLastError();
-        }
+namespace {
+
+template <typename WT, int EPI, bool SPLIT>
+void launch_gemm_small(const GemmArgs& a, const GemmSmallPlan& p, hipStream_t s) {
+    const dim3 grid(a.N / 16, p.splits), block(64 * kSmallWaves);
+    switch (ceil_div(a.M, 16)) {
+        case 1: hipLaunchKernelGGL((gemm_small_kernel<WT, 1, EPI, SPLIT>), grid, block, 0, s, a, p.kchunk); break;
+        case 2: hipLaunchKernelGGL((gemm_small_kernel<WT, 2, EPI, SPLIT>), grid, block, 0, s, a, p.kchunk); break;
+        case 3: hipLaunchKernelGGL((gemm_small_kernel<WT, 3, EPI, SPLIT>), grid, block, 0, s, a, p.kchunk); break;
+        default: hipLaunchKernelGGL((gemm_small_kernel<WT, 4, EPI, SPLIT>), grid, block, 0, s, a, p.kchunk); break;
+    }
+}
+
+// Launches f<weight type, epilogue>() for the epilogue (kGemmStore and kGemmSwiglu: FP32 weights).
+template <class F>
+void with_epilogue(int epi, bool bf16, F f) {
+    switch (epi) {
+        case kGemmQkv: bf16 ? f(uint16_t{}, std::integral_constant<int, kGemmQkv>{}) : f(float{}, std::integral_constant<int, kGemmQkv>{}); break;
+        case kGemmResid: bf16 ? f(uint16_t{}, std::integral_constant<int, kGemmResid>{}) : f(float{}, std::integral_constant<int, kGemmResid>{}); break;
+        case kGemmGelu: bf16 ? f(uint16_t{}, std::integral_constant<int, kGemmGelu>{}) : f(float{}, std::integral_constant<int, kGemmGelu>{}); break;
+        case kGemmStore: f(float{}, std::integral_constant<int, kGemmStore>{}); break;
+        default: f(float{}, std::integral_constant<int, kGemmSwiglu>{}); break;
+    }
+}
+
+// After the partial sums (splits > 1) or the results: the split reduce with the epilogue, the LayerNorm.
+hipError_t finish_gemm(const GemmArgs& a, int epi, hipStream_t s) {
+    if (a.splits == 1) {
+        if (a.ln_out) hipLaunchKernelGGL(ln_rows_kernel, dim3(a.M), dim3(256), 0, s, LnRowsArgs{a.c, a.ln_out, a.ln_w, a.ln_b, a.M});
+    } else if (a.ln_out) {
+        hipLaunchKernelGGL(gemm_reduce_ln_kernel, dim3(a.M), dim3(256), 0, s, a);
+    } else {
         const int w = epi == kGemmSwiglu ? 8 : 4;  // columns of a reduce thread
         const int rblocks = static_cast<int>(std::min<size_t>((static_cast<size_t>(a.M) * a.N / w + 255) / 256, 2048));
-        switch (epi) {
-            case kGemmQkv: hipLaunchKernelGGL((gemm_reduce_kernel<kGemmQkv>), dim3(rblocks), dim3(256), 0, s, a); break;
-            case kGemmResid: hipLaunchKernelGGL((gemm_reduce_kernel<kGemmResid>), dim3(rblocks), dim3(256), 0, s, a); break;
-            case kGemmGelu: hipLaunchKernelGGL((gemm_reduce_kernel<kGemmGelu>), dim3(rblocks), dim3(256), 0, s, a); break;
-            case kGemmStore: hipLaunchKernelGGL((gemm_reduce_kernel<kGemmStore>), dim3(rblocks), dim3(256), 0, s, a); break;
-            default: hipLaunchKernelGGL((gemm_reduce_kernel<kGemmSwiglu>), dim3(rblocks), dim3(256), 0, s, a); break;
-        }
-        return hipGetLastError();
+        with_epilogue(epi, false, [&](auto, auto e) { hipLaunchKernelGGL((gemm_reduce_kernel<decltype(e)::value>), dim3(rblocks), dim3(256), 0, s, a); });
     }
-    switch (epi) {
-        case kGemmQkv: bf16 ? launch_gemm_tile<uint16_t, kGemmQkv, false>(a, p, s) : launch_gemm_tile<float, kGemmQkv, false>(a, p, s); break;
-        case kGemmResid: bf16 ? launch_gemm_tile<uint16_t, kGemmResid, false>(a, p, s) : launch_gemm_tile<float, kGemmResid, false>(a, p, s); break;
-        case kGemmGelu: bf16 ? launch_gemm_tile<uint16_t, kGemmGelu, false>(a, p, s) : launch_gemm_tile<float, kGemmGelu, false>(a, p, s); break;
-        case kGemmStore: launch_gemm_tile<float, kGemmStore, false>(a, p, s); break;
-        default: launch_gemm_tile<float, kGemmSwiglu, false>(a, p, s); break;
-    }
-    if (a.ln_out) hipLaunchKernelGGL(ln_rows_kernel, dim3(a.M), dim3(256), 0, s, LnRowsArgs{a.c, a.ln_out, a.ln_w, a.ln_b, a.M});
     return hipGetLastError();
 }
+
+hipError_t launch_gemm_plan(GemmArgs a, int epi, bool bf16, const GemmPlan& p, hipStream_t s) {
+    a.splits = p.splits;
+    if (p.splits > 1) {  // the partial tiles do not depend on the epilogue
+        if (bf16) launch_gemm_tile<uint16_t, kGemmStore, true>(a, p, s);
+        else launch_gemm_tile<float, kGemmStore, true>(a, p, s);
+    } else {
+        with_epilogue(epi, bf16, [&](auto w, auto e) { launch_gemm_tile<decltype(w), decltype(e)::value, false>(a, p, s); });
+    }
+    return finish_gemm(a, epi, s);
+}
+
+hipError_t launch_gemm_small_plan(GemmArgs a, int epi, bool bf16, const GemmSmallPlan& p, hipStream_t s) {
+    a.splits = p.splits;
+    if (p.splits > 1) {
+        if (bf16) launch_gemm_small<uint16_t, kGemmStore, true>(a, p, s);
+        else launch_gemm_small<float, kGemmStore, true>(a, p, s);
+    } else {
+        with_epilogue(epi, bf16, [&](auto w, auto e) { launch_gemm_small<decltype(w), decltype(e)::value, false>(a, p, s); });
+    }
+    return finish_gemm(a, epi, s);
+}
+
+}  // namespace
 
 hipError_t launch_gemm(const GemmArgs& a, int epi, bool bf16, hipStream_t s) {
     if (a.N % kGemmBn || a.K % kGemmK || a.M < 1 || a.splits < 1 || (a.splits > 1 && !a.ws)) return hipErrorInvalidValue;
     if ((epi == kGemmStore || epi == kGemmSwiglu) && bf16) return hipErrorInvalidValue;  // FP32 weights only (the Qwen decoder)
     if (a.ln_out && (epi != kGemmResid || a.N != kWidth)) return hipErrorInvalidValue;
-    if (split_elems(a.M, a.K) * 2 >= 0x80000000u) return hipErrorInvalidValue;  // 32-bit operand offsets
+    if (split_elems(a.M, a.K) * 2 >= 0x40000000u) return hipErrorInvalidValue;  // 32-bit operand offsets
     const int fit = static_cast<int>(std::min<size_t>(kGemmMaxSplits, kGemmWsFloats / (static_cast<size_t>(a.M) * a.N)));
-    return launch_gemm_plan(a, epi, bf16, gemm_plan(a.M, a.N, a.K, std::max(1, std::min(a.splits, fit)), bf16, true), s);
+    const int splits = std::max(1, std::min(a.splits, fit));
+    const GemmSmallPlan small = gemm_small_plan(a.M, a.N, a.K, splits, bf16);
+    if (small.splits) return launch_gemm_small_plan(a, epi, bf16, small, s);
+    return launch_gemm_plan(a, epi, bf16, gemm_plan(a.M, a.N, a.K, splits, bf16, true), s);
 }
 
 hipError_t launch_causal_attention(const CausalArgs& a, hipStream_t s) {
