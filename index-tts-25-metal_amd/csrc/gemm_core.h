@@ -113,8 +113,7 @@ struct GemmTile {
     static constexpr int WR = WR_, WC = 4 / WR_, TR = TR_, TC = TC_;
     static constexpr int RT = WR * TR, BM = RT * 16, NS = WC * TC, BN = NS * 16;
     static constexpr int PB = sizeof(WT) == 4 ? 3 : 1;       // planes of a weight
-    static constexpr int NP = BN / 64;                       // pieces of a k step per loading thread
-    static constexpr int PD = NP == 1 ? 2 * kGemmUnroll : kGemmUnroll;  // k steps of weights requested ahead
+    static constexpr int PD = 2 * kGemmUnroll;               // k steps of weights requested ahead
     static constexpr int NLOW = TR == 1 ? 2 : 1;             // accumulators of the small products per tile
     static constexpr int NA = TR <= 2 ? 4 : 3;         // operand register sets (NA - 1 k steps ahead)
     static constexpr int kStepElems = NS * PB * kPlaneElems;
@@ -122,7 +121,7 @@ struct GemmTile {
     static constexpr int kEpiFloats = 16 * (16 * TC + 4);
     static constexpr int kLdsBytes =
         kGemmRing * kStepElems * 2 > 4 * kEpiFloats * 4 ? kGemmRing * kStepElems * 2 : 4 * kEpiFloats * 4;
-    static_assert(BN % 64 == 0, "loading threads cover 64 columns");
+    static_assert(BN == 64, "the loading threads cover 64 columns");
 };
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t gemm_rsrc(const void* p, uint32_t bytes) {
@@ -138,7 +137,7 @@ __device__ __forceinline__ u32x4 gemm_load16(__amdgpu_buffer_rsrc_t rs, uint32_t
 }
 
 // ------------------------------------------------------------------ loading waves
-// Thread t of 256 owns, of each 32-wide k step, the piece (column t / 4 (+ 64), eight k at
+// Thread t of 256 owns, of each 32-wide k step, the piece (column t / 4, eight k at
 // 8 (t % 4)): four threads read 128 consecutive bytes of a weight row.  In LDS a piece goes to
 // slot 16 g + (c ^ 2 g) of its strip (g = k / 8 % 4, c = column % 16): eight neighbouring
 // threads (two columns, four g) write, and eight neighbouring lanes (one g, eight c) read,
@@ -148,60 +147,54 @@ __device__ __forceinline__ u32x4 gemm_load16(__amdgpu_buffer_rsrc_t rs, uint32_t
 template <class T>
 __device__ __forceinline__ void gemm_loader(uint16_t* ring, const typename T::W* w, int K, int nst, int t) {
     using WT = typename T::W;
-    constexpr int NL = sizeof(WT) == 4 ? 2 : 1;  // 16-byte loads per piece
+    constexpr int NL = sizeof(WT) == 4 ? 2 : 1;  // 16-byte loads per thread and step
     constexpr int PD = T::PD;
     const __amdgpu_buffer_rsrc_t rs = gemm_rsrc(w, static_cast<uint32_t>((static_cast<size_t>(T::BN - 1) * K + nst * 32) * sizeof(WT)));
-    const int g = t & 3, c0 = t >> 2;
-    uint32_t voff[T::NP];
-    uint16_t* dst[T::NP];
-#pragma unroll
-    for (int p = 0; p < T::NP; ++p) {
-        const int c = c0 + 64 * p;
-        voff[p] = static_cast<uint32_t>((static_cast<size_t>(c) * K + 8 * g) * sizeof(WT));
-        dst[p] = ring + (c >> 4) * T::PB * kPlaneElems + (16 * g + ((c & 15) ^ (2 * g))) * 8;
-    }
-    u32x4 raw[PD][T::NP][NL];
+    constexpr int kAhead = T::PB == 3 ? 3 : 2;  // steps split (FP32) or written ahead of the first barrier
+    const int g = t & 3, c = t >> 2;
+    const uint32_t voff = static_cast<uint32_t>((static_cast<size_t>(c) * K + 8 * g) * sizeof(WT));
+    uint16_t* dst = ring + (c >> 4) * T::PB * kPlaneElems + (16 * g + ((c & 15) ^ (2 * g))) * 8;
+    u32x4 raw[PD][NL];
     auto load = [&](int slot, int s) {  // steps past the last: out of the buffer's range, no memory access
+        const uint32_t o = s < nst ? voff + static_cast<uint32_t>(s) * 32 * sizeof(WT) : 0x40000000u;
 #pragma unroll
-        for (int p = 0; p < T::NP; ++p) {
-            const uint32_t o = s < nst ? voff[p] + static_cast<uint32_t>(s) * 32 * sizeof(WT) : 0x40000000u;
+        for (int q = 0; q < NL; ++q) raw[slot][q] = gemm_load16(rs, o + 16 * q, 0);
+    };
+    u32x4 plane[3];
+    auto split = [&](int slot) {
+        float x[8];
 #pragma unroll
-            for (int q = 0; q < NL; ++q) raw[slot][p][q] = gemm_load16(rs, o + 16 * q, 0);
-        }
+        for (int i = 0; i < 8; ++i) x[i] = __uint_as_float(raw[slot][i / 4 % NL][i & 3]);
+        split_piece(x, plane[0], plane[1], plane[2]);
     };
     int buf = 0;
-    auto put = [&](int slot) {
+    auto put = [&](const u32x4* v) {
 #pragma unroll
-        for (int p = 0; p < T::NP; ++p) {
-            uint16_t* d = dst[p] + buf * T::kStepElems;
-            if constexpr (T::PB == 3) {
-                float x[8];
-#pragma unroll
-                for (int i = 0; i < 8; ++i) x[i] = __uint_as_float(raw[slot][p][i >> 2][i & 3]);
-                u32x4 h, m, l;
-                split_piece(x, h, m, l);
-                *reinterpret_cast<u32x4*>(d) = h;
-                *reinterpret_cast<u32x4*>(d + kPlaneElems) = m;
-                *reinterpret_cast<u32x4*>(d + 2 * kPlaneElems) = l;
-            } else {
-                *reinterpret_cast<u32x4*>(d) = raw[slot][p][0];
-            }
-        }
+        for (int q = 0; q < T::PB; ++q) *reinterpret_cast<u32x4*>(dst + buf * T::kStepElems + q * kPlaneElems) = v[q];
         buf = buf + 1 == kGemmRing ? 0 : buf + 1;
     };
 #pragma unroll
     for (int s = 0; s < PD; ++s) load(s, s);
-    put(0);
-    load(0, PD);
-    put(1);
-    load(1, PD + 1);
+#pragma unroll
+    for (int s = 0; s < kAhead; ++s) {
+        if constexpr (T::PB == 3) split(s);
+        if (s < 2) put(T::PB == 3 ? plane : raw[s]);
+        load(s, PD + s);
+    }
     __syncthreads();
-    // sched_barrier: each step's split stays behind the barrier ahead of it and its loads are
-    // issued at once; moved across, they made a step wait for loads of the steps after it
+    // A step's FP32 pieces were split the step before, so its LDS writes are on their way while the
+    // next pieces are split (about 350 cycles): one after the other, they held up the barrier (155
+    // rows: 3840 x 1280 17.9 -> 16.5 us, 5120 x 1280 20.3 -> 19.7).  Eight loading waves of half a
+    // piece each, or two k steps per barrier, measured the same as this.
+    // sched_barrier: the split stays behind the barrier and its loads are issued at once; moved
+    // across, they made a step wait for loads of the steps after it.
     auto step = [&](int s, int u) {
+        const int n = (u + kAhead) % PD;
         __builtin_amdgcn_sched_barrier(0);
-        put((u + 2) % PD);
-        load((u + 2) % PD, s + u + 2 + PD);
+        put(T::PB == 3 ? plane : raw[n]);
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (T::PB == 3) split(n);
+        load(n, s + u + kAhead + PD);
         __builtin_amdgcn_sched_barrier(0);
         __syncthreads();
     };
