@@ -760,25 +760,33 @@ struct Engine {
         row_pos.ensure(M);
         last_rows.ensure(kMaxBatch);
         pws.ensure(kGemmWsFloats);
-        std::vector<uint32_t> slot(M), pos(M), last(kMaxBatch, 0);
         uint32_t m = 0;
         for (int b = 0; b < nseq; ++b) {
             // a null prefix: its rows were staged in px on the device (generate_segments)
             if (prefixes[b])
                 HIP_CHECK(hipMemcpyAsync(px.p + static_cast<size_t>(m) * kWidth, prefixes[b], static_cast<size_t>(rows[b]) * kWidth * 4,
                                          hipMemcpyHostToDevice, stream));
-            for (uint32_t r = 0; r < rows[b]; ++r) {
-                slot[m + r] = static_cast<uint32_t>(b);
-                pos[m + r] = r;
-            }
             m += rows[b];
-            last[b] = m - 1;
         }
-        HIP_CHECK(hipMemcpyAsync(row_slot.p, slot.data(), M * 4, hipMemcpyHostToDevice, stream));
-        HIP_CHECK(hipMemcpyAsync(row_pos.p, pos.data(), M * 4, hipMemcpyHostToDevice, stream));
-        HIP_CHECK(hipMemcpyAsync(last_rows.p, last.data(), kMaxBatch * 4, hipMemcpyHostToDevice, stream));
-        // Host vectors above must outlive the async copies.
-        HIP_CHECK(hipStreamSynchronize(stream));
+        if (nseq == 1) {  // the row tables of one sequence are formed on the device: no copies, no wait
+            HIP_CHECK(launch_prefill_rows_one(row_slot.p, row_pos.p, last_rows.p, M, stream));
+        } else {
+            std::vector<uint32_t> slot(M), pos(M), last(kMaxBatch, 0);
+            m = 0;
+            for (int b = 0; b < nseq; ++b) {
+                for (uint32_t r = 0; r < rows[b]; ++r) {
+                    slot[m + r] = static_cast<uint32_t>(b);
+                    pos[m + r] = r;
+                }
+                m += rows[b];
+                last[b] = m - 1;
+            }
+            HIP_CHECK(hipMemcpyAsync(row_slot.p, slot.data(), M * 4, hipMemcpyHostToDevice, stream));
+            HIP_CHECK(hipMemcpyAsync(row_pos.p, pos.data(), M * 4, hipMemcpyHostToDevice, stream));
+            HIP_CHECK(hipMemcpyAsync(last_rows.p, last.data(), kMaxBatch * 4, hipMemcpyHostToDevice, stream));
+            // Host vectors above must outlive the async copies.
+            HIP_CHECK(hipStreamSynchronize(stream));
+        }
         enqueue_prefill_layers(PrefillBufs{px.p, pq.p, pxn.p, patt.p, pff.p, row_slot.p, row_pos.p, last_rows.p, pws.p}, nseq, M);
     }
 
