@@ -272,6 +272,7 @@ struct Engine {
     // Persistent single-sequence step (step.hip): one launch per token for batch-1 decode
     // (bitwise the same logits as the multi-kernel path, which ITTS_GPT_PERSISTENT=0 selects).
     bool step_ok = false;
+    bool bf16_step_off = false;  // a BF16 persistent step timed out (a GPU shared with others): multi-kernel from then on
     bool step_batch_ok[kStepBatchMax + 1] = {};  // persistent batch step available for this many sequences
     uint32_t beam_slots = 0;                     // slots the beam row-owner table may name (this search's beams)
     int step_grid = 0;
@@ -553,15 +554,16 @@ struct Engine {
         return s;
     }
 
-    // Raises (and clears) a hand-off timeout reported by the persistent step; call after a sync.
-    void check_step_error() {
-        if (!step_ok) return;
+    // Whether the persistent step reported a hand-off timeout (cleared); call after a sync.
+    bool take_step_error() {
+        if (!step_ok) return false;
         uint32_t e = 0;
         HIP_CHECK(hipMemcpy(&e, step_err.p, sizeof(e), hipMemcpyDeviceToHost));
-        if (e) {
-            HIP_CHECK(hipMemset(step_err.p, 0, sizeof(uint32_t)));
-            throw std::runtime_error("GPT decode step: a workgroup hand-off timed out");
-        }
+        if (e) HIP_CHECK(hipMemset(step_err.p, 0, sizeof(uint32_t)));
+        return e != 0;
+    }
+    void check_step_error() {
+        if (take_step_error()) throw std::runtime_error("GPT decode step: a workgroup hand-off timed out");
     }
     // The persistent path takes one sequence (step.hip) or, when enabled (init_step),
     // 2..kStepBatchMax in one launch (step_batch.hip; with the beam row-owner table when every
@@ -571,7 +573,7 @@ struct Engine {
     // us a call at 250 cached rows); generate()'s documented path there is the multi-kernel graph.
     bool persistent(int nseq, bool use_table, bool sampler = true) const {
         if (!step_ok || nseq < 1 || nseq > kStepBatchMax) return false;
-        if (bf16 && sampler) return false;
+        if (bf16 && (sampler || bf16_step_off)) return false;
         if (use_table) return nseq >= 2 && step_batch_ok[nseq] && beam_slots <= static_cast<uint32_t>(kStepBatchMax);
         return nseq == 1 || step_batch_ok[nseq];
     }
@@ -933,8 +935,15 @@ struct Engine {
             HIP_CHECK(hipMemcpyAsync(out_logits, logits.p, kMelVocab * 4, hipMemcpyDeviceToHost, stream));
             HIP_CHECK(hipStreamSynchronize(stream));
         };
-        if (bf16 && persistent(1, false, false)) exclusive_step(step_dev, run);
-        else run();
+        if (bf16 && persistent(1, false, false)) {
+            exclusive_step(step_dev, run);
+            if (take_step_error()) {  // the multi-kernel path needs no free CUs: it writes the same cache row and logits
+                bf16_step_off = true;
+                run();
+            }
+        } else {
+            run();
+        }
         check_step_error();
         cached++;
     }
