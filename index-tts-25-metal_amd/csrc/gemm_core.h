@@ -115,7 +115,7 @@ struct GemmTile {
     static constexpr int PB = sizeof(WT) == 4 ? 3 : 1;       // planes of a weight
     static constexpr int PD = 2 * kGemmUnroll;               // k steps of weights requested ahead
     static constexpr int NLOW = TR == 1 ? 2 : 1;             // accumulators of the small products per tile
-    static constexpr int NA = TR <= 2 ? 4 : 3;         // operand register sets (NA - 1 k steps ahead)
+    static constexpr int NA = TR <= 2 ? 4 : 3;               // operand register sets (NA - 1 k steps ahead)
     static constexpr int kStepElems = NS * PB * kPlaneElems;
     // the epilogues that write split rows pass each wave's 16 x 16 TC values through LDS
     static constexpr int kEpiFloats = 16 * (16 * TC + 4);
@@ -141,9 +141,9 @@ __device__ __forceinline__ u32x4 gemm_load16(__amdgpu_buffer_rsrc_t rs, uint32_t
 // 8 (t % 4)): four threads read 128 consecutive bytes of a weight row.  In LDS a piece goes to
 // slot 16 g + (c ^ 2 g) of its strip (g = k / 8 % 4, c = column % 16): eight neighbouring
 // threads (two columns, four g) write, and eight neighbouring lanes (one g, eight c) read,
-// eight different 16-byte banks.  k step s + 2 is written while the multiplying waves use step
-// s, one barrier per step; PD steps are in flight from memory.  `w`: the tile's first
-// row, at its first k.
+// eight different 16-byte banks.  k step s + 2 is written while the multiplying waves use step s,
+// one barrier per step; PD steps are in flight from memory.  `w`: the tile's first row, at its
+// first k.
 template <class T>
 __device__ __forceinline__ void gemm_loader(uint16_t* ring, const typename T::W* w, int K, int nst, int t) {
     using WT = typename T::W;
@@ -211,9 +211,9 @@ __device__ __forceinline__ void gemm_loader(uint16_t* ring, const typename T::W*
 
 // ------------------------------------------------------------------ multiplying waves
 // acc[i][c] = (row tile i) x (strip c) over nst k steps.  ars: the split operand; aoff(i, s): this
-// lane's byte offset of row tile i at k step s (of nst), and the part of it that is uniform.  The next strip's weights are read from LDS
-// while the current one's matrix instructions run (the first strip of step s + 1 too: the
-// loading waves finished it before the barrier ahead of step s).
+// lane's byte offset of row tile i at k step s (of nst), and the part of it that is uniform.  The
+// next strip's weights are read from LDS while the current one's matrix instructions run (the
+// first strip of step s + 1 too: the loading waves finished it before the barrier ahead of step s).
 struct GemmOff {
     uint32_t lane, uniform;
 };

@@ -45,6 +45,17 @@ def test_codec_decode_matches_oracle(codec, codec_weights, n):
     _close(got, co.decode(codec_weights, codes), f"decode.{n}")
 
 
+@pytest.mark.parametrize("n", [15, 16, 17, 33, 48, 63, 64, 65, 127, 193])
+def test_codec_decode_tile_edges_match_oracle(codec, codec_weights, n):
+    """Lengths either side of the 16-row operand tiles, of the 64 rows up to which the plain GEMMs
+    take 16-column workgroups, and of the row blocks of the 64-column tiles (the embed and up
+    convolutions read past a tile's rows).  FP32 sums: a tenth of the codec bar, which is what the
+    reference's lengths measure (max-abs 8e-6)."""
+    codes = [int(x) for x in np.random.default_rng(1000 + n).integers(0, 8192, n)]
+    d = np.abs(codec.decode(codes).astype(np.float64) - co.decode(codec_weights, codes))
+    assert float(d.max()) < MAX_ABS / 10 and float(np.sqrt(np.mean(d * d))) < RMSE / 10, (n, float(d.max()))
+
+
 def test_codec_decode_5000_codes_matches_oracle_windows(codec, codec_weights):
     """The longest decode the reference accepts (codec.cpp:58: 1..5000 codes).  An output row
     depends only on the codes within 40 of its own (embed conv7: 3, twelve depthwise conv7:
