@@ -292,9 +292,12 @@ __global__ __launch_bounds__(256) void gemm_reduce_ln_kernel(GemmArgs a) {
 
 // Causal attention over one head for 16 consecutive rows (attn_core.h).  The rows are taken in
 // runs that share a cache slot (stacked sequences: positions restart at 0 in each slot): for
-// each run the slot's keys 0 .. max position, with the other runs' rows seeing none of them
-// (score -inf, weight 0, a rescale of exactly 1).  Later rows have more keys: they start first.
-__global__ __launch_bounds__(64 * kAttnWaves) void causal_attention_kernel(CausalArgs a) {
+// each run the slot's keys 0 .. max position, in a state of its own (a row of another slot has
+// weight 0 there, and 0 times a NaN or an infinite V is NaN), of which the run's rows are
+// stored.  Later rows have more keys: they start first.  Three waves per SIMD: left to the
+// compiler, the state in a loop takes registers for two (571 rows 30.1 us, with three 26.5; 155
+// rows 8.2 and 8.6; one state over all runs 27.7 and 8.35).
+__global__ __launch_bounds__(64 * kAttnWaves, 3) void causal_attention_kernel(CausalArgs a) {
     __shared__ AttnLds<kHeadDim> lds;
     const int m0 = (gridDim.x - 1 - blockIdx.x) * kAttnTile, h = blockIdx.y;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -304,7 +307,14 @@ __global__ __launch_bounds__(64 * kAttnWaves) void causal_attention_kernel(Causa
     SplitFrag q[kHeadDim / 32];
     attn_query<kHeadDim>(a.q + static_cast<size_t>(m0 + qr) * kWidth + h * kHeadDim, lane, q);
     AttnState<kHeadDim> st;
-    for (int r0 = 0; r0 < nq;) {
+    int r0 = 0;
+    auto finish = [&](int r1) {  // the state's rows, r0 .. r1 - 1
+        float out[4];
+        attn_merge<kHeadDim>(lds, st, wave, lane, out);
+        const int r = tid >> 4;
+        if (r >= r0 && r < r1) split_store4(a.out, split_off(m0 + r, h * kHeadDim + 4 * (tid & 15), kWidth), out);
+    };
+    while (true) {
         const int slot = __builtin_amdgcn_readlane(slot_q, r0);
         const uint32_t same = static_cast<uint32_t>(__ballot(slot_q == slot)) & ((1u << nq) - 1u) & ~((1u << r0) - 1u);
         const int r1 = r0 + __popc(same);                                // a slot's rows are consecutive
@@ -313,12 +323,13 @@ __global__ __launch_bounds__(64 * kAttnWaves) void causal_attention_kernel(Causa
         const int pos = qr >= r0 && qr < r1 ? pos_q : -1;
         for (int c0 = wave * kAttnKeys; c0 < kn; c0 += kAttnWaves * kAttnKeys)
             attn_chunk<kHeadDim>(st, q, kb, kb + a.kv_v_off, c0, kn, pos, 0.125f, lane);
+        if (r1 == nq) break;
+        finish(r1);
+        __syncthreads();  // the merge has read its LDS
+        st = AttnState<kHeadDim>();
         r0 = r1;
     }
-    float out[4];
-    attn_merge<kHeadDim>(lds, st, wave, lane, out);
-    const int r = tid >> 4;
-    if (r < nq) split_store4(a.out, split_off(m0 + r, h * kHeadDim + 4 * (tid & 15), kWidth), out);
+    finish(nq);
 }
 
 }  // namespace
