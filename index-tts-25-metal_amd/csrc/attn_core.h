@@ -13,7 +13,9 @@
 //   second product (any order of the keys serves, V is read in the same one), and its
 //   result, dimensions 4 g + r of query q, is rescaled by the lane's own factor.
 // FP32 inputs and weights are split into three BF16 numbers and multiplied with six
-// instructions, the five small products in accumulators of their own (gemm_core.h).
+// instructions, the five small products in accumulators of their own (gemm_core.h).  An infinite
+// or NaN value, and one past the largest BF16, makes every sum that it is in NaN or infinite:
+// attn_refine forms such outputs again with FP32 products.
 #pragma once
 #include "gemm_core.h"
 
@@ -148,6 +150,44 @@ __device__ __forceinline__ void attn_merge(AttnLds<HD>& lds, const AttnState<HD>
     }
 #pragma unroll
     for (int i = 0; i < HD / 16; ++i) out[i] /= den;
+}
+
+// Outputs of attn_merge that are not finite, formed again from the FP32 rows: thread t's query
+// (its row: p) and the keys 0 .. pos() of rows kb / vb, all the same for the 16 threads of a query.
+// The whole wave calls it; `valid` outputs only.
+template <int HD, class Pos>
+__device__ __forceinline__ void attn_refine(const float* p, const float* kb, const float* vb, Pos pos, float scale, bool valid, int lane,
+                                            float (&out)[HD / 16]) {
+    constexpr int D = HD / 16;
+    float t = out[0];
+#pragma unroll
+    for (int i = 1; i < D; ++i) t += out[i];
+    const uint64_t bad = __ballot(valid && !(fabsf(t) <= 3.402823466e38f));
+    if (__builtin_expect(bad == 0, 1)) return;
+    if (((bad >> (lane & 48)) & 0xffff) == 0) return;
+    const int d0 = (lane & 15) * D, keys = pos() + 1;
+    float q[D], m = -INFINITY, l = 0.0f;
+#pragma unroll
+    for (int i = 0; i < D; ++i) q[i] = p[d0 + i];
+    auto score = [&](int k) {
+        float s = 0.0f;
+#pragma unroll
+        for (int i = 0; i < D; ++i) s = __builtin_fmaf(q[i], kb[static_cast<size_t>(k) * HD + d0 + i], s);
+        return row16_sum(s) * scale;
+    };
+#pragma clang loop unroll(disable)
+    for (int k = 0; k < keys; ++k) m = fmaxf(m, score(k));
+#pragma unroll
+    for (int i = 0; i < D; ++i) out[i] = 0.0f;
+#pragma clang loop unroll(disable)
+    for (int k = 0; k < keys && l == l; ++k) {  // (NaN stays)
+        const float w = expf(score(k) - m);
+        l += w;
+#pragma unroll
+        for (int i = 0; i < D; ++i) out[i] = __builtin_fmaf(w, vb[static_cast<size_t>(k) * HD + d0 + i], out[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < D; ++i) out[i] /= l;
 }
 
 // This lane's operand of query row p (HD floats).

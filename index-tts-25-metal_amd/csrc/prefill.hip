@@ -308,18 +308,22 @@ __global__ __launch_bounds__(64 * kAttnWaves, 3) void causal_attention_kernel(Ca
     attn_query<kHeadDim>(a.q + static_cast<size_t>(m0 + qr) * kWidth + h * kHeadDim, lane, q);
     AttnState<kHeadDim> st;
     int r0 = 0;
+    const float* kb = nullptr;  // the run's keys
     auto finish = [&](int r1) {  // the state's rows, r0 .. r1 - 1
         float out[4];
         attn_merge<kHeadDim>(lds, st, wave, lane, out);
-        const int r = tid >> 4;
-        if (r >= r0 && r < r1) split_store4(a.out, split_off(m0 + r, h * kHeadDim + 4 * (tid & 15), kWidth), out);
+        const int r = tid >> 4, rc = min(r, nq - 1);
+        const bool own = r >= r0 && r < r1;
+        attn_refine<kHeadDim>(a.q + static_cast<size_t>(m0 + rc) * kWidth + h * kHeadDim, kb, kb + a.kv_v_off,
+                              [&] { return static_cast<int>(a.row_pos[m0 + rc]); }, 0.125f, own, lane, out);
+        if (own) split_store4(a.out, split_off(m0 + r, h * kHeadDim + 4 * (tid & 15), kWidth), out);
     };
     while (true) {
         const int slot = __builtin_amdgcn_readlane(slot_q, r0);
         const uint32_t same = static_cast<uint32_t>(__ballot(slot_q == slot)) & ((1u << nq) - 1u) & ~((1u << r0) - 1u);
         const int r1 = r0 + __popc(same);                                // a slot's rows are consecutive
         const int kn = __builtin_amdgcn_readlane(pos_q, r1 - 1) + 1;     // and in order
-        const float* kb = a.kv + static_cast<size_t>(slot) * a.kv_slot_stride + a.kv_layer_off + static_cast<size_t>(h) * a.kv_cap * kHeadDim;
+        kb = a.kv + static_cast<size_t>(slot) * a.kv_slot_stride + a.kv_layer_off + static_cast<size_t>(h) * a.kv_cap * kHeadDim;
         const int pos = qr >= r0 && qr < r1 ? pos_q : -1;
         for (int c0 = wave * kAttnKeys; c0 < kn; c0 += kAttnWaves * kAttnKeys)
             attn_chunk<kHeadDim>(st, q, kb, kb + a.kv_v_off, c0, kn, pos, 0.125f, lane);

@@ -607,7 +607,8 @@ __global__ __launch_bounds__(64 * kAttnWaves) void q_causal_attn_kernel(QCausalA
     for (int c0 = wave * kAttnKeys; c0 < kn; c0 += kAttnWaves * kAttnKeys) attn_chunk<kHd>(st, q, a.kc + head, a.vc + head, c0, kn, qr, kScale, lane);
     float out[8];
     attn_merge<kHd>(lds, st, wave, lane, out);
-    const int r = tid >> 4;
+    const int r = tid >> 4, mr = m0 + min(r, nq - 1);
+    attn_refine<kHd>(a.q + static_cast<size_t>(mr) * kQ + h * kHd, a.kc + head, a.vc + head, [&] { return mr; }, kScale, r < nq, lane, out);
     if (r < nq) split_store_piece(a.out, split_off(m0 + r, h * kHd + 8 * (tid & 15), kQ), out);
 }
 

@@ -1,10 +1,20 @@
-"""Infinities, NaN and values near FLT_MAX through the prefill kernels (MI355X)."""
+"""Infinities, NaN and values near FLT_MAX through the prefill kernels (MI355X).
+
+Those kernels split FP32 operands into BF16 numbers, which no infinity and no value past the
+largest BF16 (3.3895e38) survives; what they return must be what FP32 products give.  The models
+here have a finite answer that passes through such a value, so they are compared with the
+oracle, and each fails if one product of the path turns into NaN.
+"""
 import ctypes as C
 
 import numpy as np
 import pytest
 
 pytestmark = pytest.mark.gpu
+
+BIG = np.float32(3.4e38)           # past the largest BF16, below FLT_MAX
+TINY = np.float32(2.0 ** -124)     # BIG * TINY = 15.99
+ROWS = (1, 17, 33, 64, 65, 155, 331)
 
 
 def prefix_of(rows, seed=0):
@@ -42,4 +52,44 @@ def test_short_sequences_sharing_attention_tiles(itts, small_weights, rows, dtyp
     together = dec.generate_batch(prefixes, opts, 8)
     for p, o, r in zip(prefixes, opts, together):
         assert dec.generate(p, o, 8).codes == r.codes
+    dec.close()
+
+
+# ---------------------------------------------------------------------------- GPT
+@pytest.mark.parametrize("rows", ROWS)
+def test_prefill_with_huge_keys_matches_oracle(itts, oracle, rows):
+    """One dimension of a head has key 3.4e38 and query 2^-124 in every row: every score of it gains
+    the same 2, which the softmax takes out again."""
+    w = dict(itts.make_synthetic_weights(layers=2, seed=42, ln_random=True))
+    n = "gpt.gpt.h.0.attn.c_attn."
+    w[n + "weight"], w[n + "bias"] = w[n + "weight"].copy(), w[n + "bias"].copy()
+    for col, value in ((3 * 64 + 5, TINY), (1280 + 3 * 64 + 5, BIG)):
+        w[n + "weight"][:, col] = 0.0
+        w[n + "bias"][col] = value
+    dec, orc = itts.GptDecoder(w, kv_capacity=512), oracle.OracleGpt(w, kv_capacity=512)
+    got, ref = dec.prefill(prefix_of(rows)), orc.prefill(prefix_of(rows))
+    assert np.isfinite(ref).all()
+    assert np.max(np.abs(got - ref)) <= 2e-5 * np.max(np.abs(ref)), np.max(np.abs(got - ref))
+    dec.close()
+
+
+@pytest.mark.parametrize("rows", [2, 16, 17, 40, 155])
+def test_prefill_past_a_row_with_an_infinite_key_matches_oracle(itts, oracle, rows):
+    """Row 0's key overflows to +inf in a dimension where every query is negative: later rows score
+    it -inf and give it no weight.  (Row 0 itself has no finite score; one layer, so its NaN
+    reaches no other row.)"""
+    w = dict(itts.make_synthetic_weights(layers=1, seed=43))
+    n = "gpt.gpt.h.0.attn.c_attn."
+    w[n + "weight"], w[n + "bias"] = w[n + "weight"].copy(), w[n + "bias"].copy()
+    q, k, j = 5 * 64 + 9, 1280 + 5 * 64 + 9, 200
+    w[n + "weight"][:, [q, k]] = 0.0
+    w[n + "bias"][q], w[n + "bias"][k] = -TINY, 0.0
+    w[n + "weight"][j, k] = 1e38   # LayerNorm of row 0 is 35 there, of the others about 0
+    x = prefix_of(rows)
+    x[0, j] = 1000.0
+    x[1:, j] = x[1:].mean(-1)
+    dec, orc = itts.GptDecoder(w, kv_capacity=512), oracle.OracleGpt(w, kv_capacity=512)
+    got, ref = dec.prefill(x), orc.prefill(x)
+    assert np.isfinite(ref).all()
+    assert np.max(np.abs(got - ref)) <= 2e-5 * np.max(np.abs(ref)), np.max(np.abs(got - ref))
     dec.close()
