@@ -113,6 +113,16 @@ struct CodecGemm {
     int kchunk;          // K per split
 };
 
+// One result of a GEMM: the sum of row `row` and column `col` (of K range z).
+template <int EPI>
+__device__ __forceinline__ void codec_store_one(const CodecGemm& g, int z, int row, int col, float sum) {
+    if (row >= g.M) return;
+    if constexpr (EPI == kEpiPartial) g.ws[(static_cast<size_t>(z) * g.M + row) * g.N + col] = sum;
+    else if constexpr (EPI == kEpiGelu) split_store(g.cs, split_off(row, col, g.N), codec_gelu(sum + g.bias[col]));
+    else if constexpr (EPI == kEpiShift) split_store(g.cs, split_off(row + 1, col, g.N), sum + g.bias[col]);
+    else g.c[(2 * static_cast<size_t>(row) + (col >= kCW ? 1 : 0)) * kCW + (col & (kCW - 1))] = sum + g.bias[col];
+}
+
 template <class T, int EPI, bool CONV>
 __global__ __launch_bounds__(kGemmThreads) void codec_gemm_kernel(CodecGemm g) {
     __shared__ __align__(16) uint8_t lds[T::kLdsBytes];
@@ -130,7 +140,7 @@ __global__ __launch_bounds__(kGemmThreads) void codec_gemm_kernel(CodecGemm g) {
     const int tile0 = by * T::RT + wr * TR;
     const int akt = CONV ? kCW / 32 : g.K / 32;  // k steps of an operand row
     const __amdgpu_buffer_rsrc_t ars = gemm_rsrc(g.a, static_cast<uint32_t>(split_elems(g.a_rows, akt * 32) * 2));
-    f32x4 acc[TR][TC];
+    GemmAcc<T> sums;
     if constexpr (CONV) {
         // k step s is step s % 32 of tap s / 32, which reads a row further down; rows past the
         // operand's buffer read as zero (result rows past M only)
@@ -142,16 +152,32 @@ __global__ __launch_bounds__(kGemmThreads) void codec_gemm_kernel(CodecGemm g) {
                 return GemmOff{static_cast<uint32_t>(row >> 4) * (kCW / 32 * kTileElems * 2) + ((row & 15) + (lane & 48)) * 16,
                                static_cast<uint32_t>(sg & 31) * (kTileElems * 2)};
             },
-            nst, wc, lane, acc);
+            nst, wc, lane, sums);
     } else {
         const int tiles = (g.M + 15) / 16;
         uint32_t off[TR];
 #pragma unroll
         for (int i = 0; i < TR; ++i) off[i] = (static_cast<uint32_t>(min(tile0 + i, tiles - 1)) * akt + kb / 32) * (kTileElems * 2) + lane * 16;
         gemm_compute<T>(
-            ring, ars, [&](int i, int s) { return GemmOff{off[i], static_cast<uint32_t>(s) * (kTileElems * 2)}; }, nst, wc, lane, acc);
+            ring, ars, [&](int i, int s) { return GemmOff{off[i], static_cast<uint32_t>(s) * (kTileElems * 2)}; }, nst, wc, lane, sums);
     }
-    const int cw = bx * T::BN + wc * TC * 16, col0 = cw + (lane & 15);
+    const int n0 = bx * T::BN + wc * TC * 16;  // the wave's first column
+    const auto dot = [&](int m, int n) {
+        return gemm_dot(g.w + static_cast<size_t>(n0 + n) * g.K + kb, nst * 32, [&](int k) {
+            const int kk = kb + k;  // of a convolution: tap kk / kCW, a row further down each
+            return split_value(g.a + (CONV ? split_off(m + (n0 >= kCW ? 1 : 0) + kk / kCW, kk % kCW, kCW) : split_off(m, kk, g.K)));
+        });
+    };
+    const bool suspect = sums.suspect();
+    if constexpr (EPI == kEpiPartial || EPI == kEpiUp) {
+        if (__builtin_expect(suspect, 0)) {
+            gemm_refine<T>(lds, g.M, tile0, wave, lane, sums, dot, [&](int m, int n, float v) { codec_store_one<EPI>(g, bz, m, n0 + n, v); });
+            return;
+        }
+    }
+    f32x4 acc[TR][TC];
+    sums.sum(acc);
+    const int col0 = n0 + (lane & 15);
     if constexpr (EPI == kEpiPartial) {
         gemm_store_partial<T>(g.ws + static_cast<size_t>(bz) * g.M * g.N, g.M, g.N, tile0, col0, lane, acc);
     } else {
@@ -159,10 +185,13 @@ __global__ __launch_bounds__(kGemmThreads) void codec_gemm_kernel(CodecGemm g) {
 #pragma unroll
         for (int c = 0; c < TC; ++c) bias[c] = g.bias[col0 + 16 * c];
         if constexpr (EPI == kEpiGelu) {
-            gemm_store_split<T, false>(lds, wave, lane, g.cs, g.M, g.N, 0, tile0, cw,
-                                       [&](int i, int c, int r) { return codec_gelu(acc[i][c][r] + bias[c]); });
+            gemm_store_split<T, false>(
+                lds, wave, lane, g.cs, g.M, g.N, 0, tile0, n0, [&](int i, int c, int r) { return codec_gelu(acc[i][c][r] + bias[c]); }, suspect,
+                [&](int m, int n) { return codec_gelu(dot(m, n) + g.bias[n0 + n]); });
         } else if constexpr (EPI == kEpiShift) {
-            gemm_store_split<T, false>(lds, wave, lane, g.cs, g.M, g.N, 1, tile0, cw, [&](int i, int c, int r) { return acc[i][c][r] + bias[c]; });
+            gemm_store_split<T, false>(
+                lds, wave, lane, g.cs, g.M, g.N, 1, tile0, n0, [&](int i, int c, int r) { return acc[i][c][r] + bias[c]; }, suspect,
+                [&](int m, int n) { return dot(m, n) + g.bias[n0 + n]; });
         } else {
 #pragma unroll
             for (int i = 0; i < TR; ++i) {
@@ -174,7 +203,7 @@ __global__ __launch_bounds__(kGemmThreads) void codec_gemm_kernel(CodecGemm g) {
                         acc[i][c][r] += bias[c];
                         pin_value(acc[i][c][r]);
                     }
-                const int odd = cw >= kCW ? 1 : 0;
+                const int odd = n0 >= kCW ? 1 : 0;
 #pragma unroll
                 for (int r = 0; r < 4; ++r)
                     if (row + r < g.M) {
@@ -195,17 +224,10 @@ __global__ __launch_bounds__(64 * kSmallWaves) void codec_gemm_small_kernel(Code
     float sum[2];
     gemm_small<float, RT>(lds, g.w + static_cast<size_t>(blockIdx.x) * 16 * g.K + kb, g.K, nst,
                           gemm_rsrc(g.a, static_cast<uint32_t>(split_elems(g.M, g.K) * 2)), kb / 32 * (kTileElems * 2),
-                          g.K / 32 * (kTileElems * 2), (g.M + 15) / 16, sum);
-    const int col = blockIdx.x * 16 + (threadIdx.x & 15);
-    const float bias = EPI == kEpiPartial ? 0.0f : g.bias[col];
+                          g.K / 32 * (kTileElems * 2), g.M, [&](int m, int k) { return split_value(g.a + split_off(m, kb + k, g.K)); }, sum);
 #pragma unroll
-    for (int q = 0; q < (RT > 2 ? 2 : 1); ++q) {
-        const int row = (threadIdx.x >> 4) + 32 * q;
-        if (row >= g.M) continue;
-        if constexpr (EPI == kEpiPartial) g.ws[(static_cast<size_t>(blockIdx.y) * g.M + row) * g.N + col] = sum[q];
-        else if constexpr (EPI == kEpiGelu) split_store(g.cs, split_off(row, col, g.N), codec_gelu(sum[q] + bias));
-        else split_store(g.cs, split_off(row + 1, col, g.N), sum[q] + bias);
-    }
+    for (int q = 0; q < (RT > 2 ? 2 : 1); ++q)
+        codec_store_one<EPI>(g, blockIdx.y, (threadIdx.x >> 4) + 32 * q, blockIdx.x * 16 + (threadIdx.x & 15), sum[q]);
 }
 
 // The up conv's splits, added in split order, + bias; a thread takes four columns.
@@ -409,9 +431,12 @@ struct CodecEngine {
     }
     static GemmPlan embed_plan(int T) { return plan(T, kCH, kCK * kCW, kCodecSplits, false); }
     static GemmPlan up_plan(int T) { return plan(T, kUpN, kUpTaps * kCW, 8, true); }
-    template <class B>
-    void grow(B& b, size_t n) {
-        if (b.ensure(n)) ++generation;
+    template <class T>
+    void grow(Buf<T>& b, size_t n) {
+        if (!b.ensure(n)) return;
+        ++generation;
+        if (std::is_same_v<T, uint16_t>)  // padding rows of operands: finite, whatever the memory held
+            CODEC_CHECK(hipMemsetAsync(b.p, 0, b.n * sizeof(T), stream));
     }
     // Every buffer a decode of T codes touches, sized before anything is queued (and captured).
     void reserve(int T) {

@@ -5,16 +5,19 @@
 // to what the ones before it leave (8 + 8 + 8 significant bits: nothing is left over), and a
 // product is the sum of the six partial products whose size can reach an FP32 rounding:
 //   hi hi + (hi mid + mid hi) + (mid mid + hi lo + lo hi),
-// each exact in the matrix cores and added in FP32.  The three dropped products are below
-// 2^-25 of hi hi, less than the rounding of one FP32 addition.  A BF16 weight is its own hi:
+// each exact in the matrix cores and added in FP32.  Of the three dropped products, mid lo and
+// lo mid are at most 2^-25 of |hi hi| each and 2^-24 together, half a unit in the last place of
+// one product, and lo lo is 2^-34 of it.  A BF16 weight is its own hi:
 // three products.  The hi hi products have an accumulator of their own and the others, 2^-8
 // of it and less, a second one added at the end, so the running sum is rounded by one
 // instruction in six (all six into one accumulator: twice the error, and above the FP32
 // instruction's).  Against that instruction (v_mfma_f32_16x16x4f32: 2048 FLOP in 32 cycles) six
 // v_mfma_f32_16x16x32_bf16 (16384 FLOP in 16 cycles each) take 96 cycles where it takes 256.
 //
-// Non-finite inputs: an infinity (or a value past the largest BF16) turns into NaN products, so
-// a result that would have been infinite may come out NaN; NaN stays NaN.
+// Infinities, NaN and weights past the largest BF16 do not survive the split: they make every sum
+// of the small products that they are in NaN or infinite.  Such a tile's results are formed again
+// with FP32 products where they are not finite (gemm_refine): an activation's value is in its
+// three numbers all the same, a weight's is in memory.
 #pragma once
 #include <algorithm>
 
@@ -31,8 +34,9 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 // mid and lo planes of 64 pieces of eight consecutive k, piece 16 (k / 8 % 4) + row % 16.  A
 // plane of a tile is what the 64 lanes of one matrix instruction hold (lane l: row l & 15,
 // k 8 (l >> 4) .. + 7), 1 KB in lane order, so a wave reads its operand with one 16-byte load
-// per lane and no LDS.  Rows are padded to a multiple of 16; the padding is never written
-// (a result row depends on its own operand row only).
+// per lane and no LDS.  Rows are padded to a multiple of 16.  The padding is zeroed when the
+// buffer is made and then holds what longer operands left: a result row depends on its own
+// operand row only, but NaN in the padding sends its tile through the slower epilogue.
 constexpr int kPlaneElems = 512;              // one plane of a tile
 constexpr int kTileElems = 3 * kPlaneElems;   // hi, mid, lo
 __host__ __device__ inline size_t split_elems(size_t rows, size_t k) { return (rows + 15) / 16 * 16 * k * 3; }
@@ -48,19 +52,23 @@ __device__ __forceinline__ uint32_t bf16_pair(float a, float b) {
 __device__ __forceinline__ float bf16_lo(uint32_t v) { return __uint_as_float(v << 16); }
 __device__ __forceinline__ float bf16_hi(uint32_t v) { return __uint_as_float(v & 0xffff0000u); }
 
-// hi, mid and lo of a pair; x - hi and (x - hi) - mid are exact.
+// hi, mid and lo of a pair; x - hi and (x - hi) - mid are exact.  STORED: hi is at most the largest
+// BF16, so a finite x is hi + (mid + lo) whatever its size, and mid is infinite if x is (split_value).
+constexpr float kBf16Max = 3.3895314e38f;
+template <bool STORED = false>
 __device__ __forceinline__ void split_pair(float a, float b, uint32_t& h, uint32_t& m, uint32_t& l) {
-    h = bf16_pair(a, b);
+    h = STORED ? bf16_pair(__builtin_amdgcn_fmed3f(a, -kBf16Max, kBf16Max), __builtin_amdgcn_fmed3f(b, -kBf16Max, kBf16Max)) : bf16_pair(a, b);
     a -= bf16_lo(h);
     b -= bf16_hi(h);
     m = bf16_pair(a, b);
     l = bf16_pair(a - bf16_lo(m), b - bf16_hi(m));
 }
+template <bool STORED = false>
 __device__ __forceinline__ void split_piece(const float (&x)[8], u32x4& h, u32x4& m, u32x4& l) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         uint32_t a, b, c;
-        split_pair(x[2 * i], x[2 * i + 1], a, b, c);
+        split_pair<STORED>(x[2 * i], x[2 * i + 1], a, b, c);
         h[i] = a;
         m[i] = b;
         l[i] = c;
@@ -69,7 +77,7 @@ __device__ __forceinline__ void split_piece(const float (&x)[8], u32x4& h, u32x4
 // Stores one element / four / one eight-element piece of a split operand.
 __device__ __forceinline__ void split_store(uint16_t* p, size_t off, float x) {
     uint32_t h, m, l;
-    split_pair(x, 0.0f, h, m, l);
+    split_pair<true>(x, 0.0f, h, m, l);
     p[off] = static_cast<uint16_t>(h);
     p[off + kPlaneElems] = static_cast<uint16_t>(m);
     p[off + 2 * kPlaneElems] = static_cast<uint16_t>(l);
@@ -80,7 +88,7 @@ __device__ __forceinline__ void split_store4(uint16_t* p, size_t off, const floa
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
         uint32_t a, b, c;
-        split_pair(x[2 * i], x[2 * i + 1], a, b, c);
+        split_pair<true>(x[2 * i], x[2 * i + 1], a, b, c);
         h[i] = a;
         m[i] = b;
         l[i] = c;
@@ -91,10 +99,29 @@ __device__ __forceinline__ void split_store4(uint16_t* p, size_t off, const floa
 }
 __device__ __forceinline__ void split_store_piece(uint16_t* p, size_t off, const float (&x)[8]) {
     u32x4 h, m, l;
-    split_piece(x, h, m, l);
+    split_piece<true>(x, h, m, l);
     *reinterpret_cast<u32x4*>(p + off) = h;
     *reinterpret_cast<u32x4*>(p + off + kPlaneElems) = m;
     *reinterpret_cast<u32x4*>(p + off + 2 * kPlaneElems) = l;
+}
+
+// The value stored at p (its hi).
+__device__ __forceinline__ float split_value(const uint16_t* p) {
+    const float h = bf16_to_f32(p[0]), m = bf16_to_f32(p[kPlaneElems]), l = bf16_to_f32(p[2 * kPlaneElems]);
+    return fabsf(m) == INFINITY ? m : h + (m + l);
+}
+
+// One sum in FP32, in k order: a(k) is the operand's value, w the weight row at its first k.
+// NaN stays NaN, and ends it.
+__device__ __forceinline__ bool not_finite(float v) { return !(fabsf(v) <= 3.402823466e38f); }
+__device__ __forceinline__ float gemm_weight(float w) { return w; }
+__device__ __forceinline__ float gemm_weight(uint16_t w) { return bf16_to_f32(w); }
+template <typename WT, class A>
+__device__ __forceinline__ float gemm_dot(const WT* w, int len, A a) {
+    float s = 0.0f;
+#pragma clang loop unroll(disable)
+    for (int k = 0; k < len && s == s; ++k) s = __builtin_fmaf(a(k), gemm_weight(w[k]), s);
+    return s;
 }
 
 // ------------------------------------------------------------------ tile shapes
@@ -210,7 +237,32 @@ __device__ __forceinline__ void gemm_loader(uint16_t* ring, const typename T::W*
 }
 
 // ------------------------------------------------------------------ multiplying waves
-// acc[i][c] = (row tile i) x (strip c) over nst k steps.  ars: the split operand; aoff(i, s): this
+// A wave's sums of the hi hi products and of the small ones: (row tile i) x (strip c).
+template <class T>
+struct GemmAcc {
+    f32x4 hi[T::TR][T::TC], low[T::NLOW][T::TR][T::TC];
+    __device__ __forceinline__ f32x4 small(int i, int c) const { return T::NLOW == 2 ? low[0][i][c] + low[1][i][c] : low[0][i][c]; }
+    __device__ __forceinline__ void sum(f32x4 (&acc)[T::TR][T::TC]) const {
+#pragma unroll
+        for (int i = 0; i < T::TR; ++i)
+#pragma unroll
+            for (int c = 0; c < T::TC; ++c) acc[i][c] = hi[i][c] + small(i, c);
+    }
+    // Whether gemm_refine is needed.  An operand that is not finite shows in the small products of
+    // its whole row, a weight (or one past the largest BF16) in those of its whole column.
+    __device__ __forceinline__ bool suspect() const {
+        float t = 0.0f;
+#pragma unroll
+        for (int i = 0; i < T::TR; ++i) {
+            const f32x4 v = small(i, 0);
+            t += (v[0] + v[1]) + (v[2] + v[3]);
+        }
+#pragma unroll
+        for (int c = 1; c < T::TC; ++c) t += T::NLOW == 2 ? low[0][0][c][0] + low[1][0][c][0] : low[0][0][c][0];
+        return __ballot(not_finite(t)) != 0;
+    }
+};
+// acc over nst k steps.  ars: the split operand; aoff(i, s): this
 // lane's byte offset of row tile i at k step s (of nst), and the part of it that is uniform.  The
 // next strip's weights are read from LDS while the current one's matrix instructions run (the
 // first strip of step s + 1 too: the loading waves finished it before the barrier ahead of step s).
@@ -219,15 +271,14 @@ struct GemmOff {
 };
 template <class T, class AOff>
 __device__ __forceinline__ void gemm_compute(const uint16_t* ring, __amdgpu_buffer_rsrc_t ars, AOff aoff, int nst, int wc, int lane,
-                                             f32x4 (&acc)[T::TR][T::TC]) {
+                                             GemmAcc<T>& acc) {
     bf16x8 av[T::NA][T::TR][3], bv[2][T::PB];
-    f32x4 low[T::NLOW][T::TR][T::TC];
 #pragma unroll
     for (int q = 0; q < T::NLOW; ++q)
 #pragma unroll
         for (int i = 0; i < T::TR; ++i)
 #pragma unroll
-            for (int c = 0; c < T::TC; ++c) low[q][i][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+            for (int c = 0; c < T::TC; ++c) acc.low[q][i][c] = f32x4{0.f, 0.f, 0.f, 0.f};
     auto load_a = [&](int set, int s, int i, int p) {  // plane p of row tile i; steps past the last reread it
         const GemmOff o = aoff(i, min(s, nst - 1));
         av[set][i][p] = __builtin_bit_cast(bf16x8, gemm_load16(ars, o.lane + p * kPlaneElems * 2, o.uniform));
@@ -235,7 +286,7 @@ __device__ __forceinline__ void gemm_compute(const uint16_t* ring, __amdgpu_buff
 #pragma unroll
     for (int i = 0; i < T::TR; ++i)
 #pragma unroll
-        for (int c = 0; c < T::TC; ++c) acc[i][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int c = 0; c < T::TC; ++c) acc.hi[i][c] = f32x4{0.f, 0.f, 0.f, 0.f};
     const int g = lane >> 4;
     const uint16_t* src = ring + wc * T::TC * T::PB * kPlaneElems + (16 * g + ((lane & 15) ^ (2 * g))) * 8;
     int buf = 0;
@@ -270,7 +321,7 @@ __device__ __forceinline__ void gemm_compute(const uint16_t* ring, __amdgpu_buff
                     else load_b(cur ^ 1, nbuf, 0, g);
                 }
                 __builtin_amdgcn_sched_barrier(0);
-                auto& d = g == 0 ? acc : low[(g + 1) % T::NLOW];
+                auto& d = g == 0 ? acc.hi : acc.low[(g + 1) % T::NLOW];
 #pragma unroll
                 for (int i = 0; i < T::TR; ++i)
                     d[i][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[u % T::NA][i][pa[g]], bv[cur][pb[g]], d[i][c], 0, 0, 0);
@@ -297,10 +348,6 @@ __device__ __forceinline__ void gemm_compute(const uint16_t* ring, __amdgpu_buff
             }
         }
     }
-#pragma unroll
-    for (int i = 0; i < T::TR; ++i)
-#pragma unroll
-        for (int c = 0; c < T::TC; ++c) acc[i][c] += T::NLOW == 2 ? low[0][i][c] + low[1][i][c] : low[0][i][c];
 }
 
 // ------------------------------------------------------------------ placement and results
@@ -353,13 +400,50 @@ __device__ __forceinline__ void gemm_store_partial(float* ws, int M, int N, int 
             }
 }
 
+// The epilogue of a suspect tile: each sum that is not finite is formed again, dot(m, n) for row m
+// and column n of the wave's tile, and store(m, n, v) takes them all (rows past M too).  The tile
+// passes through the wave's part of LDS (the ring is no longer read), so that the loop is over
+// memory and not over registers, and the ordinary epilogue stays as it is (155 rows, 3840 x 1280:
+// 22.0 us without this and with it; sums corrected in their registers took 22.7, by the copies
+// and by the stores that had to wait for the test).  For epilogues that only add: another copy of
+// a function's code may round a finite value differently (gemm_store_split).
+template <class T, class Dot, class Store>
+__device__ __forceinline__ void gemm_refine(uint8_t* lds, int M, int tile0, int wave, int lane, const GemmAcc<T>& acc, Dot dot, Store store) {
+    constexpr int W = 16 * T::TC, S = W + 4;
+    float* buf = reinterpret_cast<float*>(lds) + wave * T::kEpiFloats;
+#pragma unroll
+    for (int i = 0; i < T::TR; ++i) {
+#pragma unroll
+        for (int c = 0; c < T::TC; ++c)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                float l = T::NLOW == 2 ? acc.low[0][i][c][r] + acc.low[1][i][c][r] : acc.low[0][i][c][r];
+                asm volatile("" : "+v"(l));  // an addition of this branch, not shared with the ordinary epilogue's
+                buf[(4 * (lane >> 4) + r) * S + 16 * c + (lane & 15)] = acc.hi[i][c][r] + l;
+            }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+#pragma clang loop unroll(disable)
+        for (int q = lane; q < 16 * W; q += 64) {
+            const int n = q % W, m = (tile0 + i) * 16 + q / W;
+            float v = buf[q / W * S + n];
+            if (m < M && not_finite(v)) v = dot(m, n);
+            store(m, n, v);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    }
+}
+
 // Results as split rows of the next GEMM's operand ([.][on], from row row_off on): each wave
 // passes its row tiles through its own part of LDS (the ring is no longer read), so that a lane
 // holds eight consecutive columns.  f(i, c, r) is the value of acc[i][c][r]; with PAIRS, of a
-// column pair, given in its even lane, and `oc0` counts pairs.
-template <class T, bool PAIRS, class F>
-__device__ __forceinline__ void gemm_store_split(uint8_t* lds, int wave, int lane, uint16_t* out, int M, int on, int row_off, int tile0, int oc0,
-                                                 F f) {
+// column pair, given in its even lane, and `oc0` counts pairs.  `suspect`: values that are not
+// finite are replaced by again(m, n), row m and column (pair) n of the wave's tile, the value from
+// sums formed again.
+template <class T, bool PAIRS, class F, class G>
+__device__ __forceinline__ void gemm_store_split(uint8_t* lds, int wave, int lane, uint16_t* out, int M, int on, int row_off, int tile0, int oc0, F f,
+                                                 bool suspect, G again) {
     constexpr int W = PAIRS ? 8 * T::TC : 16 * T::TC, S = W + 4;  // columns written; row stride
     float* buf = reinterpret_cast<float*>(lds) + wave * T::kEpiFloats;
     const int rq = 4 * (lane >> 4);
@@ -378,6 +462,15 @@ __device__ __forceinline__ void gemm_store_split(uint8_t* lds, int wave, int lan
             }
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         __builtin_amdgcn_wave_barrier();
+        if (__builtin_expect(suspect, 0)) {
+#pragma clang loop unroll(disable)
+            for (int q = lane; q < 16 * W; q += 64) {
+                const int n = q % W, m = (tile0 + i) * 16 + q / W;
+                if (m < M && not_finite(buf[q / W * S + n])) buf[q / W * S + n] = again(m, n);
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+        }
         for (int q = lane; q < 2 * W; q += 64) {
             const int r = q & 15, e0 = 8 * (q >> 4), row = (tile0 + i) * 16 + r;
             float x[8];
@@ -406,9 +499,10 @@ struct GemmSmallLds {
 // Thread t ends with the sum (over the waves, in order) of row t / 16, column t % 16 for
 // t < 256 RT / (RT > 2 ? 2 : 1); with RT > 2, also of row t / 16 + 32 in `out[1]`.  w: the
 // workgroup's first weight row at its first k; a_row_bytes: bytes of a row tile of the operand.
-template <typename WT, int RT>
+// Sums of rows below M that are not finite are formed again: value(m, k) as gemm_refine's a.
+template <typename WT, int RT, class A>
 __device__ __forceinline__ void gemm_small(GemmSmallLds<RT>& lds, const WT* w, int K, int nst, __amdgpu_buffer_rsrc_t ars, uint32_t a0,
-                                           uint32_t a_row_bytes, int tiles, float (&out)[2]) {
+                                           uint32_t a_row_bytes, int M, A value, float (&out)[2]) {
     constexpr int NL = sizeof(WT) == 4 ? 2 : 1;
     constexpr int kBatch = RT == 1 ? 5 : 2;  // two workgroups per CU up to two row tiles
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), g = lane >> 4, c = lane & 15;
@@ -416,7 +510,7 @@ __device__ __forceinline__ void gemm_small(GemmSmallLds<RT>& lds, const WT* w, i
     const uint32_t boff = static_cast<uint32_t>((static_cast<size_t>(c) * K + 8 * g) * sizeof(WT));
     uint32_t aoff[RT];
 #pragma unroll
-    for (int i = 0; i < RT; ++i) aoff[i] = a0 + static_cast<uint32_t>(min(i, tiles - 1)) * a_row_bytes + lane * 16;
+    for (int i = 0; i < RT; ++i) aoff[i] = a0 + static_cast<uint32_t>(min(i, (M - 1) >> 4)) * a_row_bytes + lane * 16;
     f32x4 acc[RT], low[2][RT];
 #pragma unroll
     for (int i = 0; i < RT; ++i) acc[i] = low[0][i] = low[1][i] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -480,6 +574,8 @@ __device__ __forceinline__ void gemm_small(GemmSmallLds<RT>& lds, const WT* w, i
 #pragma unroll
             for (int z = 0; z < kSmallWaves; ++z) v += lds.sum[z][i][row & 15][tid & 15];
         }
+        if (__builtin_expect(not_finite(v) && row < M, 0))
+            v = gemm_dot(w + static_cast<size_t>(tid & 15) * K, nst * 32, [&](int k) { return value(row, k); });
         out[q] = v;
     }
 }

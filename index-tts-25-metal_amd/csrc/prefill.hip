@@ -47,6 +47,30 @@ __device__ __forceinline__ size_t kv_off(const GemmArgs& a, int rr, uint32_t slo
            (static_cast<size_t>(c >> 6) * a.kv_cap + pos) * kHeadDim + (c & 63);
 }
 
+// One result of a GEMM: the sum of row `row` and column `col` (of split z).  Every lane of a wave calls
+// it, lanes l and l ^ 1 with columns col and col ^ 1 of a row; rows past the last are not stored.
+template <int EPI, bool SPLIT>
+__device__ __forceinline__ void gemm_store_one(const GemmArgs& a, int z, int row, int col, float sum) {
+    const bool live = row < a.M;
+    const float v = sum + (SPLIT ? 0.0f : a.bias[col]);
+    if constexpr (SPLIT) {
+        if (live) a.ws[(static_cast<size_t>(z) * a.M + row) * a.N + col] = sum;
+    } else if constexpr (EPI == kGemmGelu) {
+        if (live) split_store(a.c_split, split_off(row, col, a.N), gelu_f(v));
+    } else if constexpr (EPI == kGemmSwiglu) {
+        const float u = __shfl_xor(v, 1, 64);
+        if (live && !(col & 1)) split_store(a.c_split, split_off(row, col / 2, a.N / 2), swiglu_f(v, u));
+    } else if constexpr (EPI == kGemmQkv) {
+        if (!live) return;
+        if (col < kWidth) a.c[static_cast<size_t>(row) * kWidth + col] = v;
+        else a.kv[kv_off(a, col - kWidth, a.row_slot[row], a.row_pos[row])] = v;
+    } else {
+        if (!live) return;
+        float* p = a.c + static_cast<size_t>(row) * a.N + col;
+        *p = EPI == kGemmResid ? *p + v : v;
+    }
+}
+
 // Row block y covers row tiles [y RT, (y + 1) RT) of A; split z covers K range
 // [z kchunk, min(K, (z + 1) kchunk)) and, with SPLIT, writes its raw partial tile to
 // a.ws[z][M][N] for gemm_reduce_kernel.  Row tiles past the last are clamped to it (their
@@ -72,12 +96,26 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_kernel(GemmArgs a, int kchu
     uint32_t off[TR];
 #pragma unroll
     for (int i = 0; i < TR; ++i) off[i] = (static_cast<uint32_t>(min(tile0 + i, tiles - 1)) * (a.K / 32) + kb / 32) * (kTileElems * 2) + lane * 16;
-    f32x4 acc[TR][TC];
+    GemmAcc<T> sums;
     gemm_compute<T>(
-        ring, ars, [&](int i, int s) { return GemmOff{off[i], static_cast<uint32_t>(s) * (kTileElems * 2)}; }, nst, wc, lane, acc);
+        ring, ars, [&](int i, int s) { return GemmOff{off[i], static_cast<uint32_t>(s) * (kTileElems * 2)}; }, nst, wc, lane, sums);
+    const int n0 = bx * T::BN + wc * TC * 16;  // the wave's first column
+    const auto dot = [&](int m, int n) {
+        return gemm_dot(static_cast<const typename T::W*>(a.w) + static_cast<size_t>(n0 + n) * a.K + kb, nst * 32,
+                        [&](int k) { return split_value(a.a + split_off(m, kb + k, a.K)); });
+    };
+    const bool suspect = sums.suspect();
+    if constexpr (SPLIT || (EPI != kGemmGelu && EPI != kGemmSwiglu)) {
+        if (__builtin_expect(suspect, 0)) {
+            gemm_refine<T>(lds, a.M, tile0, wave, lane, sums, dot, [&](int m, int n, float v) { gemm_store_one<EPI, SPLIT>(a, bz, m, n0 + n, v); });
+            return;
+        }
+    }
+    f32x4 acc[TR][TC];
+    sums.sum(acc);
 
     // acc[i][c][r]: row 16 (tile0 + i) + rq + r, column col0 + 16 c
-    const int col0 = bx * T::BN + wc * TC * 16 + (lane & 15);
+    const int col0 = n0 + (lane & 15);
     const int rq = 4 * (lane >> 4);
     if constexpr (SPLIT) {
         gemm_store_partial<T>(a.ws + static_cast<size_t>(bz) * a.M * a.N, a.M, a.N, tile0, col0, lane, acc);
@@ -86,13 +124,17 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_kernel(GemmArgs a, int kchu
 #pragma unroll
         for (int c = 0; c < TC; ++c) bias[c] = a.bias[col0 + 16 * c];
         if constexpr (EPI == kGemmGelu) {
-            gemm_store_split<T, false>(lds, wave, lane, a.c_split, a.M, a.N, 0, tile0, bx * T::BN + wc * TC * 16,
-                                       [&](int i, int c, int r) { return gelu_f(acc[i][c][r] + bias[c]); });
+            gemm_store_split<T, false>(
+                lds, wave, lane, a.c_split, a.M, a.N, 0, tile0, n0, [&](int i, int c, int r) { return gelu_f(acc[i][c][r] + bias[c]); }, suspect,
+                [&](int m, int n) { return gelu_f(dot(m, n) + a.bias[n0 + n]); });
         } else {  // columns col and col ^ 1 sit in lanes l and l ^ 1, on the same rows
-            gemm_store_split<T, true>(lds, wave, lane, a.c_split, a.M, a.N / 2, 0, tile0, (bx * T::BN + wc * TC * 16) / 2, [&](int i, int c, int r) {
-                const float v = acc[i][c][r] + bias[c];
-                return swiglu_f(v, __shfl_xor(v, 1, 64));
-            });
+            gemm_store_split<T, true>(
+                lds, wave, lane, a.c_split, a.M, a.N / 2, 0, tile0, n0 / 2,
+                [&](int i, int c, int r) {
+                    const float v = acc[i][c][r] + bias[c];
+                    return swiglu_f(v, __shfl_xor(v, 1, 64));
+                },
+                suspect, [&](int m, int n) { return swiglu_f(dot(m, 2 * n) + a.bias[n0 + 2 * n], dot(m, 2 * n + 1) + a.bias[n0 + 2 * n + 1]); });
         }
     } else {
         float bias[TC];
@@ -150,31 +192,11 @@ __global__ __launch_bounds__(64 * kSmallWaves) void gemm_small_kernel(GemmArgs a
     const uint32_t row_bytes = a.K / 32 * (kTileElems * 2);
     float sum[2];
     gemm_small<WT, RT>(lds, static_cast<const WT*>(a.w) + static_cast<size_t>(blockIdx.x) * 16 * a.K + kb, a.K, nst,
-                       gemm_rsrc(a.a, static_cast<uint32_t>(split_elems(a.M, a.K) * 2)), kb / 32 * (kTileElems * 2), row_bytes, (a.M + 15) / 16, sum);
-    const int col = blockIdx.x * 16 + (threadIdx.x & 15);
-    const float bias = SPLIT ? 0.0f : a.bias[col];
+                       gemm_rsrc(a.a, static_cast<uint32_t>(split_elems(a.M, a.K) * 2)), kb / 32 * (kTileElems * 2), row_bytes, a.M,
+                       [&](int m, int k) { return split_value(a.a + split_off(m, kb + k, a.K)); }, sum);
 #pragma unroll
-    for (int q = 0; q < (RT > 2 ? 2 : 1); ++q) {
-        const int row = (threadIdx.x >> 4) + 32 * q;
-        const bool live = row < a.M;
-        const float v = sum[q] + bias;
-        if constexpr (SPLIT) {
-            if (live) a.ws[(static_cast<size_t>(blockIdx.y) * a.M + row) * a.N + col] = sum[q];
-        } else if constexpr (EPI == kGemmGelu) {
-            if (live) split_store(a.c_split, split_off(row, col, a.N), gelu_f(v));
-        } else if constexpr (EPI == kGemmSwiglu) {
-            const float u = __shfl_xor(v, 1, 64);
-            if (live && !(col & 1)) split_store(a.c_split, split_off(row, col / 2, a.N / 2), swiglu_f(v, u));
-        } else if constexpr (EPI == kGemmQkv) {
-            if (!live) continue;
-            if (col < kWidth) a.c[static_cast<size_t>(row) * kWidth + col] = v;
-            else a.kv[kv_off(a, col - kWidth, a.row_slot[row], a.row_pos[row])] = v;
-        } else {
-            if (!live) continue;
-            float* p = a.c + static_cast<size_t>(row) * a.N + col;
-            *p = EPI == kGemmResid ? *p + v : v;
-        }
-    }
+    for (int q = 0; q < (RT > 2 ? 2 : 1); ++q)
+        gemm_store_one<EPI, SPLIT>(a, blockIdx.y, (threadIdx.x >> 4) + 32 * q, blockIdx.x * 16 + (threadIdx.x & 15), sum[q]);
 }
 
 // Partial 0 + partial 1 + ... of four consecutive elements from e on, in split order.  Every
@@ -295,8 +317,8 @@ __global__ __launch_bounds__(256) void gemm_reduce_ln_kernel(GemmArgs a) {
 // each run the slot's keys 0 .. max position, in a state of its own (a row of another slot has
 // weight 0 there, and 0 times a NaN or an infinite V is NaN), of which the run's rows are
 // stored.  Later rows have more keys: they start first.  Three waves per SIMD: left to the
-// compiler, the state in a loop takes registers for two (571 rows 30.1 us, with three 26.5; 155
-// rows 8.2 and 8.6; one state over all runs 27.7 and 8.35).
+// compiler, the state in a loop takes registers for two (571 rows 30.1 us, with three 27.0; 155
+// rows 8.2 and 8.8; one state over all runs 28.1 and 8.2).
 __global__ __launch_bounds__(64 * kAttnWaves, 3) void causal_attention_kernel(CausalArgs a) {
     __shared__ AttnLds<kHeadDim> lds;
     const int m0 = (gridDim.x - 1 - blockIdx.x) * kAttnTile, h = blockIdx.y;
@@ -327,7 +349,7 @@ __global__ __launch_bounds__(64 * kAttnWaves, 3) void causal_attention_kernel(Ca
         const int pos = qr >= r0 && qr < r1 ? pos_q : -1;
         for (int c0 = wave * kAttnKeys; c0 < kn; c0 += kAttnWaves * kAttnKeys)
             attn_chunk<kHeadDim>(st, q, kb, kb + a.kv_v_off, c0, kn, pos, 0.125f, lane);
-        if (r1 == nq) break;
+        if (__builtin_expect(r1 == nq, 1)) break;
         finish(r1);
         __syncthreads();  // the merge has read its LDS
         st = AttnState<kHeadDim>();

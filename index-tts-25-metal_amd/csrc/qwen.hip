@@ -791,6 +791,7 @@ struct Engine {
         Qp.alloc(static_cast<size_t>(cap) * kQ);
         ATT.alloc(split_elems(cap, kQ));
         FF.alloc(split_elems(cap, kF));
+        for (auto* b : {&Xn, &ATT, &FF}) QWEN_CHECK(hipMemsetAsync(b->p, 0, b->n * 2, stream));  // padding rows: finite, whatever the memory held
         if (!ws.p) ws.alloc(kGemmWsFloats);
         pcap = cap;
     }

@@ -24,6 +24,7 @@
 #include <string>
 #include <thread>
 #include <tuple>
+#include <utility>
 #include <unordered_map>
 #include <vector>
 
@@ -754,10 +755,12 @@ struct Engine {
         uint32_t M = 0;
         for (auto r : rows) M += r;
         px.ensure(static_cast<size_t>(M) * kWidth);
-        pxn.ensure(split_elems(M, kWidth));
         pq.ensure(static_cast<size_t>(M) * kWidth);
-        patt.ensure(split_elems(M, kWidth));
-        pff.ensure(split_elems(M, kFfn));
+        for (auto [b, k] : {std::pair{&pxn, kWidth}, std::pair{&patt, kWidth}, std::pair{&pff, kFfn}}) {
+            if (b->n >= split_elems(M, k)) continue;
+            b->alloc(split_elems(M, k));
+            HIP_CHECK(hipMemsetAsync(b->p, 0, b->n * 2, stream));  // padding rows: finite, whatever the memory held
+        }
         row_slot.ensure(M);
         row_pos.ensure(M);
         last_rows.ensure(kMaxBatch);
