@@ -1004,7 +1004,8 @@ struct Engine {
         QWEN_CHECK(hipStreamSynchronize(stream));
         const QState s = pinned->down;
         *count = std::min(s.count, maximum);
-        QWEN_CHECK(hipMemcpy(out, toks.p, sizeof(uint32_t) * *count, hipMemcpyDeviceToHost));
+        QWEN_CHECK(hipMemcpyAsync(out, toks.p, sizeof(uint32_t) * *count, hipMemcpyDeviceToHost, stream));  // (not on the null stream)
+        QWEN_CHECK(hipStreamSynchronize(stream));
         cached = n + *count - 1;
         submissions += *count;
         if (!s.eos) throw std::runtime_error("Qwen did not reach EOS within 1024 generated tokens");

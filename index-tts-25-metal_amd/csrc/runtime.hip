@@ -267,12 +267,14 @@ struct Engine {
     DevBuf<float> api_out;
     DevBuf<uint32_t> api_tokens;
     uint32_t* pinned = nullptr;  // host pinned staging (flags)
+    static constexpr int kPinnedStepError = 60;  // its entry for the persistent step's error flag
     SeqState* pinned_state = nullptr;
     int splits = 16;
     bool use_graphs = true;  // ITTS_GPT_GRAPHS=0: launch the same kernels eagerly (profilers)
     // Persistent single-sequence step (step.hip): one launch per token for batch-1 decode
     // (bitwise the same logits as the multi-kernel path, which ITTS_GPT_PERSISTENT=0 selects).
     bool step_ok = false;
+    bool step_launched = false;  // persistent steps queued whose error flag has not been
     bool bf16_step_off = false;  // a BF16 persistent step timed out (a GPU shared with others): multi-kernel from then on
     bool step_batch_ok[kStepBatchMax + 1] = {};  // persistent batch step available for this many sequences
     uint32_t beam_slots = 0;                     // slots the beam row-owner table may name (this search's beams)
@@ -555,13 +557,21 @@ struct Engine {
         return s;
     }
 
-    // Whether the persistent step reported a hand-off timeout (cleared); call after a sync.
+    // Hand-off timeouts of the persistent steps launched since the last check: queue_step_error()
+    // copies the flag to the host behind them, and after the stream has been waited for,
+    // take_step_error() says whether it was set (and clears it).  Nothing here touches the null
+    // stream: a blocking copy there waits for every blocking stream of the process, and fails
+    // while another thread captures a graph.
+    void queue_step_error() {
+        pinned[kPinnedStepError] = 0;
+        if (step_launched) HIP_CHECK(hipMemcpyAsync(pinned + kPinnedStepError, step_err.p, sizeof(uint32_t), hipMemcpyDeviceToHost, stream));
+        step_launched = false;
+    }
     bool take_step_error() {
-        if (!step_ok) return false;
-        uint32_t e = 0;
-        HIP_CHECK(hipMemcpy(&e, step_err.p, sizeof(e), hipMemcpyDeviceToHost));
-        if (e) HIP_CHECK(hipMemset(step_err.p, 0, sizeof(uint32_t)));
-        return e != 0;
+        if (!pinned[kPinnedStepError]) return false;
+        pinned[kPinnedStepError] = 0;
+        HIP_CHECK(hipMemsetAsync(step_err.p, 0, sizeof(uint32_t), stream));
+        return true;
     }
     void check_step_error() {
         if (take_step_error()) throw std::runtime_error("GPT decode step: a workgroup hand-off timed out");
@@ -580,6 +590,7 @@ struct Engine {
     }
     // fuse_sampler: the single-sequence step kernel also samples the next token (its tail).
     void launch_persistent(int nseq, bool use_table, bool fuse_sampler = false) {
+        step_launched = true;
         StepArgs s = step_args(0, nseq);
         s.table = use_table ? table.p : nullptr;
         if (fuse_sampler) {
@@ -935,6 +946,7 @@ struct Engine {
         upload_states(1);
         auto run = [&] {
             run_step(1, 1, false, false);
+            queue_step_error();
             HIP_CHECK(hipMemcpyAsync(out_logits, logits.p, kMelVocab * 4, hipMemcpyDeviceToHost, stream));
             HIP_CHECK(hipStreamSynchronize(stream));
         };
@@ -946,8 +958,8 @@ struct Engine {
             }
         } else {
             run();
+            check_step_error();
         }
-        check_step_error();
         cached++;
     }
 
@@ -1025,6 +1037,7 @@ struct Engine {
         HIP_CHECK(hipMemcpyAsync(pinned_state, state.p, nseq * sizeof(SeqState), hipMemcpyDeviceToHost, stream));
         uint32_t* st = pinned + 32;
         HIP_CHECK(hipMemcpyAsync(st, status.p, nseq * 4, hipMemcpyDeviceToHost, stream));
+        queue_step_error();
         HIP_CHECK(hipStreamSynchronize(stream));
         HIP_CHECK(hipEventElapsedTime(&timing.prefill_ms, ev[0], ev[1]));
         HIP_CHECK(hipEventElapsedTime(&timing.decode_ms, ev[1], ev[2]));
@@ -1034,8 +1047,9 @@ struct Engine {
             const SeqState& s = pinned_state[b];
             if (s.error) throw std::runtime_error(sampler_message(st[b]));
             steps = std::max(steps, s.count);
-            HIP_CHECK(hipMemcpy(codes_out + static_cast<size_t>(b) * max_tokens, codes.p + static_cast<size_t>(b) * cap,
-                                s.count * 4, hipMemcpyDeviceToHost));
+            HIP_CHECK(hipMemcpyAsync(codes_out + static_cast<size_t>(b) * max_tokens, codes.p + static_cast<size_t>(b) * cap, s.count * 4,
+                                     hipMemcpyDeviceToHost, stream));
+            HIP_CHECK(hipStreamSynchronize(stream));
             n_codes[b] = s.count;
             stopped[b] = s.stopped ? 1 : 0;
         }
@@ -1289,7 +1303,8 @@ struct Engine {
         HIP_CHECK(hipEventRecord(ev[0], stream));
         for (int i = 0; i < iters; ++i) launch(one_layer ? 0 : i % layers);
         HIP_CHECK(hipEventRecord(ev[1], stream));
-        HIP_CHECK(hipEventSynchronize(ev[1]));
+        queue_step_error();
+        HIP_CHECK(hipStreamSynchronize(stream));
         float ms = 0;
         HIP_CHECK(hipEventElapsedTime(&ms, ev[0], ev[1]));
         *avg_ms = ms / iters;
@@ -1342,6 +1357,8 @@ struct Engine {
             StepArgs a = step_args(0, nseq);
             a.stamps = stamps.p;
             HIP_CHECK(launch_step_serialized(a, nseq, step_grid, step_dev, stream));
+            step_launched = true;
+            queue_step_error();
             HIP_CHECK(hipMemcpyAsync(host.data(), stamps.p, stamps.n * 8, hipMemcpyDeviceToHost, stream));
             HIP_CHECK(hipStreamSynchronize(stream));
             check_step_error();
@@ -1648,6 +1665,7 @@ void Engine::generate_beams(const float* prefix, uint32_t rows, const itts_gen_o
         }
     }
     HIP_CHECK(hipEventRecord(ev[2], stream));
+    queue_step_error();
     HIP_CHECK(hipStreamSynchronize(stream));
     HIP_CHECK(hipEventElapsedTime(&timing.prefill_ms, ev[0], ev[1]));
     HIP_CHECK(hipEventElapsedTime(&timing.decode_ms, ev[1], ev[2]));
