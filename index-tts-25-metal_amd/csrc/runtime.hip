@@ -102,53 +102,81 @@ struct Snapshot {
 // is skipped (its marker packets cost about 3 us per token).  A decoder that registers as
 // the second one drains the device first, so no unchained grid is still running when
 // chained launches begin; a decoder drains its own stream before it unregisters.
-// The chain is process-wide and never freed.
+// A BF16 decoder's step() launches one such grid and waits for it.  It does not join the chain
+// (FP32 decoders would pay for the markers): it takes the persistent kernel only while no other
+// grid of the device is queued, and the multi-kernel path, which needs no free CUs, otherwise.
+// An FP32 launch that comes while it runs waits for it on the device.
+// The state is process-wide and never freed; the mutex is held for the enqueue only.
+struct StepDevice {
+    int users = 0;                // FP32 decoders that launch persistent grids
+    int pending = 0;              // of them, those with grids queued since they last waited for their stream
+    hipEvent_t last = nullptr;    // recorded after the latest chained launch
+    hipStream_t solo = nullptr;   // the stream of a BF16 decoder's step in flight
+    hipEvent_t solo_done = nullptr;
+};
 std::mutex g_step_mu;
-std::unordered_map<int, int> g_step_users;          // device -> decoders that launch persistent grids
-std::unordered_map<int, hipEvent_t> g_step_last;    // device -> recorded after its latest chained launch
+std::unordered_map<int, StepDevice> g_step;  // by device
 
 void register_step_user(int dev) {
     int users = 0;
     {
         std::lock_guard<std::mutex> lock(g_step_mu);
-        users = ++g_step_users[dev];
+        users = ++g_step[dev].users;
     }
     if (users == 2) HIP_CHECK(hipDeviceSynchronize());
 }
 void unregister_step_user(int dev) {
     std::lock_guard<std::mutex> lock(g_step_mu);
-    --g_step_users[dev];
+    --g_step[dev].users;
 }
 
-// One persistent step that is waited for before the lock is released (a BF16 decoder's step()).
-// Such decoders are not counted as users: with the lock held no other decoder can launch a
-// grid, and those launched before are drained first, so the other decoders keep launching
-// unchained.
-template <class F>
-void exclusive_step(int dev, F run) {
+// `pending`: whether this decoder is counted in StepDevice::pending; step_waited() ends that.
+hipError_t launch_step_serialized(const StepArgs& a, int nseq, int grid, int dev, hipStream_t s, bool& pending) {
     std::lock_guard<std::mutex> lock(g_step_mu);
-    auto it = g_step_users.find(dev);
-    if (it != g_step_users.end() && it->second > 0) HIP_CHECK(hipDeviceSynchronize());
-    run();
-}
-
-hipError_t launch_step_serialized(const StepArgs& a, int nseq, int grid, int dev, hipStream_t s) {
-    std::lock_guard<std::mutex> lock(g_step_mu);
-    if (g_step_users[dev] <= 1) return nseq == 1 ? launch_step(a, grid, false, s) : launch_step_batch(a, nseq, grid, s);
-    auto& last = g_step_last;
-    auto it = last.find(dev);
-    if (it == last.end()) {
-        hipEvent_t e = nullptr;
-        const hipError_t err = hipEventCreateWithFlags(&e, hipEventDisableTiming);
+    StepDevice& d = g_step[dev];
+    if (!pending) {
+        pending = true;
+        ++d.pending;
+    }
+    auto after = [&](hipEvent_t& e) { return e ? hipSuccess : hipEventCreateWithFlags(&e, hipEventDisableTiming); };
+    if (d.solo) {
+        hipError_t err = after(d.solo_done);
+        if (err == hipSuccess) err = hipEventRecord(d.solo_done, d.solo);
+        if (err == hipSuccess) err = hipStreamWaitEvent(s, d.solo_done, 0);
         if (err != hipSuccess) return err;
-        it = last.emplace(dev, e).first;
-    } else {
-        const hipError_t err = hipStreamWaitEvent(s, it->second, 0);
+    }
+    const bool chained = d.users > 1;
+    if (chained) {
+        const bool first = !d.last;
+        hipError_t err = after(d.last);
+        if (err == hipSuccess && !first) err = hipStreamWaitEvent(s, d.last, 0);
         if (err != hipSuccess) return err;
     }
     const hipError_t err = nseq == 1 ? launch_step(a, grid, false, s) : launch_step_batch(a, nseq, grid, s);
-    if (err != hipSuccess) return err;
-    return hipEventRecord(it->second, s);
+    return err == hipSuccess && chained ? hipEventRecord(d.last, s) : err;
+}
+// After a decoder has waited for its stream.
+void step_waited(int dev, bool& pending) {
+    if (!pending) return;
+    std::lock_guard<std::mutex> lock(g_step_mu);
+    --g_step[dev].pending;
+    pending = false;
+}
+
+// Launches a BF16 decoder's step if no other persistent grid of the device is queued; says whether
+// it did.  The grid counts as in flight until step_solo_waited().
+template <class F>
+bool launch_step_solo(int dev, hipStream_t s, F launch) {
+    std::lock_guard<std::mutex> lock(g_step_mu);
+    StepDevice& d = g_step[dev];
+    if (d.solo || d.pending) return false;
+    launch();
+    d.solo = s;
+    return true;
+}
+void step_solo_waited(int dev) {
+    std::lock_guard<std::mutex> lock(g_step_mu);
+    g_step[dev].solo = nullptr;
 }
 
 // ---------------------------------------------------------------- scratch of generate_noalloc
@@ -274,6 +302,8 @@ struct Engine {
     // Persistent single-sequence step (step.hip): one launch per token for batch-1 decode
     // (bitwise the same logits as the multi-kernel path, which ITTS_GPT_PERSISTENT=0 selects).
     bool step_ok = false;
+    bool step_pending = false;   // counted in StepDevice::pending
+    bool step_solo = false;      // this (BF16) decoder's step is StepDevice::solo
     bool step_launched = false;  // persistent steps queued whose error flag has not been
     bool bf16_step_off = false;  // a BF16 persistent step timed out (a GPU shared with others): multi-kernel from then on
     bool step_batch_ok[kStepBatchMax + 1] = {};  // persistent batch step available for this many sequences
@@ -304,7 +334,7 @@ struct Engine {
         // Queued work may still write this handle's buffers (a beam search that raised with
         // later steps in flight copies into the pinned ring), and no persistent grid of this
         // decoder may outlive its registration: drain the stream before anything is freed.
-        if (stream) (void)hipStreamSynchronize(stream);
+        wait_stream(false);
         if (step_ok && !bf16) unregister_step_user(step_dev);
         for (auto& kvp : graphs) (void)hipGraphExecDestroy(kvp.second);
         for (auto& e : ev)
@@ -337,7 +367,7 @@ struct Engine {
         probs.alloc((B + 1) * kMelVocab);
         api_out.alloc(kMelVocab);
         api_tokens.alloc(1 << 16);
-        HIP_CHECK(hipStreamSynchronize(stream));
+        wait_stream();
     }
 
     void create(const itts_tensor* tensors, int32_t count, const itts_gpt_config* cfg) {
@@ -395,7 +425,7 @@ struct Engine {
             const float* src = check(name, {in, out});
             upload(src, static_cast<size_t>(in) * out, staging.p);
             HIP_CHECK(launch_transpose(staging.p, w_ptr(off), in, out, bf16, stream));
-            HIP_CHECK(hipStreamSynchronize(stream));  // staging is reused
+            wait_stream();  // staging is reused
         };
         params.alloc(static_cast<size_t>(layers) * kParLayer);
         std::vector<float> par(static_cast<size_t>(layers) * kParLayer);
@@ -428,7 +458,7 @@ struct Engine {
         off_head = off;
         upload(check("gpt.mel_head.weight", {kMelVocab, kWidth}), static_cast<size_t>(kMelVocab) * kWidth, staging.p);
         HIP_CHECK(launch_convert(staging.p, w_ptr(off_head), static_cast<size_t>(kMelVocab) * kWidth, bf16, stream));
-        HIP_CHECK(hipStreamSynchronize(stream));
+        wait_stream();
         upload(par.data(), par.size(), params.p);
         std::vector<float> hp(kHeadPar);
         std::memcpy(&hp[kHeadLnfW], check("gpt.gpt.ln_f.weight", {kWidth}), kWidth * 4);
@@ -480,7 +510,7 @@ struct Engine {
         int dev = 0;
         HIP_CHECK(hipGetDevice(&dev));
         scratch_dev = scratch_entry(dev);
-        HIP_CHECK(hipStreamSynchronize(stream));
+        wait_stream();
     }
 
     // The persistent step runs when one 512-thread workgroup fits per CU (the grid is one
@@ -557,6 +587,14 @@ struct Engine {
         return s;
     }
 
+    // Waits for the stream; the persistent grids queued on it are then over.
+    void wait_stream(bool check = true) {
+        const hipError_t e = stream ? hipStreamSynchronize(stream) : hipSuccess;
+        step_waited(step_dev, step_pending);
+        if (step_solo) step_solo_waited(step_dev);
+        step_solo = false;
+        if (check) HIP_CHECK(e);
+    }
     // Hand-off timeouts of the persistent steps launched since the last check: queue_step_error()
     // copies the flag to the host behind them, and after the stream has been waited for,
     // take_step_error() says whether it was set (and clears it).  Nothing here touches the null
@@ -588,17 +626,19 @@ struct Engine {
         if (use_table) return nseq >= 2 && step_batch_ok[nseq] && beam_slots <= static_cast<uint32_t>(kStepBatchMax);
         return nseq == 1 || step_batch_ok[nseq];
     }
-    // fuse_sampler: the single-sequence step kernel also samples the next token (its tail).
-    void launch_persistent(int nseq, bool use_table, bool fuse_sampler = false) {
-        step_launched = true;
+    // fuse_sampler: the single-sequence step kernel also samples the next token (its tail).  False
+    // (BF16 only): another persistent grid is queued on the device, nothing was launched.
+    bool launch_persistent(int nseq, bool use_table, bool fuse_sampler = false) {
         StepArgs s = step_args(0, nseq);
         s.table = use_table ? table.p : nullptr;
         if (fuse_sampler) {
             s.tail = step_tail.p;
             s.sample = sample_base(kModeDecode);
         }
-        if (bf16) HIP_CHECK(launch_step(s, step_grid, true, stream));  // inside exclusive_step
-        else HIP_CHECK(launch_step_serialized(s, nseq, step_grid, step_dev, stream));
+        if (bf16) step_solo = launch_step_solo(step_dev, stream, [&] { HIP_CHECK(launch_step(s, step_grid, true, stream)); });
+        else HIP_CHECK(launch_step_serialized(s, nseq, step_grid, step_dev, stream, step_pending));
+        step_launched |= !bf16 || step_solo;
+        return !bf16 || step_solo;
     }
 
     // ---------------------------------------------------------------- forward pieces
@@ -717,10 +757,9 @@ struct Engine {
 
     // Runs one step (forward [+ sampler]) as a replay of its captured graph, or eagerly.
     void run_step(int nseq, int nb, bool sampler, bool use_table) {
-        if (persistent(nseq, use_table, sampler)) {
+        const bool fuse = sampler && nseq == 1 && fused_sampling;
+        if (persistent(nseq, use_table, sampler) && launch_persistent(nseq, use_table, fuse)) {
             timing.decode_path = ITTS_PATH_STEP;
-            const bool fuse = sampler && nseq == 1 && fused_sampling;
-            launch_persistent(nseq, use_table, fuse);
             if (sampler && !fuse) HIP_CHECK(launch_sampler(sample_base(kModeDecode), nseq, stream));
             return;
         }
@@ -801,7 +840,7 @@ struct Engine {
             HIP_CHECK(hipMemcpyAsync(row_pos.p, pos.data(), M * 4, hipMemcpyHostToDevice, stream));
             HIP_CHECK(hipMemcpyAsync(last_rows.p, last.data(), kMaxBatch * 4, hipMemcpyHostToDevice, stream));
             // Host vectors above must outlive the async copies.
-            HIP_CHECK(hipStreamSynchronize(stream));
+            wait_stream();
         }
         enqueue_prefill_layers(PrefillBufs{px.p, pq.p, pxn.p, patt.p, pff.p, row_slot.p, row_pos.p, last_rows.p, pws.p}, nseq, M);
     }
@@ -928,7 +967,7 @@ struct Engine {
         enqueue_prefill({prefix}, {rows});
         HIP_CHECK(hipEventRecord(ev[1], stream));
         HIP_CHECK(hipMemcpyAsync(out_logits, logits.p, kMelVocab * 4, hipMemcpyDeviceToHost, stream));
-        HIP_CHECK(hipStreamSynchronize(stream));
+        wait_stream();
         HIP_CHECK(hipEventElapsedTime(&timing.prefill_ms, ev[0], ev[1]));
         cached = rows;
     }
@@ -944,22 +983,21 @@ struct Engine {
         s.position = position;
         pinned_state[0] = s;
         upload_states(1);
-        auto run = [&] {
+        struct Wait {  // on every exit, errors included: a BF16 grid left in flight would keep the others off
+            Engine& e;
+            ~Wait() {
+                if (e.step_solo) e.wait_stream(false);
+            }
+        } wait{*this};
+        for (bool again = true; again;) {
             run_step(1, 1, false, false);
             queue_step_error();
             HIP_CHECK(hipMemcpyAsync(out_logits, logits.p, kMelVocab * 4, hipMemcpyDeviceToHost, stream));
-            HIP_CHECK(hipStreamSynchronize(stream));
-        };
-        if (bf16 && persistent(1, false, false)) {
-            exclusive_step(step_dev, run);
-            if (take_step_error()) {  // the multi-kernel path needs no free CUs: it writes the same cache row and logits
-                bf16_step_off = true;
-                run();
-            }
-        } else {
-            run();
-            check_step_error();
+            wait_stream();
+            again = bf16 && take_step_error();  // repeated on the multi-kernel path, which needs no free CUs: it writes the same cache row and logits
+            bf16_step_off |= again;
         }
+        check_step_error();
         cached++;
     }
 
@@ -1038,7 +1076,7 @@ struct Engine {
         uint32_t* st = pinned + 32;
         HIP_CHECK(hipMemcpyAsync(st, status.p, nseq * 4, hipMemcpyDeviceToHost, stream));
         queue_step_error();
-        HIP_CHECK(hipStreamSynchronize(stream));
+        wait_stream();
         HIP_CHECK(hipEventElapsedTime(&timing.prefill_ms, ev[0], ev[1]));
         HIP_CHECK(hipEventElapsedTime(&timing.decode_ms, ev[1], ev[2]));
         check_step_error();
@@ -1049,7 +1087,7 @@ struct Engine {
             steps = std::max(steps, s.count);
             HIP_CHECK(hipMemcpyAsync(codes_out + static_cast<size_t>(b) * max_tokens, codes.p + static_cast<size_t>(b) * cap, s.count * 4,
                                      hipMemcpyDeviceToHost, stream));
-            HIP_CHECK(hipStreamSynchronize(stream));
+            wait_stream();
             n_codes[b] = s.count;
             stopped[b] = s.stopped ? 1 : 0;
         }
@@ -1077,9 +1115,9 @@ struct Engine {
         std::lock_guard<std::mutex> lock(*scratch_dev->lock);
         struct Drain {  // destroyed before `lock`: on every exit, errors included, the work this
                         // call queued on the shared scratch has finished before the lock is released
-            hipStream_t s;
-            ~Drain() { (void)hipStreamSynchronize(s); }
-        } drain{stream};
+            Engine& e;
+            ~Drain() { e.wait_stream(false); }
+        } drain{*this};
         uint8_t* base = scratch_dev->ptr;
         const PrefillBufs b{reinterpret_cast<float*>(base + kScratchOffX),      reinterpret_cast<float*>(base + kScratchOffQ),
                             reinterpret_cast<uint16_t*>(base + kScratchOffXn),  reinterpret_cast<uint16_t*>(base + kScratchOffAtt),
@@ -1138,7 +1176,7 @@ struct Engine {
         uint32_t st = 0;
         HIP_CHECK(hipMemcpyAsync(out, api_out.p, kMelVocab * 4, hipMemcpyDeviceToHost, stream));
         HIP_CHECK(hipMemcpyAsync(&st, status.p + slot, 4, hipMemcpyDeviceToHost, stream));
-        HIP_CHECK(hipStreamSynchronize(stream));
+        wait_stream();
         if (st) throw std::runtime_error(sampler_message(st));
     }
 
@@ -1166,7 +1204,7 @@ struct Engine {
         HIP_CHECK(hipMemcpyAsync(tokens, api_tokens.p, draws * 4, hipMemcpyDeviceToHost, stream));
         HIP_CHECK(hipMemcpyAsync(&st, status.p + slot, 4, hipMemcpyDeviceToHost, stream));
         HIP_CHECK(hipMemcpyAsync(pinned_state + slot, state.p + slot, sizeof(SeqState), hipMemcpyDeviceToHost, stream));
-        HIP_CHECK(hipStreamSynchronize(stream));
+        wait_stream();
         if (st) throw std::runtime_error(sampler_message(st));
         *rng = pinned_state[slot].rng;
     }
@@ -1180,7 +1218,7 @@ struct Engine {
         s->kv.alloc(blocks * cached * kHeadDim);
         HIP_CHECK(hipMemcpy2DAsync(s->kv.p, static_cast<size_t>(cached) * kHeadDim * 4, kv.p, static_cast<size_t>(cap) * kHeadDim * 4,
                                    static_cast<size_t>(cached) * kHeadDim * 4, blocks, hipMemcpyDeviceToDevice, stream));
-        HIP_CHECK(hipStreamSynchronize(stream));
+        wait_stream();
         return s.release();
     }
     void restore(const Snapshot& s) {
@@ -1188,7 +1226,7 @@ struct Engine {
         const size_t blocks = static_cast<size_t>(layers) * 2 * kHeads;
         HIP_CHECK(hipMemcpy2DAsync(kv.p, static_cast<size_t>(cap) * kHeadDim * 4, s.kv.p, static_cast<size_t>(s.tokens) * kHeadDim * 4,
                                    static_cast<size_t>(s.tokens) * kHeadDim * 4, blocks, hipMemcpyDeviceToDevice, stream));
-        HIP_CHECK(hipStreamSynchronize(stream));
+        wait_stream();
         cached = s.tokens;
     }
 
@@ -1224,12 +1262,12 @@ struct Engine {
             HIP_CHECK(hipMemcpyAsync(em.p, emotion, kWidth * 4, hipMemcpyHostToDevice, stream));
             HIP_CHECK(hipMemsetAsync(d.p, 0, 3ull * kWidth * 4, stream));
             HIP_CHECK(launch_speaker_row(spk_w.p, spk_b.p, sp.p, em.p, d.p, stream));
-            HIP_CHECK(hipStreamSynchronize(stream));
+            wait_stream();
         }
         HIP_CHECK(launch_text_rows(text_emb.p, text_pos.p, lang_emb.p, mel_emb.p, mel_pos.p, did.p, static_cast<int>(ids.size()),
                                    language, d.p + static_cast<size_t>(n_cond) * kWidth, stream));
         HIP_CHECK(hipMemcpyAsync(out, d.p, d.n * 4, hipMemcpyDeviceToHost, stream));
-        HIP_CHECK(hipStreamSynchronize(stream));
+        wait_stream();
         *rows = total;
     }
 
@@ -1259,7 +1297,7 @@ struct Engine {
         }
         std::copy(st.begin(), st.end(), pinned_state);
         upload_states(batch);
-        HIP_CHECK(hipStreamSynchronize(stream));
+        wait_stream();
         auto launch = [&](int l) {
             const float* par = params.p + static_cast<size_t>(l) * kParLayer;
             GemvArgs a = gemv_base(batch);
@@ -1304,7 +1342,7 @@ struct Engine {
         for (int i = 0; i < iters; ++i) launch(one_layer ? 0 : i % layers);
         HIP_CHECK(hipEventRecord(ev[1], stream));
         queue_step_error();
-        HIP_CHECK(hipStreamSynchronize(stream));
+        wait_stream();
         float ms = 0;
         HIP_CHECK(hipEventElapsedTime(&ms, ev[0], ev[1]));
         *avg_ms = ms / iters;
@@ -1356,11 +1394,11 @@ struct Engine {
             HIP_CHECK(hipMemsetAsync(stamps.p, 0, stamps.n * 8, stream));
             StepArgs a = step_args(0, nseq);
             a.stamps = stamps.p;
-            HIP_CHECK(launch_step_serialized(a, nseq, step_grid, step_dev, stream));
+            HIP_CHECK(launch_step_serialized(a, nseq, step_grid, step_dev, stream, step_pending));
             step_launched = true;
             queue_step_error();
             HIP_CHECK(hipMemcpyAsync(host.data(), stamps.p, stamps.n * 8, hipMemcpyDeviceToHost, stream));
-            HIP_CHECK(hipStreamSynchronize(stream));
+            wait_stream();
             check_step_error();
             if (it == 0) continue;
             auto T = [&](int l, int k) {
@@ -1450,7 +1488,7 @@ void Engine::generate_segments(const float* cond, uint32_t n_cond, const float* 
         HIP_CHECK(hipMemcpyAsync(em.p, emotion, kWidth * 4, hipMemcpyHostToDevice, stream));
         HIP_CHECK(hipMemsetAsync(seg_cond.p, 0, static_cast<size_t>(n_cond) * kWidth * 4, stream));
         HIP_CHECK(launch_speaker_row(spk_w.p, spk_b.p, sp.p, em.p, seg_cond.p, stream));
-        HIP_CHECK(hipStreamSynchronize(stream));  // sp and em are freed at the end of this block
+        wait_stream();  // sp and em are freed at the end of this block
     }
     // Segments i0 .. i0 + n - 1: their prefixes staged back to back in px.
     auto stage = [&](uint32_t i0, uint32_t n) {
@@ -1474,7 +1512,7 @@ void Engine::generate_segments(const float* cond, uint32_t n_cond, const float* 
             r += rows[i];
             k += tails[i].size();
         }
-        HIP_CHECK(hipStreamSynchronize(stream));  // `flat` is read by the copy above
+        wait_stream();  // `flat` is read by the copy above
     };
     float prefill_ms = 0, decode_ms = 0;
     uint32_t steps = 0;
@@ -1666,7 +1704,7 @@ void Engine::generate_beams(const float* prefix, uint32_t rows, const itts_gen_o
     }
     HIP_CHECK(hipEventRecord(ev[2], stream));
     queue_step_error();
-    HIP_CHECK(hipStreamSynchronize(stream));
+    wait_stream();
     HIP_CHECK(hipEventElapsedTime(&timing.prefill_ms, ev[0], ev[1]));
     HIP_CHECK(hipEventElapsedTime(&timing.decode_ms, ev[1], ev[2]));
     timing.decode_steps = steps;

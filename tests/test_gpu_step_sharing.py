@@ -104,3 +104,71 @@ def test_decode_calls_while_another_thread_captures(itts, small_weights, capture
         got = [f() for f in calls]
     assert all(same_bits(a, b) for a, b in zip(got[0], ref[0])) and got[1:] == ref[1:]
     dec.close()
+
+
+@pytest.mark.parametrize("null", [False, True])
+def test_bf16_step_does_not_wait_for_other_streams(itts, small_weights, held_stream, null):
+    """With an FP32 decoder of the process idle on the device and another stream busy, step() returns
+    while that stream is still busy."""
+    f32 = itts.GptDecoder(small_weights, kv_capacity=256)
+    f32.generate(prefix_of(20), itts.GenerationOptions(seed=1, suppress_stop=True), 4)
+    dec = itts.GptDecoder(small_weights, kv_capacity=256, weight_dtype="bf16")
+    ref = steps(dec, prefix_of(20))
+    done = held_stream(null)
+    got = steps(dec, prefix_of(20))
+    assert not done.is_set(), "step() waited for a stream that is not its own"
+    assert done.wait(10)
+    assert all(same_bits(a, b) for a, b in zip(got, ref))
+    dec.close()
+    f32.close()
+
+
+def test_bf16_steps_beside_other_decoders(itts, small_weights):
+    """Threads of one process, all at once: two BF16 decoders' step(), an FP32 generate() and FP32
+    step() (persistent grids), and a codec decoding new lengths (graph captures).  Every result is
+    what the call gives alone, and a BF16 step alone again takes the persistent kernel."""
+    bf = [itts.GptDecoder(small_weights, kv_capacity=512, weight_dtype="bf16") for _ in range(2)]
+    f32 = [itts.GptDecoder(small_weights, kv_capacity=512) for _ in range(2)]
+    codec = itts.EnhancedCodec(itts.make_synthetic_codec_weights(seed=5))
+    o = itts.GenerationOptions(seed=3, suppress_stop=True)
+    codes = [int(c) for c in np.random.default_rng(1).integers(0, 8192, 60)]
+
+    def bf_steps(i):
+        out = steps(bf[i], prefix_of(30 + i), codes[:24])
+        assert bf[i].last_timing()["decode_path"] in ("step", "multi")
+        return out
+
+    calls = {
+        "bf16 a": lambda: bf_steps(0),
+        "bf16 b": lambda: bf_steps(1),
+        "f32 generate": lambda: f32[0].generate(prefix_of(40), o, 64).codes,
+        "f32 step": lambda: steps(f32[1], prefix_of(41), codes[:24]),
+        "codec": lambda: [codec.decode(codes[:n]) for n in range(10, 26)],
+    }
+    ref = {k: f() for k, f in calls.items()}
+    assert bf[1].last_timing()["decode_path"] == "step"
+    out, errors = {}, []
+
+    def run(k, f):
+        try:
+            out[k] = [f() for _ in range(3)]
+        except Exception as e:  # reported below: a thread's exception is not raised by join()
+            errors.append((k, e))
+
+    threads = [threading.Thread(target=run, args=kf) for kf in calls.items()]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join(60)
+    assert not errors, errors
+    for k, r in ref.items():
+        for got in out[k]:
+            if k == "f32 generate":
+                assert got == r, k
+            else:
+                assert all(same_bits(a, b) for a, b in zip(got, r)), k
+    for d in bf:
+        steps(d, prefix_of(30), codes[:2])
+        assert d.last_timing()["decode_path"] == "step"
+    for d in bf + f32 + [codec]:
+        d.close()
