@@ -541,7 +541,9 @@ struct Engine {
         xch.alloc(kStepExchangeTotal * (batch ? kStepBatchMax : 1));
         HIP_CHECK(hipMemsetAsync(xch.p, 0, xch.n * sizeof(uint64_t), stream));
         step_err.alloc(1);
-        HIP_CHECK(hipMemsetAsync(step_err.p, 0, sizeof(uint32_t), stream));
+        // ITTS_GPT_STEP_TIMEOUT_ONCE=1 (tests): the flag starts set, so the first step counts as timed out
+        const char* once = std::getenv("ITTS_GPT_STEP_TIMEOUT_ONCE");
+        HIP_CHECK(hipMemsetAsync(step_err.p, once && std::strcmp(once, "1") == 0 ? 1 : 0, sizeof(uint32_t), stream));
         step_tail.alloc(1);
         HIP_CHECK(hipMemsetAsync(step_tail.p, 0, sizeof(uint32_t), stream));
         const char* fs = std::getenv("ITTS_GPT_FUSED_SAMPLER");

@@ -1,6 +1,7 @@
 """Decode calls beside other work of the process (MI355X): they wait for nothing but their own
 stream, and fail for nothing that other threads do."""
 import ctypes as C
+import os
 import threading
 import time
 
@@ -12,6 +13,23 @@ from conftest import same_bits
 pytestmark = pytest.mark.gpu
 
 CODES = (17, 4000, 8191, 0, 300, 5)
+
+
+@pytest.fixture
+def env():
+    """Sets environment variables for decoders made in the test."""
+    old = {}
+
+    def put(name, value):
+        old.setdefault(name, os.environ.get(name))
+        os.environ[name] = value
+
+    yield put
+    for n, v in old.items():
+        if v is None:
+            os.environ.pop(n, None)
+        else:
+            os.environ[n] = v
 
 
 def prefix_of(rows):
@@ -171,4 +189,35 @@ def test_bf16_steps_beside_other_decoders(itts, small_weights):
         steps(d, prefix_of(30), codes[:2])
         assert d.last_timing()["decode_path"] == "step"
     for d in bf + f32 + [codec]:
+        d.close()
+
+
+def test_bf16_step_repeated_on_the_multikernel_path_after_a_timeout(itts, small_weights, env):
+    """ITTS_GPT_STEP_TIMEOUT_ONCE=1: the decoder's first persistent step is reported as a hand-off
+    that timed out.  A BF16 step() is then repeated on the multi-kernel path: the same logits, one
+    row cached, and the later steps stay on that path.  An FP32 step() raises, caches nothing, and
+    the next one works."""
+    env("ITTS_GPT_STEP_TIMEOUT_ONCE", "0")
+    plain = itts.GptDecoder(small_weights, kv_capacity=256, weight_dtype="bf16")
+    plain32 = itts.GptDecoder(small_weights, kv_capacity=256)
+    env("ITTS_GPT_STEP_TIMEOUT_ONCE", "1")
+    dec = itts.GptDecoder(small_weights, kv_capacity=256, weight_dtype="bf16")
+    dec32 = itts.GptDecoder(small_weights, kv_capacity=256)
+    prefix = prefix_of(21)
+    ref, got = steps(plain, prefix), [dec.prefill(prefix)]
+    for i, c in enumerate(CODES):
+        got.append(dec.step(c, i + 2))
+        assert dec.last_timing()["decode_path"] == "multi"
+        assert dec.cached_tokens() == 22 + i
+    assert plain.last_timing()["decode_path"] == "step"
+    assert all(same_bits(a, b) for a, b in zip(got, ref))
+    dec32.prefill(prefix)
+    with pytest.raises(itts.GptRuntimeError, match="hand-off timed out"):
+        dec32.step(CODES[0], 2)
+    assert dec32.cached_tokens() == 21
+    plain32.prefill(prefix)
+    for i, c in enumerate(CODES):
+        assert same_bits(dec32.step(c, i + 2), plain32.step(c, i + 2))
+        assert dec32.last_timing()["decode_path"] == "step"
+    for d in (dec, dec32, plain, plain32):
         d.close()
