@@ -41,9 +41,10 @@ __device__ __forceinline__ void split_mfma(const SplitFrag& a, const SplitFrag& 
 constexpr int kAttnWaves = 4, kAttnTile = 16, kAttnKeys = 32;
 
 template <int HD>
-struct AttnLds {
+struct alignas(16) AttnLds {  // rows of o are written 16 bytes at a time
     float o[kAttnWaves][kAttnTile][HD + 4];
     float m[kAttnWaves][kAttnTile], l[kAttnWaves][kAttnTile];
+    static_assert((HD + 4) % 4 == 0, "16-byte rows");
 };
 
 // One wave's state over the chunks it has seen.
