@@ -581,7 +581,7 @@ __device__ __forceinline__ void gemm_small(GemmSmallLds<RT>& lds, const WT* w, i
 }
 // Its cut, or splits 0 where the 64-column tiles are faster.  Measured on MI355X in both kernels
 // (one GEMM with what follows it, weights from HBM, us, 64-column tiles -> this):
-//   at most one workgroup per CU and 1280 k each: 3840 x 1280 at 20 rows 11.0 -> 8.1, at 60 rows
+//   at most one workgroup per CU (256) and 1280 k each: 3840 x 1280 at 20 rows 11.0 -> 8.1, at 60 rows
 //   13.1 -> 11.4; 1280 x 1280 at 32 / 60 rows 8.1 -> 6.9 / 9.5 -> 8.2; 1024 x 3072 at 48 rows 10.5 -> 9.8;
 //   5120 x 1280, 320 workgroups: 8 rows 12.9 -> 11.0, but 20 rows 13.5 -> 15.3 (some CUs have two,
 //   and every one reads the whole operand); 1280 x 5120 at 20 rows 12.7 -> 17.8;
@@ -590,15 +590,7 @@ __device__ __forceinline__ void gemm_small(GemmSmallLds<RT>& lds, const WT* w, i
 struct GemmSmallPlan {
     int splits, kchunk;
 };
-inline GemmSmallPlan gemm_small_plan(int M, int N, int K, int max_splits, bool bf16) {
-    const int rt = (M + 15) / 16, tiles = N / 16;
-    if (rt > (bf16 ? 2 : 4)) return {0, 0};
-    const int want = std::max(1, std::min(max_splits, 256 / tiles));
-    const int units = (K + kSmallK - 1) / kSmallK, per = (units + want - 1) / want;
-    const GemmSmallPlan p{(units + per - 1) / per, per * kSmallK};
-    if (p.kchunk > 1280 || tiles * p.splits > (rt == 1 ? 400 : 256)) return {0, 0};
-    return p;
-}
+GemmSmallPlan gemm_small_plan(int M, int N, int K, int max_splits, bool bf16);
 
 // How one GEMM is cut: a tile shape, its row blocks, and K cut into `splits` ranges of kchunk (a
 // multiple of kGemmK).  `reduce`: the splits are added by a kernel of their own (else by one that

@@ -409,6 +409,16 @@ constexpr GemmCost kGemmCost[2][kTiles] = {
     }};
 }  // namespace
 
+GemmSmallPlan gemm_small_plan(int M, int N, int K, int max_splits, bool bf16) {
+    const int rt = ceil_div(M, 16), tiles = N / 16, cus = device_cus();
+    if (rt > (bf16 ? 2 : 4)) return {0, 0};
+    const int want = std::max(1, std::min(max_splits, cus / tiles));
+    const int units = ceil_div(K, kSmallK), per = ceil_div(units, want);
+    const GemmSmallPlan p{ceil_div(units, per), per * kSmallK};
+    if (p.kchunk > 1280 || tiles * p.splits > (rt == 1 ? cus + cus * 9 / 16 : cus)) return {0, 0};  // (one row tile: 400 of 256 CUs)
+    return p;
+}
+
 GemmPlan gemm_plan(int M, int N, int K, int max_splits, bool bf16, bool reduce) {
     const int rtot = ceil_div(M, 16), cus = device_cus();
     const double mn = static_cast<double>(M) * N;
@@ -444,14 +454,27 @@ void launch_gemm_tile(const GemmArgs& a, const GemmPlan& p, hipStream_t s) {
 
 namespace {
 
+// Row tiles that gemm_small_kernel is built for: gemm_small_plan's four (BF16 weights two), and one for
+// the GELU and SiLU epilogues, whose 5120 and 6144 columns are more than a workgroup per CU.
+template <int EPI>
+constexpr int gemm_small_tiles(bool bf16) {
+    return EPI == kGemmGelu || EPI == kGemmSwiglu ? 1 : bf16 ? 2 : 4;
+}
 template <typename WT, int EPI, bool SPLIT>
 void launch_gemm_small(const GemmArgs& a, const GemmSmallPlan& p, hipStream_t s) {
     const dim3 grid(a.N / 16, p.splits), block(64 * kSmallWaves);
+    constexpr int RTS = gemm_small_tiles<EPI>(sizeof(WT) == 2);
     switch (ceil_div(a.M, 16)) {
         case 1: hipLaunchKernelGGL((gemm_small_kernel<WT, 1, EPI, SPLIT>), grid, block, 0, s, a, p.kchunk); break;
-        case 2: hipLaunchKernelGGL((gemm_small_kernel<WT, 2, EPI, SPLIT>), grid, block, 0, s, a, p.kchunk); break;
-        case 3: hipLaunchKernelGGL((gemm_small_kernel<WT, 3, EPI, SPLIT>), grid, block, 0, s, a, p.kchunk); break;
-        default: hipLaunchKernelGGL((gemm_small_kernel<WT, 4, EPI, SPLIT>), grid, block, 0, s, a, p.kchunk); break;
+        case 2:
+            if constexpr (RTS >= 2) hipLaunchKernelGGL((gemm_small_kernel<WT, 2, EPI, SPLIT>), grid, block, 0, s, a, p.kchunk);
+            break;
+        case 3:
+            if constexpr (RTS >= 3) hipLaunchKernelGGL((gemm_small_kernel<WT, 3, EPI, SPLIT>), grid, block, 0, s, a, p.kchunk);
+            break;
+        default:
+            if constexpr (RTS >= 4) hipLaunchKernelGGL((gemm_small_kernel<WT, 4, EPI, SPLIT>), grid, block, 0, s, a, p.kchunk);
+            break;
     }
 }
 
@@ -513,7 +536,8 @@ hipError_t launch_gemm(const GemmArgs& a, int epi, bool bf16, hipStream_t s) {
     const int fit = static_cast<int>(std::min<size_t>(kGemmMaxSplits, kGemmWsFloats / (static_cast<size_t>(a.M) * a.N)));
     const int splits = std::max(1, std::min(a.splits, fit));
     const GemmSmallPlan small = gemm_small_plan(a.M, a.N, a.K, splits, bf16);
-    if (small.splits) return launch_gemm_small_plan(a, epi, bf16, small, s);
+    const bool one_tile = (epi == kGemmGelu || epi == kGemmSwiglu) && small.splits == 1;
+    if (small.splits && !(one_tile && a.M > 16)) return launch_gemm_small_plan(a, epi, bf16, small, s);
     return launch_gemm_plan(a, epi, bf16, gemm_plan(a.M, a.N, a.K, splits, bf16, true), s);
 }
 
