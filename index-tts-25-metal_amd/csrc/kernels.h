@@ -266,11 +266,11 @@ struct GemmArgs {
     uint32_t kv_cap;
     const uint32_t* row_slot;
     const uint32_t* row_pos;
-    // split-K: at most `splits` K ranges (1 forbids splitting); launch_gemm picks the tile
-    // shape and the split count from an estimate of the time.  The partial tiles go to
-    // ws[splits][M][N] and a second kernel adds them in split order.
-    int splits;
+    // Split-K workspace of kGemmWsFloats.  launch_gemm picks the tile shape and the split count
+    // (`splits`, which it sets) from an estimate of the time; with more than one, the partial tiles
+    // go to ws[splits][M][N] and a second kernel adds them in split order.
     float* ws;
+    int splits;
     // kGemmResid with ln_out (N = 1280): also ln_out[m] = LayerNorm(c[m]; ln_w, ln_b), the
     // next LayerNorm of the residual stream (kernels.metal:618-669), folded into the split-K
     // reduce when there is one

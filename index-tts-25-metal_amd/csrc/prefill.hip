@@ -529,12 +529,11 @@ hipError_t launch_gemm_small_plan(GemmArgs a, int epi, bool bf16, const GemmSmal
 }  // namespace
 
 hipError_t launch_gemm(const GemmArgs& a, int epi, bool bf16, hipStream_t s) {
-    if (a.N % kGemmBn || a.K % kGemmK || a.M < 1 || a.splits < 1 || (a.splits > 1 && !a.ws)) return hipErrorInvalidValue;
+    if (a.N % kGemmBn || a.K % kGemmK || a.M < 1 || !a.ws) return hipErrorInvalidValue;
     if ((epi == kGemmStore || epi == kGemmSwiglu) && bf16) return hipErrorInvalidValue;  // FP32 weights only (the Qwen decoder)
     if (a.ln_out && (epi != kGemmResid || a.N != kWidth)) return hipErrorInvalidValue;
     if (split_elems(a.M, a.K) * 2 >= 0x40000000u) return hipErrorInvalidValue;  // 32-bit operand offsets
-    const int fit = static_cast<int>(std::min<size_t>(kGemmMaxSplits, kGemmWsFloats / (static_cast<size_t>(a.M) * a.N)));
-    const int splits = std::max(1, std::min(a.splits, fit));
+    const int splits = std::max(1, static_cast<int>(std::min<size_t>(kGemmMaxSplits, kGemmWsFloats / (static_cast<size_t>(a.M) * a.N))));
     const GemmSmallPlan small = gemm_small_plan(a.M, a.N, a.K, splits, bf16);
     const bool one_tile = (epi == kGemmGelu || epi == kGemmSwiglu) && small.splits == 1;
     if (small.splits && !(one_tile && a.M > 16)) return launch_gemm_small_plan(a, epi, bf16, small, s);

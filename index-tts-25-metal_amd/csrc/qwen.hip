@@ -816,7 +816,6 @@ struct Engine {
         g.K = Kk;
         g.c = C;
         g.c_split = Csplit;
-        g.splits = kGemmMaxSplits;
         g.ws = ws.p;
         QWEN_CHECK(launch_gemm(g, epi, false, stream));
     }

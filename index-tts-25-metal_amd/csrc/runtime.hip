@@ -864,7 +864,6 @@ struct Engine {
             g.M = static_cast<int>(M);
             g.N = kQkv;
             g.K = kWidth;
-            g.splits = kGemmMaxSplits;
             g.ws = b.ws;
             g.c = pq_;
             g.kv = kv.p;
@@ -894,7 +893,6 @@ struct Engine {
             p.M = static_cast<int>(M);
             p.N = kWidth;
             p.K = kWidth;
-            p.splits = kGemmMaxSplits;
             p.ws = b.ws;
             p.c = px_;
             p.ln_w = par + kParLn2W;  // ln_2 of the new residual rows
@@ -908,7 +906,6 @@ struct Engine {
             f.M = static_cast<int>(M);
             f.N = kFfn;
             f.K = kWidth;
-            f.splits = kGemmMaxSplits;
             f.ws = b.ws;
             f.c_split = pff_;
             HIP_CHECK(launch_gemm(f, kGemmGelu, bf16, stream));
@@ -919,7 +916,6 @@ struct Engine {
             f2.M = static_cast<int>(M);
             f2.N = kWidth;
             f2.K = kFfn;
-            f2.splits = kGemmMaxSplits;
             f2.ws = b.ws;
             f2.c = px_;
             if (l + 1 < layers) {  // ln_1 of the next layer
