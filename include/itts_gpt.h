@@ -150,7 +150,7 @@ int itts_gpt_generate(itts_gpt* h, const float* prefix, uint32_t rows, const itt
 
 /* No counterpart in the reference: itts_gpt_generate (one sequence, num_beams 1) for callers
  * that cannot allocate device memory (tight serving loops, harnesses that forbid hipMalloc).
- * It calls no hipMalloc/hipFree: the prefill activations live in a 28 MiB device array of
+ * It calls no hipMalloc/hipFree: the prefill activations live in a 60 MiB device array of
  * the library (one per GPU, held until the process ends) instead of buffers grown per call,
  * and a decode graph not captured yet is replaced by eager launches of the same kernels.
  * Same kernels, same codes as itts_gpt_generate.  Limits (ITTS_EINVAL): prefix rows <= 512,

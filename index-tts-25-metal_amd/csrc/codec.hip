@@ -10,7 +10,7 @@
 // codec's erf form, erf from the Abramowitz-Stegun 7.1.26 polynomial (kernels.metal:3133-3137);
 // "same" convolutions pad kernel/2 zeros on each side (kernels.metal:1397-1426, 1516-1541).
 //
-// Kernels (43 launches per decode):
+// Kernels (41 launches per decode, 42 when the up conv's K is split):
 //   * codec_lookup: one workgroup per code, the 8-wide codebook row times out_project.
 //   * codec_gemm<EPI>: C = A W^T + bias on the matrix cores with split operands (gemm_core.h); every
 //     A is written split by the kernel before.  A "same" convolution of kernel k over time-major
@@ -665,7 +665,8 @@ struct CodecEngine {
     }
 
     // Mean duration of the device work of decode(n codes) over iters back-to-back runs, and its
-    // FLOPs (the GEMMs; lookup, norms, depthwise convs and copies are < 0.5% of them).
+    // FLOPs (the GEMMs as they are run, the up conv with two taps; lookup, norms, depthwise convs
+    // and copies are < 0.5% of them).
     void bench(uint32_t n, uint32_t iters, float* avg_ms, double* flops) {
         if (!iters || n < 1 || n > static_cast<uint32_t>(kMaxCodes)) throw std::invalid_argument("Invalid codec benchmark request");
         std::vector<uint32_t> codes(n);
@@ -681,8 +682,7 @@ struct CodecEngine {
         CODEC_CHECK(hipEventElapsedTime(&ms, ev[0], ev[1]));
         *avg_ms = ms / iters;
         const double T = n;
-        *flops = 2.0 * T * kCH * kCK * kCW + kCBlocks * 2.0 * (2.0 * T * kCH * kCF) + 2.0 * T * kCW * kCH +
-                 2.0 * (2 * T) * kCW * kUpK * kCW;
+        *flops = 2.0 * T * kCH * kCK * kCW + kCBlocks * 2.0 * (2.0 * T * kCH * kCF) + 2.0 * T * kCW * kCH + 2.0 * T * kUpN * kUpTaps * kCW;
     }
 };
 

@@ -26,7 +26,7 @@
 // q_argmax_kernel, which picks the token and advances the device state.  The step is
 // captured once as a hipGraph; token, cache length and count live in device QState, so
 // generate() replays it with no per-token host work and polls a flag every 16 tokens.
-// Prefill (P ids): embedding rows, RMSNorm rows, FP32 MFMA GEMMs of prefill.hip (store, residual
+// Prefill (P ids): embedding rows, RMSNorm rows, split-BF16 GEMMs of prefill.hip (store, residual
 // and SwiGLU epilogues, split K when tiles are few), q_prep_kernel over P rows, causal
 // attention, then the head on the last row.
 #include <type_traits>
@@ -120,7 +120,7 @@ struct QCausalArgs {
     const float* q;        // [rows][2048]
     const float* kc;
     const float* vc;
-    uint16_t* out;  // split operand of o_proj            // [rows][2048]
+    uint16_t* out;         // [rows][2048], split operand of o_proj
     int rows;
 };
 

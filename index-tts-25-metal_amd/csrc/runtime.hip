@@ -183,10 +183,10 @@ void step_solo_waited(int dev) {
 // itts_gpt_generate_noalloc takes the prefill's activations (which itts_gpt_generate grows
 // with hipMalloc as prefixes get longer) from this file-scope device array instead, so the
 // call allocates nothing.  Layout for M <= kNoAllocRows prefix rows, every part 256-B aligned:
-//   x, xn, q, att [kNoAllocRows][1280] f32; ff [kNoAllocRows][5120] f32;
-//   row_slot, row_pos [kNoAllocRows] u32; last_rows [64] u32; the split-K GEMM workspace
-//   (kGemmWsFloats f32).
-// Each GPU holds its own copy (28 MiB) until the process ends.  Host code never passes the
+//   x, q [kNoAllocRows][1280] f32; xn, att [kNoAllocRows][1280] and ff [kNoAllocRows][5120] as
+//   split GEMM operands (6 bytes an element, gemm_core.h); row_slot, row_pos [kNoAllocRows] u32;
+//   last_rows [64] u32; the split-K GEMM workspace (kGemmWsFloats f32).
+// Each GPU holds its own copy (60 MiB) until the process ends.  Host code never passes the
 // array's name to a kernel: it is a host-side stand-in there.  The device address, per
 // device, comes from hipGetSymbolAddress at decoder creation (scratch_address below).
 constexpr uint32_t kNoAllocRows = 512;
