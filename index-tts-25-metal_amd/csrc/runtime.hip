@@ -620,7 +620,7 @@ struct Engine {
     // 2..kStepBatchMax in one launch (step_batch.hip; with the beam row-owner table when every
     // slot it may name is below kStepBatchMax).  Other batches take the multi-kernel path,
     // whose batched GEMVs read the weights once for all of them.
-    // With BF16 weights it takes the single steps whose logits go to the host (step(): 690 -> 600
+    // With BF16 weights it takes the single steps whose logits go to the host (step(): 687 -> 588
     // us a call at 250 cached rows); generate()'s documented path there is the multi-kernel graph.
     bool persistent(int nseq, bool use_table, bool sampler = true) const {
         if (!step_ok || nseq < 1 || nseq > kStepBatchMax) return false;

@@ -66,8 +66,9 @@ using StepWeight = float;
 constexpr int kRing = 24;          // chunks in the LDS ring
 // BF16 weights: a chunk is half the bytes, so twice the slots keep as many in flight, and the
 // producers end their phases closer together.  Step at 60 / 1010 cached rows, call to logits on
-// the host: 2 slots 625 / 682 us, 3 600 / 648, 4 589 / 643, 6 613 / 680; with 4 slots, first poll
-// after 4 * 64 clocks 623 / 668, 8 608 / 657, 14 597 / 647, 20 592 / 642, 24 588 / 637.
+// the host (measured when two blocking copies of the error flag were part of the call, 25 us): 2
+// slots 625 / 682 us, 3 600 / 648, 4 589 / 643, 6 613 / 680; with 4 slots, first poll after
+// 4 * 64 clocks 623 / 668, 8 608 / 657, 14 597 / 647, 20 592 / 642, 24 588 / 637.
 constexpr int kSlotsBf16 = 4, kPollDelayBf16 = 24;
 
 // This workgroup's share of the step, identical in every wave.
